@@ -227,8 +227,8 @@ def main():
         for c in combos():
             print(lib_name(c))
         return 0
-    if not os.path.isdir(REF):
-        print("build_ref: %s absent; nothing built" % REF)
+    if not os.path.isdir(SRC):
+        print("build_ref: no reference sources under %s; nothing built" % REF)
         return 0
     os.makedirs(OUT, exist_ok=True)
     bad = 0
