@@ -31,7 +31,7 @@ __device__ __forceinline__ double wave_sum(double v) {
 }
 
 // ComputeDt.cpp:34-46 contribution of one fluid cell (std::max keeps the old
-// maximum when the candidate is NaN); amax accumulates the squared sound speed.
+// maximum when the candidate is NaN, as fmax does); amax accumulates the squared sound speed.
 __device__ __forceinline__ void dt_terms(double gam, double gm1, const double* U, double& amax, double& umax,
                                          double& vmax, int& bad) {
     PState<double> s = pstate(gm1, U);
@@ -39,10 +39,9 @@ __device__ __forceinline__ void dt_terms(double gam, double gm1, const double* U
     // the maximum sound speed is taken as sqrt of the maximum a^2: RN(sqrt) is
     // monotone, so this equals the maximum of the rounded sound speeds
     double a2 = dq(gam * p, s.ir);
-    amax = (amax < a2) ? a2 : amax;
-    double au = ib_fabs(u), av = ib_fabs(v);
-    umax = (umax < au) ? au : umax;
-    vmax = (vmax < av) ? av : vmax;
+    amax = ib_max(amax, a2);
+    umax = ib_max(umax, ib_fabs(u));
+    vmax = ib_max(vmax, ib_fabs(v));
     bad |= !(rho > 0.0 && p > 0.0);
 }
 
@@ -55,17 +54,16 @@ __device__ __forceinline__ void floor_and_dt(double gam, double gm1, const Rcp<d
     const double rho = q[0];
     Rcp<double> ir = rcp_of(rho);
     double u = dq(q[1], ir), v = dq(q[2], ir);
-    double ke = 0.5 * rho * (u * u + v * v);
-    double p = gm1 * (q[3] - ke);
+    const double rs = rho * (u * u + v * v);  // twice the kinetic energy
+    double p = gm1 * ib_fma(-0.5, rs, q[3]);
     if (!quirks && !(p > P_FLOOR)) {
-        q[3] = dq(P_FLOOR, r_gm1) + ke;
-        p = gm1 * (q[3] - ke);
+        q[3] = ib_fma(0.5, rs, dq(P_FLOOR, r_gm1));
+        p = gm1 * ib_fma(-0.5, rs, q[3]);
     }
     double a2 = dq(gam * p, ir);
-    amax = (amax < a2) ? a2 : amax;
-    double au = ib_fabs(u), av = ib_fabs(v);
-    umax = (umax < au) ? au : umax;
-    vmax = (vmax < av) ? av : vmax;
+    amax = ib_max(amax, a2);
+    umax = ib_max(umax, ib_fabs(u));
+    vmax = ib_max(vmax, ib_fabs(v));
     bad |= !(rho > 0.0 && p > 0.0);
 }
 
@@ -123,7 +121,7 @@ template <> __device__ __forceinline__ PState<float> prim_of<float>(double gm1, 
     double y = __builtin_amdgcn_rcp(rho);
     y = __builtin_fma(y, __builtin_fma(-rho, y, 1.0), y);
     const double u = U[1] * y, v = U[2] * y;
-    const double p = gm1 * (U[3] - 0.5 * rho * (u * u + v * v));
+    const double p = gm1 * ib_fma(-0.5, rho * (u * u + v * v), U[3]);
     PState<float> s;
     s.rho = (float)rho; s.u = (float)u; s.v = (float)v; s.p = (float)p; s.E = (float)U[3];
     s.ir = Rcp<float>{s.rho, (float)y};
@@ -231,8 +229,8 @@ __device__ __forceinline__ void cell_states(const double* um, const double* u0, 
                 sl = lim_vanalbada(a, b);
                 sh = lim_vanalbada(b, a);
             }
-            lo[k] = u0[k] + (double)(0.5f * sl);
-            hi[k] = u0[k] - (double)(0.5f * sh);
+            lo[k] = ib_fma(0.5, (double)sl, u0[k]);
+            hi[k] = ib_fma(-0.5, (double)sh, u0[k]);
         }
     }
 }
