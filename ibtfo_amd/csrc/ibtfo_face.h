@@ -129,13 +129,13 @@ template <> __device__ __forceinline__ PState<float> prim_of<float>(double gm1, 
 }
 
 // Face states of one face from the reconstructed FP64 conserved states Ulo/Uhi
-// (in/out; the cell averages for Godunov) and the two cell averages u1, u2
-// beside it: the MUSCL-Hancock predictor and the corrected mode's positivity
+// (in/out; the cell averages for Godunov) and the two cell averages u1(k), u2(k)
+// beside it (functions, so that a caller can leave them in LDS): the MUSCL-Hancock predictor and the corrected mode's positivity
 // fallback. T is the compute type of the primitive states and fluxes (double,
 // or float in the mixed-precision form).
-template <int SCH, bool Y, typename T>
-__device__ __forceinline__ void face_states(const GasT<T>& g, double gm1, T dt, int quirks, const double* u1,
-                                            const double* u2, double* Ulo, double* Uhi, PState<T>& L,
+template <int SCH, bool Y, typename T, typename C1, typename C2>
+__device__ __forceinline__ void face_states(const GasT<T>& g, double gm1, T dt, int quirks, const C1& u1,
+                                            const C2& u2, double* Ulo, double* Uhi, PState<T>& L,
                                             PState<T>& R) {
     L = prim_of<T>(gm1, Ulo);
     R = prim_of<T>(gm1, Uhi);
@@ -155,7 +155,7 @@ __device__ __forceinline__ void face_states(const GasT<T>& g, double gm1, T dt, 
     }
     if (SCH != SCH_GODUNOV && !quirks && !(physical(L) && physical(R))) {
 #pragma unroll
-        for (int k = 0; k < 4; k++) { Ulo[k] = u1[k]; Uhi[k] = u2[k]; }
+        for (int k = 0; k < 4; k++) { Ulo[k] = u1(k); Uhi[k] = u2(k); }
         L = prim_of<T>(gm1, Ulo);
         R = prim_of<T>(gm1, Uhi);
     }
@@ -174,31 +174,31 @@ __device__ __forceinline__ bool riemann(const GasT<T>& g, const PState<T>& L, co
 }
 
 // x face between cells u1 (left) and u2 (right), reconstructed states UL, UR
-template <int SCH, int RS, typename T>
-__device__ __forceinline__ void xface(const GasT<T>& g, double gm1, T dt, int quirks, const double* u1,
-                                      const double* u2, double* UL, double* UR, T* F) {
+template <int SCH, int RS, typename T, typename C1, typename C2>
+__device__ __forceinline__ void xface(const GasT<T>& g, double gm1, T dt, int quirks, const C1& u1,
+                                      const C2& u2, double* UL, double* UR, T* F) {
     PState<T> L, R;
     face_states<SCH, false>(g, gm1, dt, quirks, u1, u2, UL, UR, L, R);
     bool stray;
     riemann<false, RS>(g, L, R, UL, UR, F, quirks != 0, stray);
 }
 
-// y face between cells u1 (below) and u2 (above); Fx is the lower cell's x-face
+// y face between cells u1 (below) and u2 (above); Fx(k) is the lower cell's x-face
 // flux in the same row, which is what the reference leaves in the aliased G_OLD
 // slot when its y solver stores nothing (HLL/Riemann_solver.cpp:224-226,
 // PVRS/Riemann_solver.cpp:550).
-template <int SCH, int RS, typename T>
-__device__ __forceinline__ void yface(const GasT<T>& g, double gm1, T dt, int quirks, const double* u1,
-                                      const double* u2, double* UD, double* UU, const T* Fx, T* G) {
+template <int SCH, int RS, typename T, typename C1, typename C2, typename FX>
+__device__ __forceinline__ void yface(const GasT<T>& g, double gm1, T dt, int quirks, const C1& u1,
+                                      const C2& u2, double* UD, double* UU, const FX& Fx, T* G) {
     PState<T> D, Uu;
     face_states<SCH, true>(g, gm1, dt, quirks, u1, u2, UD, UU, D, Uu);
     bool stray;
     bool up = riemann<true, RS>(g, D, Uu, UD, UU, G, quirks != 0, stray);
     if (quirks) {
-        if (RS == RS_PVRS && stray) G[3] = Fx[3];
+        if (RS == RS_PVRS && stray) G[3] = Fx(3);
         if (RS == RS_HLL && up) {
 #pragma unroll
-            for (int k = 0; k < 4; k++) G[k] = Fx[k];
+            for (int k = 0; k < 4; k++) G[k] = Fx(k);
         }
     }
 }

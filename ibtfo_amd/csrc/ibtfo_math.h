@@ -35,9 +35,9 @@ template <> struct FpConst<float> {
 // scaling, without the scaling and special-value fixups: the same arithmetic on
 // the same operands, so the same correctly rounded result. Other x (zero,
 // tiny, infinite, negative, NaN) take the full IEEE sequence.
-IB_HD double ib_sqrt(double x) {
 #if defined(__HIP_DEVICE_COMPILE__)
-    if (!(x >= 0x1p-767 && x <= 0x1.fffffffffffffp+1023)) return __builtin_sqrt(x);
+IB_HD bool sqrt_plain(double x) { return x >= 0x1p-767 && x <= 0x1.fffffffffffffp+1023; }
+IB_HD double sqrt_unscaled(double x) {
     double y = __builtin_amdgcn_rsq(x);
     double g = x * y, h = 0.5 * y;
     double r = __builtin_fma(-h, g, 0.5);
@@ -47,8 +47,29 @@ IB_HD double ib_sqrt(double x) {
     g = __builtin_fma(d, h, g);
     d = __builtin_fma(-g, g, x);
     return __builtin_fma(d, h, g);
+}
+#endif
+IB_HD double ib_sqrt(double x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    double g = sqrt_unscaled(x);
+    if (__builtin_expect(!sqrt_plain(x), 0)) g = __builtin_sqrt(x);
+    return g;
 #else
     return __builtin_sqrt(x);
+#endif
+}
+// Two roots with one test for the rare operands, so that their chains overlap.
+IB_HD void ib_sqrt2(double x, double y, double& gx, double& gy) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    gx = sqrt_unscaled(x);
+    gy = sqrt_unscaled(y);
+    if (__builtin_expect(!(sqrt_plain(x) && sqrt_plain(y)), 0)) {
+        gx = __builtin_sqrt(x);
+        gy = __builtin_sqrt(y);
+    }
+#else
+    gx = __builtin_sqrt(x);
+    gy = __builtin_sqrt(y);
 #endif
 }
 // FP32 (mixed-precision form): the hardware square root (1 ulp)
@@ -58,6 +79,10 @@ IB_HD float ib_sqrt(float x) {
 #else
     return __builtin_sqrtf(x);
 #endif
+}
+IB_HD void ib_sqrt2(float x, float y, float& gx, float& gy) {
+    gx = ib_sqrt(x);
+    gy = ib_sqrt(y);
 }
 IB_HD double ib_fabs(double x) { return __builtin_fabs(x); }
 IB_HD float ib_fabs(float x) { return __builtin_fabsf(x); }
@@ -223,8 +248,10 @@ template <typename T> IB_HD PState<T> pstate(T gm1, const T* U) {
     s.E = U[3];
     return s;
 }
-// sqrt(gamma p / rho), where the reference calls pow(gamma p / rho, 0.5)
-template <typename T> IB_HD T sound(const GasT<T>& g, const PState<T>& s) { return ib_sqrt(dq(g.gam * s.p, s.ir)); }
+// sqrt(gamma p / rho) of both states of a face, where the reference calls pow(gamma p / rho, 0.5)
+template <typename T> IB_HD void sounds(const GasT<T>& g, const PState<T>& L, const PState<T>& R, T& al, T& ah) {
+    ib_sqrt2(dq(g.gam * L.p, L.ir), dq(g.gam * R.p, R.ir), al, ah);
+}
 
 // Conserve2Flux.cpp:71-74 (x) / :106-109 (y): physical flux of a conserved state.
 // The tangential momentum term is rho*u*v evaluated left to right in both directions.
@@ -260,7 +287,8 @@ template <bool Y, typename T>
 IB_HD bool hll_face(const GasT<T>& g, const PState<T>& L, const PState<T>& R, const T* Ulo, const T* Uhi, T* F,
                     bool quirks) {
     const T unl = Y ? L.v : L.u, unh = Y ? R.v : R.u;
-    const T al = sound(g, L), ah = sound(g, R);
+    T al, ah;
+    sounds(g, L, R, al, ah);
     // p* = (p_lo + p_hi)/2 + (un_lo - un_hi)/2 * (rho_bar * a_bar)
     const T x = (unl - unh) * ((L.rho + R.rho) * (al + ah));
     T p_star = ib_fma(T(0.125), x, T(0.5) * (L.p + R.p));
@@ -313,7 +341,8 @@ template <bool Y, typename T> IB_HD void sw_half(const GasT<T>& g, T rho, T un, 
     out[3] = dq(rho * (g.gm1 * u2 * l1 + (h - a * un) * l3 + (h + a * un) * l4) * T(0.5), g.r_gam);
 }
 template <bool Y, typename T> IB_HD void sw_face(const GasT<T>& g, const PState<T>& L, const PState<T>& R, T* F) {
-    T al = sound(g, L), ah = sound(g, R);
+    T al, ah;
+    sounds(g, L, R, al, ah);
     // e = p / (gamma-1) / rho ; h = e + u*u/2 + v*v/2 + p/rho
     T el = dq(dq(L.p, g.r_gm1), L.ir), eh = dq(dq(R.p, g.r_gm1), R.ir);
     T hl = el + L.u * L.u * T(0.5) + L.v * L.v * T(0.5) + dq(L.p, L.ir);

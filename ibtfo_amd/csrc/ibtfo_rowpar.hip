@@ -338,14 +338,15 @@ __device__ __forceinline__ void step_rowpar(const StepArgs& a, const int bx, con
         double xr[4];
 #pragma unroll
         for (int k = 0; k < 4; k++) xr[k] = hb[wv][k][ln];
-        xface<SCH, RS>(g, a.gm1, dtc, a.quirks, w0, xp, xlo, xr, F);
+        xface<SCH, RS>(g, a.gm1, dtc, a.quirks, [&](int k) { return w0[k]; }, [&](int k) { return xp[k]; }, xlo, xr, F);
     }
     T G[4] = {0, 0, 0, 0};
     if (live) {
         double ylo[4], hi_unused[4], ynlo[4], ynhi[4];
         cell_states<SCH, LIM, T>(wm, w0, w1, ylo, hi_unused, a.quirks);
         cell_states<SCH, LIM, T>(w0, w1, w2, ynlo, ynhi, a.quirks);
-        yface<SCH, RS>(g, a.gm1, dtc, a.quirks, w0, w1, ylo, ynhi, F, G);
+        yface<SCH, RS>(g, a.gm1, dtc, a.quirks, [&](int k) { return w0[k]; }, [&](int k) { return w1[k]; }, ylo, ynhi,
+                       [&](int k) { return F[k]; }, G);
     }
 #pragma unroll
     for (int k = 0; k < 4; k++) {

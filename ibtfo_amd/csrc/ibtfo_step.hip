@@ -276,6 +276,8 @@ __device__ __forceinline__ void step_strip(const StepArgs& a, const int bx, cons
     const double dtdx = dt * a.r_dx, dtdy = dt * a.r_dy;  // mixed form only
     const double dx = a.dx, dy = a.dy;
     const int ng = L.ng, nx = L.nx, ny = L.ny;
+    // the cut-cell and mixed-precision forms exist in corrected mode only
+    const int quirks = CUT || !FP64 ? 0 : a.quirks;
 
     const int cb = ng + STRIP_W * bx;  // first interior column of the strip
     const int c = cb - 2 + lane;
@@ -283,7 +285,8 @@ __device__ __forceinline__ void step_strip(const StepArgs& a, const int bx, cons
     const int j0 = ng + a.rows * by;
     const int j1 = min(j0 + a.rows, ny + ng);
 
-    __shared__ double rb[2][4][64];  // row values of columns cb-2 .. cb+61
+    // 10 KB in all (FP64), so that 16 blocks, four waves per SIMD, fit a CU's 160 KB
+    __shared__ double rb[4][64];     // row values of columns cb-2 .. cb+61 (read before the next barrier)
     __shared__ double hb[4][64];     // lower-face states of the x pairs
     __shared__ T fb[4][64];          // x-face fluxes
     // carried from one row to the next, per lane: kept in LDS rather than in
@@ -307,22 +310,29 @@ __device__ __forceinline__ void step_strip(const StepArgs& a, const int bx, cons
         }
     }
 
+    // Rows are addressed as a wave-uniform base (scalar registers) plus the lane's
+    // 32-bit column offset: no 64-bit address arithmetic in the vector unit.
+    const unsigned int co = (unsigned int)cl * 8u, ct = (unsigned int)cl;
+    auto ld = [&](const double* base, int row, int k) {
+        return *(const double*)((const char*)(base + L.at(0, row) + k * PL) + co);
+    };
+    auto st = [&](double* base, int row, int k, double v) {
+        *(double*)((char*)(base + L.at(0, row) + k * PL) + co) = v;
+    };
+
     // column window: w[0..2] = rows j, j+1, j+2 of column c at iteration j;
     // ylb = the y state of row j on its upper face (from the previous pair)
     double w[3][4];
     {
         double wm[4];
-        long long o = L.at(cl, j0 - 2);
 #pragma unroll
-        for (int k = 0; k < 4; k++) wm[k] = Ui[o + k * PL];
+        for (int k = 0; k < 4; k++) wm[k] = ld(Ui, j0 - 2, k);
 #pragma unroll
-        for (int r = 0; r < 3; r++) {
-            o = L.at(cl, j0 - 1 + r);
+        for (int r = 0; r < 3; r++)
 #pragma unroll
-            for (int k = 0; k < 4; k++) w[r][k] = Ui[o + k * PL];
-        }
+            for (int k = 0; k < 4; k++) w[r][k] = ld(Ui, j0 - 1 + r, k);
         double hi_unused[4], ylo[4];
-        cell_states<SCH, LIM, T>(wm, w[0], w[1], ylo, hi_unused, a.quirks);
+        cell_states<SCH, LIM, T>(wm, w[0], w[1], ylo, hi_unused, quirks);
 #pragma unroll
         for (int k = 0; k < 4; k++) { ylb[k][lane] = ylo[k]; gpb[k][lane] = T(0); }
     }
@@ -333,129 +343,123 @@ __device__ __forceinline__ void step_strip(const StepArgs& a, const int bx, cons
     const int ln = min(lane + 1, 63), lp = max(lane - 1, 0);
 
     for (int j = j0 - 1; j < j1; j++) {
-        const int b = j & 1;
-        // prefetch the next window row and next halo value (none after the last
-        // row: they would only be discarded)
+        // prefetch the next window row (none after the last row: it would only be
+        // discarded; j + 3 <= ny + ng + 1 lies in the grid, ng >= 2)
         double nw[4];
         if (j + 1 < j1) {
-            long long o = L.at(cl, min(j + 3, L.N - 1));
 #pragma unroll
-            for (int k = 0; k < 4; k++) nw[k] = Ui[o + k * PL];
+            for (int k = 0; k < 4; k++) nw[k] = ld(Ui, j + 3, k);
         }
+        // FP64: row j's cells and x fluxes stay in LDS (rb, fb) and are read back
+        // where they are used, so that no register holds them through the y face.
+#pragma unroll
+        for (int k = 0; k < 4; k++) rb[k][lane] = w[0][k];
+        __syncthreads();
         T F[4] = {0, 0, 0, 0};
+        auto cell = [&](int k) { return FP64 ? rb[k][lane] : w[0][k]; };
+        auto flux = [&](int k) { return FP64 ? fb[k][lane] : F[k]; };
         // x faces of row j; the first iteration (j = j0-1) only needs the y face
         // below row j0, unless that face may take the aliased x flux
-        if (j >= j0 || (a.quirks && RS != RS_SW)) {
-#pragma unroll
-            for (int k = 0; k < 4; k++) rb[b][k][lane] = w[0][k];
-            __syncthreads();
+        if (j >= j0 || (quirks && RS != RS_SW)) {
             double xm[4], xp[4], xlo[4], xhi[4];
 #pragma unroll
             for (int k = 0; k < 4; k++) {
-                xm[k] = rb[b][k][lp];
-                xp[k] = rb[b][k][ln];
+                xm[k] = rb[k][lp];
+                xp[k] = rb[k][ln];
             }
-            cell_states<SCH, LIM, T>(xm, w[0], xp, xlo, xhi, a.quirks);
+            cell_states<SCH, LIM, T>(xm, w[0], xp, xlo, xhi, quirks);
 #pragma unroll
             for (int k = 0; k < 4; k++) hb[k][lane] = xhi[k];
             __syncthreads();
             double xr[4];
 #pragma unroll
             for (int k = 0; k < 4; k++) xr[k] = hb[k][ln];
-            xface<SCH, RS>(g, a.gm1, dtc, a.quirks, w[0], xp, xlo, xr, F);
+            xface<SCH, RS>(g, a.gm1, dtc, quirks, cell, [&](int k) { return FP64 ? rb[k][ln] : xp[k]; }, xlo, xr, F);
+#pragma unroll
+            for (int k = 0; k < 4; k++) fb[k][lane] = F[k];
         }
         // y face j+1/2: this row's upper state and the lower state of row j+1
-        double ynlo[4], ynhi[4];
         T G[4];
-        cell_states<SCH, LIM, T>(w[0], w[1], w[2], ynlo, ynhi, a.quirks);
         {
-            double ylo[4];
+            double ylo[4], ynlo[4], ynhi[4];
+            cell_states<SCH, LIM, T>(w[0], w[1], w[2], ynlo, ynhi, quirks);
 #pragma unroll
-            for (int k = 0; k < 4; k++) ylo[k] = ylb[k][lane];
-            yface<SCH, RS>(g, a.gm1, dtc, a.quirks, w[0], w[1], ylo, ynhi, F, G);
+            for (int k = 0; k < 4; k++) {
+                ylo[k] = ylb[k][lane];
+                ylb[k][lane] = ynlo[k];
+            }
+            yface<SCH, RS>(g, a.gm1, dtc, quirks, cell, [&](int k) { return w[1][k]; }, ylo, ynhi, flux, G);
         }
 
         if (j >= j0) {
-#pragma unroll
-            for (int k = 0; k < 4; k++) fb[k][lane] = F[k];
             __syncthreads();
             if (upd_col) {
-                double un[4];
-                const long long o = L.at(c, j);
-                const uint8_t tc = a.type[o];
+                double u0[4], un[4];
+                const uint8_t tc = *(a.type + L.at(0, j) + ct);
                 const bool fluid = CUT ? (tc & 3) == 0 : tc == 0;
                 const bool merged = CUT && (tc & MERGED_BIT);
+                // the floors; the dt / mass partials (a merge group's come from the merge)
+                bool floors = fluid;
+                double vol = 1.0;  // the cell's fluid fraction
+#pragma unroll
+                for (int k = 0; k < 4; k++) un[k] = u0[k] = cell(k);
                 if (fluid) {
 #pragma unroll
                     for (int k = 0; k < 4; k++) {
-                        if (FP64) {
-                            double Fm = fb[k][lane - 1];
-                            double v = w[0][k] - dq(dt * ((double)F[k] - Fm), r_dx);
-                            un[k] = v - dq(dt * ((double)G[k] - (double)gpb[k][lane]), r_dy);
-                        } else {  // FP32 fluxes, FP64 accumulation
-                            double Fm = (double)fb[k][lane - 1];
-                            un[k] = w[0][k] - dtdx * ((double)F[k] - Fm) - dtdy * ((double)G[k] - (double)gpb[k][lane]);
-                        }
+                        const double dF = (double)flux(k) - (double)fb[k][lane - 1];
+                        const double dG = (double)G[k] - (double)gpb[k][lane];
+                        // FP64, or FP32 fluxes with FP64 accumulation
+                        if (FP64) un[k] = (u0[k] - dq(dt * dF, r_dx)) - dq(dt * dG, r_dy);
+                        else un[k] = u0[k] - dtdx * dF - dtdy * dG;
                     }
-                    if (stage == 0) {
-                        if (!merged) {
-                            floor_and_dt(a.gam, a.gm1, r_gm1, un, a.quirks, amax, umax, vmax, bad);
-                        } else {  // a merge target: floored here, its partials come from the merge
-                            double d0 = 0.0, d1 = 0.0, d2 = 0.0;
-                            int db = 0;
-                            floor_and_dt(a.gam, a.gm1, r_gm1, un, a.quirks, d0, d1, d2, db);
-                        }
-                    } else {
-                        // RK2 (Heun): each stage's update takes the floors; the second
-                        // stage then averages with U^n, which the output buffer holds
-                        double d0 = 0.0, d1 = 0.0, d2 = 0.0;
-                        int db = 0;
-                        floor_and_dt(a.gam, a.gm1, r_gm1, un, a.quirks, d0, d1, d2, db);
-                        if (stage >= 2) {
-#pragma unroll
-                            for (int k = 0; k < 4; k++) un[k] = 0.5 * (Uo[o + k * PL] + un[k]);
-                            dt_terms(a.gam, a.gm1, un, amax, umax, vmax, bad);
-                        }
-                    }
-                    if (!merged) msum += un[0] * dx * dy;
                 } else if (CUT && (tc & 3) == 3) {
                     // cut cell: aperture-weighted face fluxes and the wall's pressure
                     // force S p (S closes the cell's faces), over the fluid volume
                     // alpha dx dy; small cells are merged (and floored) afterwards
-                    const CutCell cc = a.cut[a.cut_index[o]];
-                    const double rho = w[0][0], u0 = w[0][1] / rho, v0 = w[0][2] / rho;
-                    const double pw = a.gm1 * (w[0][3] - 0.5 * rho * (u0 * u0 + v0 * v0));
-                    const double wall[4] = {0.0, pw * cc.sbx, pw * cc.sby, 0.0};
+                    const CutCell cc = a.cut[a.cut_index[L.at(c, j)]];
+                    const PState<double> s0 = pstate(a.gm1, u0);
+                    const double wall[4] = {0.0, s0.p * cc.sbx, s0.p * cc.sby, 0.0};
+                    const Rcp<double> rv = rcp_of(cc.alpha * dx * dy);
 #pragma unroll
                     for (int k = 0; k < 4; k++) {
-                        const double Fk = (double)F[k], Fm = (double)fb[k][lane - 1];
+                        const double Fk = (double)flux(k), Fm = (double)fb[k][lane - 1];
                         const double Gk = (double)G[k], Gm = (double)gpb[k][lane];
-                        double v = w[0][k] - dt * ((cc.ae * Fk - cc.aw * Fm) * dy) / (cc.alpha * dx * dy);
-                        un[k] = v - dt * ((cc.an * Gk - cc.as * Gm) * dx + wall[k]) / (cc.alpha * dx * dy);
+                        const double v = u0[k] - dq(dt * ((cc.ae * Fk - cc.aw * Fm) * dy), rv);
+                        un[k] = v - dq(dt * ((cc.an * Gk - cc.as * Gm) * dx + wall[k]), rv);
                     }
-                    // a merge-group cell (small cell or target) takes its floors and
-                    // partials from the merge; the others are floored and counted here
-                    if (!merged) {
-                        floor_and_dt(a.gam, a.gm1, r_gm1, un, a.quirks, amax, umax, vmax, bad);
-                        msum += cc.alpha * un[0] * dx * dy;
-                    } else if (cc.alpha >= 0.5) {
-                        double d0 = 0.0, d1 = 0.0, d2 = 0.0;
-                        int db = 0;
-                        floor_and_dt(a.gam, a.gm1, r_gm1, un, a.quirks, d0, d1, d2, db);
-                    }
-                } else {
+                    floors = !merged || cc.alpha >= 0.5;
+                    vol = cc.alpha;
+                }
+                if (floors) {
+                    double am = 0.0, um = 0.0, vm = 0.0;
+                    int nb = 0;
+                    floor_and_dt(a.gam, a.gm1, r_gm1, un, quirks, am, um, vm, nb);
+                    if (stage >= 2) {
+                        // RK2 (Heun): each stage's update takes the floors; the second stage
+                        // then averages with U^n, which the output buffer holds
 #pragma unroll
-                    for (int k = 0; k < 4; k++) un[k] = w[0][k];
+                        for (int k = 0; k < 4; k++) un[k] = 0.5 * (ld(Uo, j, k) + un[k]);
+                        am = um = vm = 0.0;
+                        nb = 0;
+                        dt_terms(a.gam, a.gm1, un, am, um, vm, nb);
+                    }
+                    if (!merged) {
+                        amax = ib_max(amax, am);
+                        umax = ib_max(umax, um);
+                        vmax = ib_max(vmax, vm);
+                        bad |= nb;
+                        msum += fluid ? un[0] * dx * dy : vol * un[0] * dx * dy;
+                    }
                 }
 #pragma unroll
-                for (int k = 0; k < 4; k++) Uo[o + k * PL] = un[k];
+                for (int k = 0; k < 4; k++) st(Uo, j, k, un[k]);
                 if (a.edge_fused == 1) {
                     // Test/Sod/Global_Boudary.cpp:24-59 (rows) and :62-75 (columns), which
                     // read U_NEW: the updated state, or for a non-fluid cell under
                     // SimpleBound the value its U_NEW kept
                     double e[4] = {un[0], un[1], un[2], un[3]};
                     if (a.unew_nf && !fluid)
-                        for (int k = 0; k < 4; k++) e[k] = a.unew_nf[o + k * PL];
+                        for (int k = 0; k < 4; k++) e[k] = a.unew_nf[L.at(c, j) + k * PL];
                     if (j < 2 * ng) Uo[L.at(c, 2 * ng - 1 - j) + 2 * PL] = -e[2];
                     if (j == 2 * ng - 1)
                         for (int r = 0; r < ng; r++) {
@@ -484,7 +488,6 @@ __device__ __forceinline__ void step_strip(const StepArgs& a, const int bx, cons
 #pragma unroll
         for (int k = 0; k < 4; k++) {
             gpb[k][lane] = G[k];
-            ylb[k][lane] = ynlo[k];
             w[0][k] = w[1][k];
             w[1][k] = w[2][k];
             w[2][k] = nw[k];
@@ -503,12 +506,17 @@ __device__ __forceinline__ void step_strip(const StepArgs& a, const int bx, cons
     block_partials(a.mass_part, by * a.nbx + bx, amax, umax, vmax, msum, bad);
 }
 
+// Four waves per SIMD (128 VGPRs): the strip's chains of dependent FP64 work and
+// LDS exchanges need them (4096x2048 cut cells, HLL: 245 us at three waves, 226 at
+// four; Steger-Warming, 132 VGPRs unbounded: 325 us, 302 us with 12 bytes spilled).
+// PVRS, whose pow() calls need far more registers, is left to the compiler.
+constexpr int step_waves(int rs) { return rs == RS_PVRS ? 1 : 4; }
 template <int SCH, int RS, int LIM, typename T, bool CUT>
-__global__ __launch_bounds__(64) void k_step(StepArgs a) {
+__global__ __launch_bounds__(64, step_waves(RS)) void k_step(StepArgs a) {
     step_strip<SCH, RS, LIM, T, CUT>(a, blockIdx.x, blockIdx.y, a.stage);
 }
 template <int SCH, int RS, int LIM, typename T>
-__global__ __launch_bounds__(64) void k_step_periodic(StepArgs a) {
+__global__ __launch_bounds__(64, step_waves(RS)) void k_step_periodic(StepArgs a) {
     step_strip<SCH, RS, LIM, T, false, true>(a, blockIdx.x, blockIdx.y, a.stage);
 }
 
@@ -517,7 +525,7 @@ __global__ __launch_bounds__(64) void k_step_periodic(StepArgs a) {
 // map[b].x < 0 marks an idle block (the grid is sized for the batch capacity so
 // that a captured graph stays valid while solves come and go).
 template <int SCH, int RS, int LIM, typename T>
-__global__ __launch_bounds__(64) void k_step_batch(const StepArgs* __restrict__ slots, const int2* __restrict__ map,
+__global__ __launch_bounds__(64, step_waves(RS)) void k_step_batch(const StepArgs* __restrict__ slots, const int2* __restrict__ map,
                                                    int stage) {
     const int2 m = map[blockIdx.x];
     if (m.x < 0) return;
