@@ -423,28 +423,24 @@ static int rebuild_tables(ibtfo_batch* b) {
 static int enqueue_batch_step(ibtfo_batch* b) {
     const ibtfo_batch_config& k = b->bc;
     hipStream_t s = b->run;
-    auto bounds = [&]() -> int {
-        if (k.boundary != IBTFO_REGULAR && k.max_ghost_blocks > 0)
-            HIPCHK(launch_fill_batch(b->d_fill, b->d_gmap, k.max_ghost_blocks, s));
-        if (k.max_ring_blocks > 0) HIPCHK(launch_edge_batch(b->d_edge, b->d_rmap, k.max_ring_blocks, s));
-        if (k.boundary != IBTFO_REGULAR && k.max_ghost_blocks > 0)
-            HIPCHK(launch_scatter_batch(b->d_fill, b->d_gmap, k.max_ghost_blocks, s));
-        return IBTFO_OK;
+    // after an update: every solve's finish, ghost fill and edge ring in one launch
+    const int ngb = k.boundary != IBTFO_REGULAR ? k.max_ghost_blocks : 0;
+    auto post = [&](int advance) {
+        return launch_post_batch(b->d_fin, k.max_slots, advance, b->d_fill, b->d_gmap, ngb, b->d_edge, b->d_rmap,
+                                 k.max_ring_blocks, s);
     };
-    int rc;
     if (k.time == IBTFO_RK2) {
         HIPCHK(launch_step_batch(k.scheme, k.riemann, k.limiter, k.precision, b->d_step, b->d_smap,
                                  k.max_step_blocks, 1, s));
-        HIPCHK(launch_finish_batch(b->d_fin, k.max_slots, 2, s));
-        if ((rc = bounds())) return rc;
+        HIPCHK(post(2));
         HIPCHK(launch_step_batch(k.scheme, k.riemann, k.limiter, k.precision, b->d_step, b->d_smap,
                                  k.max_step_blocks, 2, s));
     } else {
         HIPCHK(launch_step_batch(k.scheme, k.riemann, k.limiter, k.precision, b->d_step, b->d_smap,
                                  k.max_step_blocks, 0, s));
     }
-    HIPCHK(launch_finish_batch(b->d_fin, k.max_slots, 1, s));
-    return bounds();
+    HIPCHK(post(1));
+    return IBTFO_OK;
 }
 
 // The chunk as one persistent launch: every resident solve's steps, phases

@@ -894,27 +894,26 @@ void ibtfo::build_args(ibtfo_ctx* x) {
     mg.part = x->merge_part;
 }
 
-// Boundary and Global_Boundary after an update (the state just made current):
-// ghost fill phase 1, the edge ring, ghost fill phase 2.
-static int enqueue_boundaries(ibtfo_ctx* x) {
+// What follows an update: the finish `f` (clock and dt, or the RK2 stage flip),
+// Boundary (ghost fill) and Global_Boundary (edge ring). One launch, with two
+// exceptions, which keep the separate kernels: SimpleBound's fill (dependency
+// levels, U_NEW's unrefreshed cells) and Lax's reference ring (its corners come
+// from the ring being rewritten).
+static int enqueue_finish_boundaries(ibtfo_ctx* x, const FinishArgs& f) {
     const ibtfo_config& c = x->cfg;
-    if (c.boundary != IBTFO_REGULAR && c.edge != IBTFO_EDGE_REFERENCE) {
-        // fill (first level) and ring in one launch; further SimpleBound levels after
-        FillArgs f = x->fa;
-        f.level = 0;
-        HIPCHK(launch_fill_edge(f, x->ea, x->stream));
-        for (int l = 1; l < x->nlevels; l++) {
-            f.level = l;
-            HIPCHK(launch_fill(f, x->stream));
-        }
-        HIPCHK(launch_scatter(x->fa, x->stream));
+    const bool fill = c.boundary != IBTFO_REGULAR && x->nghost > 0;
+    const bool ring = c.edge != IBTFO_EDGE_REFERENCE && x->sa.edge_fused != 2;
+    const bool lax_ring = c.edge == IBTFO_EDGE_REFERENCE && c.scheme == IBTFO_LAX;
+    if (c.boundary != IBTFO_SIMPLE_BOUND && !lax_ring) {
+        if (fill || ring) HIPCHK(launch_post(f, fill ? &x->fa : nullptr, ring ? &x->ea : nullptr, x->stream));
+        else HIPCHK(launch_finish(f, x->stream));
         return IBTFO_OK;
     }
-    if (c.boundary != IBTFO_REGULAR) HIPCHK(launch_fill_levels(x, x->fa));
-    if (c.edge == IBTFO_EDGE_REFERENCE && c.scheme == IBTFO_LAX)
-        HIPCHK(launch_edge_ref(x->ea, x->corner, x->sa.corner_from_input, x->stream));
-    if (c.edge != IBTFO_EDGE_REFERENCE && x->sa.edge_fused != 2) HIPCHK(launch_edge(x->ea, x->stream));
-    if (c.boundary != IBTFO_REGULAR) HIPCHK(launch_scatter(x->fa, x->stream));
+    HIPCHK(launch_finish(f, x->stream));
+    if (fill) HIPCHK(launch_fill_levels(x, x->fa));
+    if (lax_ring) HIPCHK(launch_edge_ref(x->ea, x->corner, x->sa.corner_from_input, x->stream));
+    if (ring) HIPCHK(launch_edge(x->ea, x->stream));
+    if (fill) HIPCHK(launch_scatter(x->fa, x->stream));
     return IBTFO_OK;
 }
 
@@ -939,8 +938,7 @@ static int enqueue_step(ibtfo_ctx* x, hipEvent_t* ev = nullptr, int k = 0) {
         if (!in_place) {
             FinishArgs flip = x->fin;
             flip.advance = 2;
-            HIPCHK(launch_finish(flip, x->stream));
-            if ((rc = enqueue_boundaries(x))) return rc;
+            if ((rc = enqueue_finish_boundaries(x, flip))) return rc;
         }
         StepArgs s2 = x->sa;
         s2.stage = in_place ? 3 : 2;
@@ -963,8 +961,7 @@ static int enqueue_step(ibtfo_ctx* x, hipEvent_t* ev = nullptr, int k = 0) {
         // ComputeDt / mass over both kernels' partials
         HIPCHK(launch_merge(x->ma, x->stream));
     }
-    HIPCHK(launch_finish(x->fin, x->stream));
-    return enqueue_boundaries(x);
+    return enqueue_finish_boundaries(x, x->fin);
 }
 
 // n steps, queued as one batch: with the deferred finish, n step kernels and

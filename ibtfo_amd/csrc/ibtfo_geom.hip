@@ -221,10 +221,14 @@ __global__ void k_geom_ghosts(GeomArgs g) {
         }
     }
     gh.ring = 0;
-    auto in_ring = [&](int ii, int jj) { return ii < ng || ii >= L.nx + ng || jj < ng || jj >= L.ny + ng; };
+    // the ring's type is 2 as well, so the type decides both cases
+    auto from_prev = [&](int ii, int jj) {
+        const uint8_t t = g.type[L.at(ii, jj)];
+        return t != 0 && !(g.cut && t == 3);
+    };
     for (int q = 0; q < 4; q++) {
-        if (in_ring(gh.idx + di[q], gh.idy + dj[q])) gh.ring |= 1 << q;
-        if (bc >= 4 && in_ring(gh.idxe + di[q], gh.idye + dj[q])) gh.ring |= 1 << (4 + q);
+        if (from_prev(gh.idx + di[q], gh.idy + dj[q])) gh.ring |= 1 << q;
+        if (bc >= 4 && from_prev(gh.idxe + di[q], gh.idye + dj[q])) gh.ring |= 1 << (4 + q);
     }
     gh.pick = -1;
     if (bc == 2 || bc == 3) {

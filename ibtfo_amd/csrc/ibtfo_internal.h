@@ -46,6 +46,7 @@ struct Ctl {
     int done;       // 1 once now_t >= Psy_time or iter >= max_iter
     int cur;        // which state buffer holds the current state
     int ran;        // 1 if the last launched step executed
+    int out;        // the buffer the last step kernel wrote (set by the step kernel, beside ran)
     int status;     // 0 ok; 1 non-finite value met in the dt reduction
     unsigned int folded;  // fold blocks done in the running finish (0 between launches)
     double mass_now;                      // CaculateMass of the state seen by the last reduction
@@ -141,7 +142,9 @@ struct Ghost {
     int idx, idy, idxe, idye, pick;  // SimpleBound: idx/idy = donor offsets IDX/IDY, idxe/idye = ghost
                                      // index of an x/y donor that is a ghost filled earlier (else -1),
                                      // pick = dependency level
-    int ring;           // bit q (image) / 4+q (extra): donor q lies in the domain ring
+    int ring;           // bit q (image) / 4+q (extra): donor q is read from the previous state: it
+                        // lies in the domain ring (not yet rewritten by Global_Boundary), or is a
+                        // non-active interior cell, which a step leaves as it was until the fill
 };
 
 struct FillArgs {
@@ -223,6 +226,7 @@ constexpr int FOLD_MIN_PARTS = 2048;  // fewer partials: one block reads them al
 
 constexpr int FILL_THREADS = 128;  // ghost-fill and scatter blocks
 constexpr int EDGE_THREADS = 256;  // edge-ring blocks
+constexpr int POST_THREADS = 256;  // a single solve's post kernel (k_post)
 
 // Persistent batched step (k_persist): one launch runs `nsteps` whole steps of
 // every resident solve of a batch, its phases (strips; per-solve finish; ghost
@@ -259,7 +263,6 @@ hipError_t launch_step(int scheme, int rs, int lim, int prec, const StepArgs& a,
 hipError_t launch_fill(const FillArgs& a, hipStream_t s);
 hipError_t launch_scatter(const FillArgs& a, hipStream_t s);
 hipError_t launch_edge(const EdgeArgs& a, hipStream_t s);
-hipError_t launch_fill_edge(const FillArgs& f, const EdgeArgs& e, hipStream_t s);  // fill phase 1 + ring
 hipError_t launch_reduce(const ReduceArgs& a, hipStream_t s);
 hipError_t launch_merge(const MergeArgs& a, hipStream_t s);
 // a uniform state (conserved U[0..3]) into every element of s0, s1 and s2 (if
@@ -267,13 +270,15 @@ hipError_t launch_merge(const MergeArgs& a, hipStream_t s);
 hipError_t launch_uniform_state(double* s0, double* s1, double* s2, long long plane, const double* U, Ctl* ctl,
                                 hipStream_t s);
 hipError_t launch_finish(const FinishArgs& f, hipStream_t s);
+// the finish, the ghost fill (in place) and the edge ring of a step in one launch
+// (fill / edge null: none)
+hipError_t launch_post(const FinishArgs& f, const FillArgs* fill, const EdgeArgs* edge, hipStream_t s);
+hipError_t launch_post_batch(const FinishArgs* f, int nslots, int advance, const FillArgs* fill, const int2* gmap,
+                             int nghost_blocks, const EdgeArgs* edge, const int2* rmap, int nring_blocks,
+                             hipStream_t s);
 // batched forms: one launch over many solves (maps: block -> {slot, first index})
 hipError_t launch_step_batch(int scheme, int rs, int lim, int prec, const StepArgs* slots, const int2* map,
                              int nblocks, int stage, hipStream_t s);
-hipError_t launch_finish_batch(const FinishArgs* f, int nslots, int advance, hipStream_t s);
-hipError_t launch_fill_batch(const FillArgs* f, const int2* map, int nblocks, hipStream_t s);
-hipError_t launch_scatter_batch(const FillArgs* f, const int2* map, int nblocks, hipStream_t s);
-hipError_t launch_edge_batch(const EdgeArgs* e, const int2* map, int nblocks, hipStream_t s);
 hipError_t launch_gather(const FinishArgs* f, int nslots, SlotStatus* out, hipStream_t s);
 // the persistent batched step: a zeroing of the barrier counter, then one launch of
 // `blocks` blocks (persist_blocks: the grid the kernel can hold resident at once)

@@ -273,6 +273,10 @@ __device__ __forceinline__ void step_rowpar(const StepArgs& a, const int bx, con
         }
         cur = ctl->cur ^ (stage == 3 ? 1 : 0);  // the input buffer
         dt = ctl->dt;
+        if (bx == 0 && by == 0 && threadIdx.x == 0) {
+            ctl->ran = 1;
+            ctl->out = cur ^ 1;
+        }
     }
     const double* __restrict__ Ui = a.buf[cur];
     double* __restrict__ Uo = a.buf[cur ^ 1];

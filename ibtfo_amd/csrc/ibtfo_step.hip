@@ -126,9 +126,8 @@ __global__ __launch_bounds__(FINISH_THREADS) void k_finish(FinishArgs f) {
 // one round trip, the control fields are read beside them rather than first,
 // and the lanes reduce through cross-lane shuffles instead of an LDS tree.
 constexpr int FINISH_SMALL_PER_LANE = FINISH_SMALL_MAX / 64;
-__global__ __launch_bounds__(64) void k_finish_small(FinishArgs f) {
+__device__ __forceinline__ void finish_small(const FinishArgs& f, const int advance) {
     Ctl* ctl = f.ctl;
-    const int advance = f.advance;
     if (advance == 2) {
         if (threadIdx.x == 0) {
             if (!ctl->done) {
@@ -170,6 +169,7 @@ __global__ __launch_bounds__(64) void k_finish_small(FinishArgs f) {
     if (advance && done) return;  // the step kernel did not run
     if (t == 0) finish_clock(f, ctl, A, Um, Vm, m, bad, advance, now_t, iter);
 }
+__global__ __launch_bounds__(64) void k_finish_small(FinishArgs f) { finish_small(f, f.advance); }
 
 // Partials of a 256-thread block: wave reductions, then the four waves in order.
 __device__ __forceinline__ void block4_partials(double* part, int bid, double amax, double umax, double vmax,
@@ -206,10 +206,10 @@ __device__ __forceinline__ void block4_partials(double* part, int bid, double am
 // Ctl::folded, with device-scope fences around the count) reduces the fold
 // records and runs the clock. Only the records cross blocks, so the fences
 // write back and invalidate little.
-__global__ __launch_bounds__(FOLD_THREADS) void k_fold(FinishArgs f) {
+__device__ __forceinline__ void fold_body(const FinishArgs& f, const int block) {
     if (f.ctl->done) return;  // the step kernel did not run (every block sees the same flag)
     const int nrec = f.nblocks + (f.part2 ? f.nblocks2 : 0);
-    const int q0 = blockIdx.x * f.fold_per, q1 = min(q0 + f.fold_per, nrec);
+    const int q0 = block * f.fold_per, q1 = min(q0 + f.fold_per, nrec);
     double A = 0.0, U = 0.0, V = 0.0, m = 0.0;
     int bad = 0;
     for (int q = q0 + (int)threadIdx.x; q < q1; q += FOLD_THREADS) {
@@ -220,11 +220,11 @@ __global__ __launch_bounds__(FOLD_THREADS) void k_fold(FinishArgs f) {
         m += r[3];
         bad |= r[4] != 0.0;
     }
-    block4_partials(f.fold, blockIdx.x, A, U, V, m, bad);
+    block4_partials(f.fold, block, A, U, V, m, bad);
     __shared__ int last;
     if (threadIdx.x == 0) {
         __threadfence();  // this block's record before its count
-        last = atomicAdd(&f.ctl->folded, 1u) == gridDim.x - 1;
+        last = atomicAdd(&f.ctl->folded, 1u) == (unsigned int)f.nfold - 1;
     }
     __syncthreads();
     if (!last) return;
@@ -232,18 +232,12 @@ __global__ __launch_bounds__(FOLD_THREADS) void k_fold(FinishArgs f) {
     if (threadIdx.x == 0) f.ctl->folded = 0;  // no other block touches it any more
     FinishArgs g = f;
     g.part = f.fold;
-    g.nblocks = gridDim.x;
+    g.nblocks = f.nfold;
     g.part2 = nullptr;
     g.nblocks2 = 0;
     finish_body<FOLD_THREADS>(g, 1);
 }
-
-// Batched finish: block s finishes solve s (slots with a null control block are idle).
-__global__ __launch_bounds__(FINISH_THREADS) void k_finish_batch(const FinishArgs* __restrict__ f, int nslots,
-                                                                 int advance) {
-    if ((int)blockIdx.x >= nslots || f[blockIdx.x].ctl == nullptr) return;
-    finish_body<FINISH_THREADS>(f[blockIdx.x], advance);
-}
+__global__ __launch_bounds__(FOLD_THREADS) void k_fold(FinishArgs f) { fold_body(f, blockIdx.x); }
 
 // The step body for one 64-lane block: strip (bx, by) of the solve described
 // by `a`; `stage` as StepArgs::stage. Used by the single-solve kernel and by the
@@ -504,6 +498,10 @@ __device__ __forceinline__ void step_strip(const StepArgs& a, const int bx, cons
         }
     }
     block_partials(a.mass_part, by * a.nbx + bx, amax, umax, vmax, msum, bad);
+    if (bx == 0 && by == 0 && lane == 0) {  // for the kernels after this one
+        ctl->ran = 1;
+        ctl->out = cur ^ 1;
+    }
 }
 
 // Four waves per SIMD (128 VGPRs): the strip's chains of dependent FP64 work and
@@ -544,6 +542,10 @@ __global__ __launch_bounds__(64) void k_step_lax(StepArgs a) {
     }
     const Layout L = a.L;
     const int cur = ctl->cur;
+    if (blockIdx.x == 0 && blockIdx.y == 0 && lane == 0) {
+        ctl->ran = 1;
+        ctl->out = cur ^ 1;
+    }
     const double dt = ctl->dt;
     const double* __restrict__ Ui = a.buf[cur];
     double* __restrict__ Uo = a.buf[cur ^ 1];
@@ -660,20 +662,13 @@ __global__ __launch_bounds__(MERGE_THREADS) void k_merge(MergeArgs a) {
     block_partials(a.part, blockIdx.x, amax, umax, vmax, msum, bad);
 }
 
-// Ghost-cell fill, phase 1: values from the donors of U_NEW (the state right
-// after the update, before any ghost is rewritten) into a compact buffer.
-// IDWBaseGFM/GFM_Bound.cpp:65-106, LinearBaseGFM/GFM_Bound.cpp:58-575,
-// BCGFM/BCGFM_Bound.cpp:81-175, HBCGFM/HBCGFM_Bound.cpp:163-178.
-__device__ __forceinline__ void fill_one(const FillArgs& a, const int gi) {
-    if (a.require_ran && !a.ctl->ran) return;
-    if (gi >= a.nghost) return;
-    const Ghost gh = a.ghosts[gi];
-    if (a.bc == IBTFO_SIMPLE_BOUND && gh.pick != a.level) return;
-    const int cur = a.use_cur ? a.ctl->cur : a.fixed;
-    const double* U = a.buf[cur];
-    // Boundary runs before Global_Boundary in the reference, so a donor in the
-    // domain ring still holds the ring of the previous state
-    const double* Uring = a.ring_prev ? a.buf[cur ^ 1] : U;
+// A ghost's new value v (Boundary): IDWBaseGFM/GFM_Bound.cpp:65-106,
+// LinearBaseGFM/GFM_Bound.cpp:58-575, BCGFM/BCGFM_Bound.cpp:81-175,
+// HBCGFM/HBCGFM_Bound.cpp:163-178, SimpleBound/LS_SimpleBound.cpp:38-105. U: the
+// state right after the update, before any ghost is rewritten; Uring: where the
+// donors marked in Ghost::ring are read.
+__device__ __forceinline__ void ghost_value(const FillArgs& a, const Ghost& gh, const double* U, const double* Uring,
+                                            double (&v4)[4]) {
     const long long PL = a.L.plane, P = a.L.pitch;
     const double gm1 = a.gm1;
     auto prim = [&](long long d, bool ring, double& r, double& u, double& v, double& p) {
@@ -699,8 +694,7 @@ __device__ __forceinline__ void fill_one(const FillArgs& a, const int gi) {
     if (a.bc == 1) {  // IDWBaseGFM
         if (!a.quirks && gh.a[0] + gh.a[1] + gh.a[2] + gh.a[3] == 0.0) {
             // corrected mode: no fluid donor, the ghost keeps its value
-            double* o = a.out + 4 * (long long)gi;
-            for (int k = 0; k < 4; k++) o[k] = U[gh.cell + k * PL];
+            for (int k = 0; k < 4; k++) v4[k] = U[gh.cell + k * PL];
             return;
         }
         idw(gh.d1, gh.ring & 15, gh.a, rw, uw, vw, pw);
@@ -716,8 +710,7 @@ __device__ __forceinline__ void fill_one(const FillArgs& a, const int gi) {
         // value (an earlier dependency level), any other from the state.
         const int IDX = gh.idx, IDY = gh.idy;
         if (IDX == 0 && IDY == 0) {  // no fluid within reach: the ghost keeps its value
-            double* o = a.out + 4 * (long long)gi;
-            for (int k = 0; k < 4; k++) o[k] = U[gh.cell + k * PL];
+            for (int k = 0; k < 4; k++) v4[k] = U[gh.cell + k * PL];
             return;
         }
         auto donor = [&](long long d, int earlier, bool ring, double& r, double& u, double& v, double& p) {
@@ -774,17 +767,45 @@ __device__ __forceinline__ void fill_one(const FillArgs& a, const int gi) {
         uw = un * n_x + ut * n_y;
         vw = un * n_y - ut * n_x;
     }
+    v4[0] = rw;
+    v4[1] = rw * uw;
+    v4[2] = rw * vw;
+    v4[3] = pw / gm1 + 0.5 * rw * (uw * uw + vw * vw);
+}
+
+// Ghost-cell fill, phase 1: the values into a compact buffer (stand-alone
+// Boundary, SimpleBound's dependency levels, the persistent batch kernel).
+__device__ __forceinline__ void fill_one(const FillArgs& a, const int gi) {
+    if (a.require_ran && !a.ctl->ran) return;
+    if (gi >= a.nghost) return;
+    const Ghost gh = a.ghosts[gi];
+    if (a.bc == IBTFO_SIMPLE_BOUND && gh.pick != a.level) return;
+    const int cur = a.use_cur ? a.ctl->cur : a.fixed;
+    const double* U = a.buf[cur];
+    // Boundary runs before Global_Boundary in the reference, so a donor in the
+    // domain ring still holds the ring of the previous state
+    double v[4];
+    ghost_value(a, gh, U, a.ring_prev ? a.buf[cur ^ 1] : U, v);
     double* o = a.out + 4 * (long long)gi;
-    o[0] = rw;
-    o[1] = rw * uw;
-    o[2] = rw * vw;
-    o[3] = pw / gm1 + 0.5 * rw * (uw * uw + vw * vw);
+    for (int k = 0; k < 4; k++) o[k] = v[k];
 }
 __global__ void k_fill(FillArgs a) { fill_one(a, blockIdx.x * blockDim.x + threadIdx.x); }
-// Batched fill: block b covers ghosts map[b].y .. +FILL_THREADS-1 of solve map[b].x.
-__global__ void k_fill_batch(const FillArgs* __restrict__ slots, const int2* __restrict__ map) {
-    const int2 m = map[blockIdx.x];
-    if (m.x >= 0) fill_one(slots[m.x], m.y + threadIdx.x);
+
+// The fill after a step in one phase, in place. The reference's Boundary reads
+// every donor before any ghost is rewritten; a step leaves non-active cells as
+// they were (U_NEW = U_OLD there), so a donor that is a ghost, or lies in the
+// ring, still holds its value in the state before the step, which nothing in
+// this launch writes. The active donors are written by no one here either.
+__device__ __forceinline__ void fill_in_place(const FillArgs& a, const int gi) {
+    if (gi >= a.nghost) return;
+    // the record and the flags in one round trip
+    const Ghost gh = a.ghosts[gi];
+    const int ran = a.ctl->ran, out = a.ctl->out;
+    if (!ran) return;
+    double* U = a.buf[out];
+    double v[4];
+    ghost_value(a, gh, U, a.buf[out ^ 1], v);
+    for (int k = 0; k < 4; k++) U[gh.cell + k * a.L.plane] = v[k];
 }
 
 // Ghost-cell fill, phase 2: write the values into the current state.
@@ -800,16 +821,15 @@ __device__ __forceinline__ void scatter_one(const FillArgs& a, const int gi) {
     U[c + 3 * PL] = v[3];
 }
 __global__ void k_scatter(FillArgs a) { scatter_one(a, blockIdx.x * blockDim.x + threadIdx.x); }
-__global__ void k_scatter_batch(const FillArgs* __restrict__ slots, const int2* __restrict__ map) {
-    const int2 m = map[blockIdx.x];
-    if (m.x >= 0) scatter_one(slots[m.x], m.y + threadIdx.x);
-}
 
 // Ring of the current state for the edge policies that are not fused into the
 // step (the reference policy for Lax; periodic; inflow). Reads the interior of
 // the current state, writes its ring; one thread per ring cell.
-__device__ __forceinline__ void edge_one(const EdgeArgs& a, const int q) {
-    if (a.require_ran && !a.ctl->ran) return;
+// PREV: beside the in-place fill: the state is the buffer the step wrote, and a
+// non-active source cell is read from the state before the step, where it has
+// the value it had before the fill.
+template <bool PREV> __device__ __forceinline__ void edge_one(const EdgeArgs& a, const int q) {
+    if (PREV ? !a.ctl->ran : a.require_ran && !a.ctl->ran) return;
     const Layout L = a.L;
     const int ng = L.ng, nx = L.nx, ny = L.ny;
     const int nring = L.M * L.N - nx * ny;
@@ -820,14 +840,22 @@ __device__ __forceinline__ void edge_one(const EdgeArgs& a, const int q) {
     if (q < nb) { j = q / L.M; i = q % L.M; }
     else if (q < 2 * nb) { int r = q - nb; j = ny + ng + r / L.M; i = r % L.M; }
     else { int r = q - 2 * nb; j = ng + r / (2 * ng); int s = r % (2 * ng); i = s < ng ? s : nx + s; }
-    double* U = a.buf[a.ctl->cur];
+    const int b = PREV ? a.ctl->out : a.ctl->cur;
+    double* U = a.buf[b];
+    auto source = [&](long long s) -> const double* {
+        if (PREV) {
+            const uint8_t t = a.type[s];
+            return t == 0 || t == 3 ? U : a.buf[b ^ 1];
+        }
+        return (a.unew_nf && a.type[s] != 0) ? a.unew_nf : U;
+    };
     const long long PL = L.plane;
     double v[4];
     if (a.kind == 1) {  // periodic
         int si = i < ng ? i + nx : (i >= nx + ng ? i - nx : i);
         int sj = j < ng ? j + ny : (j >= ny + ng ? j - ny : j);
         long long s = L.at(si, sj);
-        const double* S = (a.unew_nf && a.type[s] != 0) ? a.unew_nf : U;
+        const double* S = source(s);
         for (int k = 0; k < 4; k++) v[k] = S[s + k * PL];
     } else if (a.kind == 3) {
         // Test/PNGGeo/Global_Boudary.cpp:14-79 (U_NEW = the state before the ghost
@@ -836,10 +864,7 @@ __device__ __forceinline__ void edge_one(const EdgeArgs& a, const int q) {
         // the ring corners are not written
         const bool row = j < ng || j >= ny + ng;
         if (row && (i < ng || i >= nx + ng)) return;
-        auto src = [&](long long s, int k) {
-            const double* S = (a.unew_nf && a.type[s] != 0) ? a.unew_nf : U;
-            return S[s + k * PL];
-        };
+        auto src = [&](long long s, int k) { return source(s)[s + k * PL]; };
         if (row) {
             const int sr = j < ng ? 2 * ng - 1 : ny + ng - 1;
             const int rr = j < ng ? 2 * ng - j - 1 : 2 * (ny + ng) - 1 - j;
@@ -857,7 +882,7 @@ __device__ __forceinline__ void edge_one(const EdgeArgs& a, const int q) {
             int si = i >= nx + ng ? nx + ng - 1 : i;
             int sj = j < ng ? ng : (j >= ny + ng ? ny + ng - 1 : j);
             long long s = L.at(si, sj);
-            const double* S = (a.unew_nf && a.type[s] != 0) ? a.unew_nf : U;
+            const double* S = source(s);
             for (int k = 0; k < 4; k++) v[k] = S[s + k * PL];
         }
     } else {
@@ -866,18 +891,55 @@ __device__ __forceinline__ void edge_one(const EdgeArgs& a, const int q) {
     long long o = L.at(i, j);
     for (int k = 0; k < 4; k++) U[o + k * PL] = v[k];
 }
-__global__ void k_edge(EdgeArgs a) { edge_one(a, blockIdx.x * blockDim.x + threadIdx.x); }
-// Ghost fill phase 1 and the edge ring in one launch (independent work: the fill
-// reads ring donors from the previous state): blocks below nfb fill, the rest
-// write the ring.
-__global__ __launch_bounds__(FILL_THREADS) void k_fill_edge(FillArgs f, EdgeArgs e, int nfb) {
-    if ((int)blockIdx.x < nfb) fill_one(f, blockIdx.x * FILL_THREADS + threadIdx.x);
-    else edge_one(e, (blockIdx.x - nfb) * FILL_THREADS + threadIdx.x);
+__global__ void k_edge(EdgeArgs a) { edge_one<false>(a, blockIdx.x * blockDim.x + threadIdx.x); }
+
+// What follows a step's update in one launch: the dt / mass reduction and clock
+// (blocks below nfin), the ghost fill in place (the next nfb) and the edge ring.
+// They are independent given Ctl::ran and Ctl::out, which the step kernel wrote
+// and no block here changes (the finish sets ran to the value it has; it flips
+// cur, which the others do not read). Each is a few microseconds of latency, so
+// as launches of their own (finish, fill and ring, scatter) they cost a launch
+// each: 16.7 -> 10.9 us per step on 64x64 cells with a ghost-fluid body (1-row
+// strips), 39.6 -> 32.5 on the 800x400 channel, 253 -> 245 on 4096x2048 cut cells.
+__global__ __launch_bounds__(POST_THREADS) void k_post(FinishArgs f, FillArgs fl, EdgeArgs e, int nfin, int nfb) {
+    const int b = blockIdx.x;
+    if (b < nfin) {
+        if (nfin > 1) {
+            fold_body(f, b);
+        } else if (f.nblocks + (f.part2 ? f.nblocks2 : 0) <= FINISH_SMALL_MAX) {
+            if (threadIdx.x < 64) finish_small(f, f.advance);
+        } else {
+            finish_body<POST_THREADS>(f, f.advance);
+        }
+    } else if (b < nfin + nfb) {
+        fill_in_place(fl, (b - nfin) * POST_THREADS + threadIdx.x);
+    } else {
+        edge_one<true>(e, (b - nfin - nfb) * POST_THREADS + threadIdx.x);
+    }
 }
-// Batched edge ring: block b covers ring cells map[b].y .. +EDGE_THREADS-1 of solve map[b].x.
-__global__ void k_edge_batch(const EdgeArgs* __restrict__ slots, const int2* __restrict__ map) {
-    const int2 m = map[blockIdx.x];
-    if (m.x >= 0) edge_one(slots[m.x], m.y + threadIdx.x);
+
+// The same over a batch's solves: block s < nslots finishes solve s (idle slots
+// have a null control block), then the ghost and ring blocks of the maps
+// (gmap[b]: FILL_THREADS ghosts from .y of solve .x; rmap[b]: EDGE_THREADS ring cells).
+constexpr int POST_BATCH_THREADS = 128;
+__global__ __launch_bounds__(POST_BATCH_THREADS) void k_post_batch(
+    const FinishArgs* __restrict__ f, int nslots, int advance, const FillArgs* __restrict__ fill,
+    const int2* __restrict__ gmap, int ngb, const EdgeArgs* __restrict__ edge, const int2* __restrict__ rmap) {
+    static_assert(FILL_THREADS <= POST_BATCH_THREADS, "one ghost per thread");
+    int b = blockIdx.x;
+    if (b < nslots) {
+        if (f[b].ctl) finish_body<POST_BATCH_THREADS>(f[b], advance);
+        return;
+    }
+    b -= nslots;
+    if (b < ngb) {
+        const int2 m = gmap[b];
+        if (m.x >= 0 && threadIdx.x < FILL_THREADS) fill_in_place(fill[m.x], m.y + threadIdx.x);
+        return;
+    }
+    const int2 m = rmap[b - ngb];
+    if (m.x < 0) return;
+    for (int k = threadIdx.x; k < EDGE_THREADS; k += POST_BATCH_THREADS) edge_one<true>(edge[m.x], m.y + k);
 }
 
 // ------------------------------------------------------ persistent batched step
@@ -933,7 +995,7 @@ __global__ __launch_bounds__(64) void k_persist(PersistArgs p) {
                 }
             for (int w = blockIdx.x; w < nring; w += G) {
                 const int2 m = p.rmap[w];
-                for (int k = threadIdx.x; k < EDGE_THREADS; k += 64) edge_one(p.edge[m.x], m.y + k);
+                for (int k = threadIdx.x; k < EDGE_THREADS; k += 64) edge_one<false>(p.edge[m.x], m.y + k);
             }
             if (!grid_sync(p, target)) return;
             // Boundary phase 2
@@ -1092,20 +1154,11 @@ hipError_t launch_persist(int scheme, int rs, int lim, int prec, const PersistAr
     void* args[] = {(void*)&p};
     return hipLaunchKernel(persist_kernel(scheme, rs, lim, prec), dim3(blocks), dim3(64), args, 0, s);
 }
-hipError_t launch_finish_batch(const FinishArgs* f, int nslots, int advance, hipStream_t s) {
-    hipLaunchKernelGGL(k_finish_batch, dim3(nslots), dim3(FINISH_THREADS), 0, s, f, nslots, advance);
-    return hipGetLastError();
-}
-hipError_t launch_fill_batch(const FillArgs* f, const int2* map, int nblocks, hipStream_t s) {
-    hipLaunchKernelGGL(k_fill_batch, dim3(nblocks), dim3(FILL_THREADS), 0, s, f, map);
-    return hipGetLastError();
-}
-hipError_t launch_scatter_batch(const FillArgs* f, const int2* map, int nblocks, hipStream_t s) {
-    hipLaunchKernelGGL(k_scatter_batch, dim3(nblocks), dim3(FILL_THREADS), 0, s, f, map);
-    return hipGetLastError();
-}
-hipError_t launch_edge_batch(const EdgeArgs* e, const int2* map, int nblocks, hipStream_t s) {
-    hipLaunchKernelGGL(k_edge_batch, dim3(nblocks), dim3(EDGE_THREADS), 0, s, e, map);
+hipError_t launch_post_batch(const FinishArgs* f, int nslots, int advance, const FillArgs* fill, const int2* gmap,
+                             int nghost_blocks, const EdgeArgs* edge, const int2* rmap, int nring_blocks,
+                             hipStream_t s) {
+    hipLaunchKernelGGL(k_post_batch, dim3(nslots + nghost_blocks + nring_blocks), dim3(POST_BATCH_THREADS), 0, s, f,
+                       nslots, advance, fill, gmap, nghost_blocks, edge, rmap);
     return hipGetLastError();
 }
 // Batched status read-out: one record per slot (idle slots: ctl null -> zeros).
@@ -1136,14 +1189,6 @@ hipError_t launch_fill(const FillArgs& a, hipStream_t s) {
 hipError_t launch_scatter(const FillArgs& a, hipStream_t s) {
     if (a.nghost == 0) return hipSuccess;
     hipLaunchKernelGGL(k_scatter, dim3((a.nghost + FILL_THREADS - 1) / FILL_THREADS), dim3(FILL_THREADS), 0, s, a);
-    return hipGetLastError();
-}
-hipError_t launch_fill_edge(const FillArgs& f, const EdgeArgs& e, hipStream_t s) {
-    if (f.nghost == 0) return launch_edge(e, s);
-    const int nfb = (f.nghost + FILL_THREADS - 1) / FILL_THREADS;
-    const int nring = e.L.M * e.L.N - e.L.nx * e.L.ny;
-    const int neb = (nring + FILL_THREADS - 1) / FILL_THREADS;
-    hipLaunchKernelGGL(k_fill_edge, dim3(nfb + neb), dim3(FILL_THREADS), 0, s, f, e, nfb);
     return hipGetLastError();
 }
 hipError_t launch_edge(const EdgeArgs& a, hipStream_t s) {
@@ -1197,17 +1242,32 @@ hipError_t launch_reduce(const ReduceArgs& a, hipStream_t s) {
     f.advance = 0; f.reset = a.reset;
     return launch_finish(f, s);
 }
-hipError_t launch_finish(const FinishArgs& f, hipStream_t s) {
+// The fold blocks of a finish (FinishArgs::nfold, fold_per), 1: no fold
+static int fold_blocks(FinishArgs& f) {
     const int nrec = f.nblocks + (f.part2 ? f.nblocks2 : 0);
-    if (f.advance == 1 && f.fold && nrec >= FOLD_MIN_PARTS) {
-        FinishArgs g = f;
-        g.nfold = std::min(FOLD_MAX, (nrec + FOLD_THREADS - 1) / FOLD_THREADS);
-        g.fold_per = (nrec + g.nfold - 1) / g.nfold;
-        hipLaunchKernelGGL(k_fold, dim3(g.nfold), dim3(FOLD_THREADS), 0, s, g);
-        return hipGetLastError();
-    }
-    if (nrec <= FINISH_SMALL_MAX) hipLaunchKernelGGL(k_finish_small, dim3(1), dim3(64), 0, s, f);
+    if (f.advance != 1 || !f.fold || nrec < FOLD_MIN_PARTS) return 1;
+    f.nfold = std::min(FOLD_MAX, (nrec + FOLD_THREADS - 1) / FOLD_THREADS);
+    f.fold_per = (nrec + f.nfold - 1) / f.nfold;
+    return f.nfold;
+}
+hipError_t launch_finish(const FinishArgs& f, hipStream_t s) {
+    FinishArgs g = f;
+    const int nfold = fold_blocks(g);
+    const int nrec = f.nblocks + (f.part2 ? f.nblocks2 : 0);
+    if (nfold > 1) hipLaunchKernelGGL(k_fold, dim3(nfold), dim3(FOLD_THREADS), 0, s, g);
+    else if (nrec <= FINISH_SMALL_MAX) hipLaunchKernelGGL(k_finish_small, dim3(1), dim3(64), 0, s, f);
     else hipLaunchKernelGGL(k_finish, dim3(1), dim3(FINISH_THREADS), 0, s, f);
+    return hipGetLastError();
+}
+hipError_t launch_post(const FinishArgs& f, const FillArgs* fill, const EdgeArgs* edge, hipStream_t s) {
+    static_assert(POST_THREADS == FOLD_THREADS, "the fold's blocks are blocks of the post kernel");
+    FinishArgs g = f;
+    const int nfin = fold_blocks(g);
+    const int nfb = fill ? (fill->nghost + POST_THREADS - 1) / POST_THREADS : 0;
+    const int nring = edge ? edge->L.M * edge->L.N - edge->L.nx * edge->L.ny : 0;
+    const int neb = (nring + POST_THREADS - 1) / POST_THREADS;
+    hipLaunchKernelGGL(k_post, dim3(nfin + nfb + neb), dim3(POST_THREADS), 0, s, g, fill ? *fill : FillArgs(),
+                       edge ? *edge : EdgeArgs(), nfin, nfb);
     return hipGetLastError();
 }
 
