@@ -677,11 +677,13 @@ static int upload_aos(ibtfo_ctx* x, const double* U, int buf) { return upload_ao
 static int read_ctl_head(ibtfo_ctx* x, Ctl& c) {
     HIPCHK(hipStreamSynchronize(x->stream));
     HIPCHK(scopy(x, &c, x->ctl, offsetof(Ctl, log_dt), hipMemcpyDeviceToHost));
+    x->cur_guess = c.cur;
     return IBTFO_OK;
 }
 static int write_ctl_head(ibtfo_ctx* x, const Ctl& c) {
     HIPCHK(hipStreamSynchronize(x->stream));
     HIPCHK(scopy(x, x->ctl, &c, offsetof(Ctl, log_dt), hipMemcpyHostToDevice));
+    x->cur_guess = c.cur;
     return IBTFO_OK;
 }
 
@@ -757,6 +759,7 @@ extern "C" int ibtfo_initialize(ibtfo_ctx* x, int kind, const double* prm, int n
         HIPCHK(launch_uniform_state(x->state[0], x->state[1],
                                     x->cfg.boundary == IBTFO_SIMPLE_BOUND ? x->unew0 : nullptr, L.plane, U, x->ctl,
                                     x->stream));
+        x->cur_guess = 0;
         x->corner_host.assign(2 * 2 * L.ng * 4, 0.0);
         for (size_t q = 0; q < x->corner_host.size(); q++) x->corner_host[q] = U[q % 4];
         HIPCHK(hipMemcpyAsync(x->corner, x->corner_host.data(), x->corner_host.size() * sizeof(double),
@@ -932,6 +935,7 @@ static int enqueue_step(ibtfo_ctx* x, hipEvent_t* ev = nullptr, int k = 0) {
         const bool in_place = rk2_in_place(x);
         StepArgs s1 = x->sa;
         s1.stage = 1;
+        s1.in_hint = x->cur_guess;
         if (ev) HIPCHK(hipEventRecord(ev[0], x->stream));
         HIPCHK(launch_step(c.scheme, c.riemann, c.limiter, c.precision, s1, x->stream));
         if (ev) HIPCHK(hipEventRecord(ev[1], x->stream));
@@ -942,11 +946,14 @@ static int enqueue_step(ibtfo_ctx* x, hipEvent_t* ev = nullptr, int k = 0) {
         }
         StepArgs s2 = x->sa;
         s2.stage = in_place ? 3 : 2;
+        s2.in_hint = x->cur_guess ^ 1;  // either way: the buffer stage 1 wrote
         if (ev) HIPCHK(hipEventRecord(ev[2], x->stream));
         HIPCHK(launch_step(c.scheme, c.riemann, c.limiter, c.precision, s2, x->stream));
         if (ev) HIPCHK(hipEventRecord(ev[3], x->stream));
     } else {
         StepArgs s = x->sa;
+        s.in_hint = x->cur_guess;
+        x->cur_guess ^= 1;
         if (k > 0) {
             s.df = k == 1 ? 1 : 2;
             s.df_k = k & 1;
@@ -1039,8 +1046,9 @@ extern "C" int ibtfo_step_graph(ibtfo_ctx* x, int nsteps, int chunk) {
         if (x->graph) { (void)hipGraphExecDestroy(x->graph); x->graph = nullptr; }
         hipGraph_t g = nullptr;
         HIPCHK(hipStreamBeginCapture(x->stream, hipStreamCaptureModeThreadLocal));
-        int rc = IBTFO_OK;
-        rc = enqueue_steps(x, chunk);
+        const int guess = x->cur_guess;  // capturing takes no step
+        int rc = enqueue_steps(x, chunk);
+        x->cur_guess = guess;
         hipError_t e = hipStreamEndCapture(x->stream, &g);
         if (e == hipSuccess && rc == IBTFO_OK && g) e = hipGraphInstantiate(&x->graph, g, nullptr, nullptr, 0);
         if (g) (void)hipGraphDestroy(g);
@@ -1050,6 +1058,7 @@ extern "C" int ibtfo_step_graph(ibtfo_ctx* x, int nsteps, int chunk) {
     }
     int full = nsteps / chunk, rest = nsteps % chunk;
     for (int r = 0; r < full; r++) HIPCHK(hipGraphLaunch(x->graph, x->stream));
+    if (x->cfg.time == IBTFO_SINGLESTEP) x->cur_guess ^= (full * (long long)chunk) & 1;
     return ibtfo_step(x, rest);
 }
 

@@ -17,18 +17,6 @@ enum { SCH_LAX = 0, SCH_MUSCL = 1, SCH_MHM = 2, SCH_GODUNOV = 3 };
 enum { RS_HLL = 0, RS_HLLC = 1, RS_PVRS = 2, RS_SW = 3 };
 enum { LIM_MINMOD = 0, LIM_VANLEER = 1, LIM_VANALBADA = 2 };
 
-template <typename T> struct FpConst;
-template <> struct FpConst<double> {
-    static constexpr double half_ulp_one = 0x1p-53;  // half the spacing of doubles just above 1
-    static constexpr double tiny = 0x1p-968;         // below this b*half_ulp_one may round
-    static constexpr double huge = 0x1.fffffffffffffp+1023;
-};
-template <> struct FpConst<float> {
-    static constexpr float half_ulp_one = 0x1p-24f;
-    static constexpr float tiny = 0x1p-100f;
-    static constexpr float huge = 0x1.fffffep+127f;
-};
-
 // Square root. On the device, for x in [2^-767, 2^1023] (every sound speed and
 // shock factor of a physical state), the rsq seed + Goldschmidt refinement +
 // two residual corrections that the compiler's IEEE sqrt runs after its range
@@ -144,17 +132,14 @@ IB_HD float dq(float a, const Rcp<float>& r) { return a * r.y; }
 template <typename T> IB_HD T ddiv(T a, T b) { return dq(a, rcp_of(b)); }
 
 // minmod/Slope_limiter.H:4: (a*b > 0) ? ((a/b > 1) ? b : a) : 0.
-// For a*b > 0 the rounded quotient exceeds 1 exactly when |a| > |b|(1 + 2^-53)
-// (the tie at 1 + 2^-53 rounds to 1.0), which is tested without a division:
-// |a| - |b| is exact by Sterbenz whenever |a| < 2|b|. Tiny or infinite |b|
-// falls back to the quotient itself.
+// For a*b > 0 the rounded quotient exceeds 1 exactly when |a| > |b|: the next
+// number above |b| is larger by more than |b| 2^-53 (half the spacing above 1),
+// in the subnormal range too; equal infinities and NaN compare false both ways.
+// So no division, and with a = b the only case in which the order of the
+// arguments could matter, a cell's two slopes in one direction are one value.
 template <typename T> IB_HD T lim_minmod(T a, T b) {
-    if (!(a * b > T(0))) return T(0);
-    T A = ib_fabs(a), B = ib_fabs(b);
-    bool gt;
-    if (B >= FpConst<T>::tiny && B <= FpConst<T>::huge) gt = (A >= T(2) * B) || (A - B > B * FpConst<T>::half_ulp_one);
-    else gt = (a / b > T(1));
-    return gt ? b : a;
+    const T m = ib_fabs(a) > ib_fabs(b) ? b : a;
+    return a * b > T(0) ? m : T(0);
 }
 // VanLeer/Slope_limiter.H:4 as expanded at the call sites, whose second argument
 // is the unparenthesised difference P - Q: `(r*r + r) * b / (r*r + 1)` becomes
@@ -172,14 +157,23 @@ template <typename T> IB_HD T lim_vanleer_fixed(T a, T b) {
     T A = a + T(1e-7), B = b + T(1e-7);
     return (A * B > T(0)) ? ddiv(b * (A * (A + B)), A * A + B * B) : T(0);
 }
-// {lim(a, b), lim(b, a)} of lim_vanleer_fixed
-template <typename T> IB_HD void vanleer_pair(T a, T b, T& sab, T& sba) {
+// {lim(a, b), lim(b, a)} of lim_vanleer_fixed. FLAT evaluates the quotients before
+// the selects, so that the four components' chains overlap (a wave with few others
+// beside it); else each component becomes a branch of its own, with far fewer
+// registers (the marching strip: 118 VGPRs instead of 139).
+template <bool FLAT, typename T> IB_HD void vanleer_pair(T a, T b, T& sab, T& sba) {
     T A = a + T(1e-7), B = b + T(1e-7);
     T n = A + B;
     Rcp<T> rd = rcp_of(A * A + B * B);
-    bool pos = A * B > T(0);
-    sab = pos ? dq(b * (A * n), rd) : T(0);
-    sba = pos ? dq(a * (B * n), rd) : T(0);
+    const bool pos = A * B > T(0);
+    if (FLAT) {
+        const T qab = dq(b * (A * n), rd), qba = dq(a * (B * n), rd);
+        sab = pos ? qab : T(0);
+        sba = pos ? qba : T(0);
+    } else {
+        sab = pos ? dq(b * (A * n), rd) : T(0);
+        sba = pos ? dq(a * (B * n), rd) : T(0);
+    }
 }
 // VanAlbada/Slope_limiter.H:4 does not compile (undeclared r); its evident
 // intent, with r defined as in the sibling limiter.
@@ -197,13 +191,15 @@ template <int LIM, typename T> IB_HD T slope(T a, T P, T Q, bool quirks) {
 // lo = u0 + 0.5 lim(u0 - um, up - u0) is the cell's state on its upper face
 // (U_L of face +1/2), hi = u0 - 0.5 lim(up - u0, u0 - um) its state on its lower
 // face (U_R of face -1/2); recon() below evaluates the same expressions face by face.
-template <int LIM, typename T> IB_HD void slope_pair(const T* um, const T* u0, const T* up, T* lo, T* hi,
-                                                     bool quirks) {
+template <int LIM, bool FLAT, typename T> IB_HD void slope_pair(const T* um, const T* u0, const T* up, T* lo, T* hi,
+                                                                bool quirks) {
 #pragma unroll
     for (int k = 0; k < 4; k++) {
         T sl, sh;
-        if (LIM == LIM_VANLEER && !quirks) {
-            vanleer_pair(u0[k] - um[k], up[k] - u0[k], sl, sh);
+        if (LIM == LIM_MINMOD) {
+            sl = sh = lim_minmod(u0[k] - um[k], up[k] - u0[k]);
+        } else if (LIM == LIM_VANLEER && !quirks) {
+            vanleer_pair<FLAT>(u0[k] - um[k], up[k] - u0[k], sl, sh);
         } else {
             sl = slope<LIM>(u0[k] - um[k], up[k], u0[k], quirks);
             sh = slope<LIM>(up[k] - u0[k], u0[k], um[k], quirks);

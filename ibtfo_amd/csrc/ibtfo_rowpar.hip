@@ -8,94 +8,81 @@
 
 namespace ibtfo {
 
-// The update of cell (c, j) from its face fluxes (F, G on its upper x / y faces;
-// fm_lds[k * 64], gm_lds[k * 64] on its lower faces, in the LDS slots of the
-// lanes that computed them): the conservative or cut-cell update, floors,
-// dt/mass partial terms, the RK2 stage average, the store and the fused
-// Global_Boundary ring writes. The same statements as the update inside
-// step_strip, which keeps its own inline copy: factoring it out of the strip
-// kernel changed that kernel's register allocation (the mixed-precision
-// cut-cell variants went from 128 to 165 VGPRs, 4 to 3 waves per SIMD). The
-// two copies are held equal by the row-parallel tests, which compare the two
-// kernels' states bit for bit over every scheme, flux, boundary and stage.
+// The update of cell (c, j), of type tc, from its face fluxes (F, G on its upper
+// x / y faces; fm_lds[k * 64], gm_lds[k * 64] on its lower faces, in the LDS slots
+// of the lanes that computed them): the conservative or cut-cell update, floors,
+// dt/mass partial terms, the RK2 stage average (with U^n in uo), the store and the
+// fused Global_Boundary ring writes. The same statements as the update inside
+// step_strip, which keeps its own inline copy (LDS slots for the cell and the
+// fluxes); the row-parallel tests hold the two equal, comparing the two kernels'
+// states bit for bit over every scheme, flux, boundary and stage.
 template <int SCH, int RS, int LIM, typename T, bool CUT>
 __device__ __forceinline__ void update_cell(const StepArgs& a, const Layout& L, const int c, const int j,
-                                            const double (&w0)[4], const T (&F)[4], const T (&G)[4],
-                                            const T* fm_lds, const T* gm_lds, const double dt,
-                                            const Rcp<double>& r_dx, const Rcp<double>& r_dy,
-                                            const Rcp<double>& r_gm1, const double dtdx, const double dtdy,
-                                            double* __restrict__ Uo, const int stage, double& amax, double& umax,
-                                            double& vmax, double& msum, int& bad) {
+                                            const uint8_t tc, const double (&u0)[4], const double (&uo)[4],
+                                            const T (&F)[4], const T (&G)[4], const T* fm_lds, const T* gm_lds,
+                                            const double dt, const int quirks, const Rcp<double>& r_dx,
+                                            const Rcp<double>& r_dy, const Rcp<double>& r_gm1, const double dtdx,
+                                            const double dtdy, double* __restrict__ Uo, const int stage,
+                                            double& amax, double& umax, double& vmax, double& msum, int& bad) {
     constexpr bool FP64 = sizeof(T) == sizeof(double);
     const long long PL = L.plane;
     const double dx = a.dx, dy = a.dy;
     const int ng = L.ng, nx = L.nx, ny = L.ny;
-    double un[4];
     const long long o = L.at(c, j);
-    const uint8_t tc = a.type[o];
     const bool fluid = CUT ? (tc & 3) == 0 : tc == 0;
     const bool merged = CUT && (tc & MERGED_BIT);
+    bool floors = fluid;
+    double vol = 1.0;
+    double un[4] = {u0[0], u0[1], u0[2], u0[3]};
     if (fluid) {
 #pragma unroll
         for (int k = 0; k < 4; k++) {
-            if (FP64) {
-                double Fm = fm_lds[k * 64];
-                double v = w0[k] - dq(dt * ((double)F[k] - Fm), r_dx);
-                un[k] = v - dq(dt * ((double)G[k] - (double)gm_lds[k * 64]), r_dy);
-            } else {  // FP32 fluxes, FP64 accumulation
-                double Fm = (double)fm_lds[k * 64];
-                un[k] = w0[k] - dtdx * ((double)F[k] - Fm) - dtdy * ((double)G[k] - (double)gm_lds[k * 64]);
-            }
+            const double dF = (double)F[k] - (double)fm_lds[k * 64];
+            const double dG = (double)G[k] - (double)gm_lds[k * 64];
+            // FP64, or FP32 fluxes with FP64 accumulation
+            if (FP64) un[k] = (u0[k] - dq(dt * dF, r_dx)) - dq(dt * dG, r_dy);
+            else un[k] = u0[k] - dtdx * dF - dtdy * dG;
         }
-        if (stage == 0) {
-            if (!merged) {
-                floor_and_dt(a.gam, a.gm1, r_gm1, un, a.quirks, amax, umax, vmax, bad);
-            } else {  // a merge target: floored here, its partials come from the merge
-                double d0 = 0.0, d1 = 0.0, d2 = 0.0;
-                int db = 0;
-                floor_and_dt(a.gam, a.gm1, r_gm1, un, a.quirks, d0, d1, d2, db);
-            }
-        } else {
-            // RK2 (Heun): each stage's update takes the floors; the second
-            // stage then averages with U^n, which the output buffer holds
-            double d0 = 0.0, d1 = 0.0, d2 = 0.0;
-            int db = 0;
-            floor_and_dt(a.gam, a.gm1, r_gm1, un, a.quirks, d0, d1, d2, db);
-            if (stage >= 2) {
-#pragma unroll
-                for (int k = 0; k < 4; k++) un[k] = 0.5 * (Uo[o + k * PL] + un[k]);
-                dt_terms(a.gam, a.gm1, un, amax, umax, vmax, bad);
-            }
-        }
-        if (!merged) msum += un[0] * dx * dy;
     } else if (CUT && (tc & 3) == 3) {
         // cut cell: aperture-weighted face fluxes and the wall's pressure
         // force S p (S closes the cell's faces), over the fluid volume
         // alpha dx dy; small cells are merged (and floored) afterwards
         const CutCell cc = a.cut[a.cut_index[o]];
-        const double rho = w0[0], u0 = w0[1] / rho, v0 = w0[2] / rho;
-        const double pw = a.gm1 * (w0[3] - 0.5 * rho * (u0 * u0 + v0 * v0));
-        const double wall[4] = {0.0, pw * cc.sbx, pw * cc.sby, 0.0};
+        const PState<double> s0 = pstate(a.gm1, u0);
+        const double wall[4] = {0.0, s0.p * cc.sbx, s0.p * cc.sby, 0.0};
+        const Rcp<double> rv = rcp_of(cc.alpha * dx * dy);
 #pragma unroll
         for (int k = 0; k < 4; k++) {
             const double Fk = (double)F[k], Fm = (double)fm_lds[k * 64];
             const double Gk = (double)G[k], Gm = (double)gm_lds[k * 64];
-            double v = w0[k] - dt * ((cc.ae * Fk - cc.aw * Fm) * dy) / (cc.alpha * dx * dy);
-            un[k] = v - dt * ((cc.an * Gk - cc.as * Gm) * dx + wall[k]) / (cc.alpha * dx * dy);
+            const double v = u0[k] - dq(dt * ((cc.ae * Fk - cc.aw * Fm) * dy), rv);
+            un[k] = v - dq(dt * ((cc.an * Gk - cc.as * Gm) * dx + wall[k]), rv);
         }
         // a merge-group cell (small cell or target) takes its floors and
         // partials from the merge; the others are floored and counted here
-        if (!merged) {
-            floor_and_dt(a.gam, a.gm1, r_gm1, un, a.quirks, amax, umax, vmax, bad);
-            msum += cc.alpha * un[0] * dx * dy;
-        } else if (cc.alpha >= 0.5) {
-            double d0 = 0.0, d1 = 0.0, d2 = 0.0;
-            int db = 0;
-            floor_and_dt(a.gam, a.gm1, r_gm1, un, a.quirks, d0, d1, d2, db);
-        }
-    } else {
+        floors = !merged || cc.alpha >= 0.5;
+        vol = cc.alpha;
+    }
+    if (floors) {
+        double am = 0.0, um = 0.0, vm = 0.0;
+        int nb = 0;
+        floor_and_dt(a.gam, a.gm1, r_gm1, un, quirks, am, um, vm, nb);
+        if (stage >= 2) {
+            // RK2 (Heun): each stage's update takes the floors; the second stage
+            // then averages with U^n, which the output buffer holds
 #pragma unroll
-        for (int k = 0; k < 4; k++) un[k] = w0[k];
+            for (int k = 0; k < 4; k++) un[k] = 0.5 * (uo[k] + un[k]);
+            am = um = vm = 0.0;
+            nb = 0;
+            dt_terms(a.gam, a.gm1, un, am, um, vm, nb);
+        }
+        if (!merged) {
+            amax = am;
+            umax = um;
+            vmax = vm;
+            bad = nb;
+            msum = fluid ? un[0] * dx * dy : vol * un[0] * dx * dy;
+        }
     }
 #pragma unroll
     for (int k = 0; k < 4; k++) Uo[o + k * PL] = un[k];
@@ -137,28 +124,9 @@ __device__ __forceinline__ void update_cell(const StepArgs& a, const Layout& L, 
 // (k_finish_small: lane t takes records t, t + 64, ... in turn, then the
 // cross-lane max / sum), so dt, mass and the clock come out bit for bit as
 // they do with a finish kernel between the steps.
-constexpr int DF_PER_LANE = DF_MAX_REC / 64;
 __device__ __forceinline__ void df_reduce(const double* part, const int nrec, double& A, double& Um, double& Vm,
                                           double& m, int& bad) {
-    const int t = threadIdx.x & 63;
-    double ra[DF_PER_LANE], ru[DF_PER_LANE], rv[DF_PER_LANE], rm[DF_PER_LANE], rb[DF_PER_LANE];
-#pragma unroll
-    for (int b = 0; b < DF_PER_LANE; b++) {
-        const int q = t + 64 * b;
-        const double* r = part + PART_STRIDE * (long long)(q < nrec ? q : 0);
-        ra[b] = r[0]; ru[b] = r[1]; rv[b] = r[2]; rm[b] = r[3]; rb[b] = r[4];
-    }
-    A = 0.0; Um = 0.0; Vm = 0.0; m = 0.0;
-    bad = 0;
-#pragma unroll
-    for (int b = 0; b < DF_PER_LANE; b++) {
-        if (t + 64 * b >= nrec) break;
-        A = (A < ra[b]) ? ra[b] : A;
-        Um = (Um < ru[b]) ? ru[b] : Um;
-        Vm = (Vm < rv[b]) ? rv[b] : Vm;
-        m += rm[b];
-        bad |= rb[b] != 0.0;
-    }
+    lane_records<DF_MAX_REC>(nrec, [&](int q) { return part + PART_STRIDE * (long long)q; }, A, Um, Vm, m, bad);
     A = wave_max(A);
     Um = wave_max(Um);
     Vm = wave_max(Vm);
@@ -203,10 +171,15 @@ __device__ __forceinline__ DfHead df_head(const StepArgs& a, const bool first_bl
         h.iter = ctl->iter; h.done = ctl->done; h.cur = ctl->cur; h.pending = 0;
     } else {
         const int p = a.df_k ^ 1;
-        const DfHead prev = ctl->df[p];
+        const DfHead* q = &ctl->df[p];
+        static_assert(offsetof(DfHead, iter) % 8 == 0 && offsetof(DfHead, cur) % 8 == 0, "pairs read as 8 bytes");
+        const unsigned long long l[5] = {ld8_here(&q->dt), ld8_here(&q->now_t), ld8_here(&q->mass),
+                                         ld8_here(&q->iter), ld8_here(&q->cur)};
         double A, Um, Vm, m;
         int bad;
         df_reduce(a.df_part + (long long)p * DF_MAX_REC * PART_STRIDE, a.nbx * a.nby, A, Um, Vm, m, bad);
+        const DfHead prev{uniform_double(l[0]), uniform_double(l[1]), uniform_double(l[2]), uniform_half(l[3], 0),
+                          uniform_half(l[3], 1), uniform_half(l[4], 0), uniform_half(l[4], 1)};
         h = prev.pending ? df_advance(a, prev, A, Um, Vm, m, bad, first_block && threadIdx.x == 0) : prev;
     }
     h.pending = !h.done;
@@ -214,20 +187,42 @@ __device__ __forceinline__ DfHead df_head(const StepArgs& a, const bool first_bl
     return h;
 }
 
+// Orders a wave's own LDS exchanges: its LDS operations execute in order, so only
+// the compiler has to keep them so.
+__device__ __forceinline__ void wave_lds_order() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // Row-parallel strip (small grids, where a strip's rows marching one after the
 // other set the step's latency): the block has rows + 1 waves over the same
 // 60-column x `rows` strip as step_strip; wave w takes row j = j0 - 1 + w at
-// once. It loads rows j-1 .. j+2 of its column, reconstructs them, computes
-// the x faces of row j (for j >= j0, or in quirks mode where the y face may
-// take the aliased x flux) and the y face j+1/2, and after a block barrier the
-// waves of rows j0 .. j1-1 update their cells with the y flux of face j-1/2
-// from the wave below. Every face is computed by the same statements as in
+// once. It loads rows j-1 .. j+1 of its column (the top wave one more),
+// reconstructs row j in y and hands the lower-face state to the wave below (the
+// top wave reconstructs row j+1's itself), computes the x faces of row j (for
+// j >= j0, or in quirks mode where the y face may take the aliased x flux) and,
+// after a block barrier, the y face j+1/2; after another the waves of rows
+// j0 .. j1-1 update their cells with the y flux of face j-1/2 from the wave below.
+// Every face is computed by the same statements as in
 // step_strip, so the state is bit for bit the same; only the grouping of the
 // mass partial sum differs. Block barriers are reached by every wave.
+// The kernel is a chain of latencies. Everything it reads from memory is asked
+// for at its start, in one round trip (the cell types and RK2's U^n too, which
+// used to be read where the update needed them); the x exchange is within a wave
+// and takes no block barrier; the limiters are evaluated without branches (FLAT).
+// LDS per wave: 2 KB for the x exchange (cells, face states and fluxes in turn), 2 KB
+// for its lower-face states and its y fluxes, sized by the launch: with the 64 KB of
+// four arrays for 8 waves, two blocks filled a CU whatever their height.
+constexpr int rowpar_lds(int rows, size_t flux) { return (rows + 1) * 4 * 64 * (int)(2 * sizeof(double) + flux); }
 template <int SCH, int RS, int LIM, typename T, bool CUT>
 __device__ __forceinline__ void step_rowpar(const StepArgs& a, const int bx, const int by, const int stage) {
+    constexpr bool FP64 = sizeof(T) == sizeof(double);
+    // the cut-cell and mixed-precision forms exist in corrected mode only
+    const int quirks = CUT || !FP64 ? 0 : a.quirks;
     Ctl* ctl = a.ctl;
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    // the wave's number as a scalar: its row, addresses and branches are wave-uniform
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const Layout L = a.L;
     const long long PL = L.plane;
     const int ng = L.ng, nx = L.nx, ny = L.ny;
@@ -239,26 +234,32 @@ __device__ __forceinline__ void step_rowpar(const StepArgs& a, const int bx, con
     const int j = j0 - 1 + wv;
     const bool live = j < j1;  // the waves past a short last strip only reach the barriers
 
-    // rows j-1 .. j+2 of column c (in range for every live wave: ng >= 2) of both
-    // state buffers, read together with the control block: the rows' addresses
-    // do not depend on which buffer is current, so no load waits for another
-    // (on a latency-bound small grid that is one memory round trip less)
-    double q0[4][4], q1[4][4];
-    if (live) {
-        const long long o = L.at(cl, j - 1);
+    // Rows j-1 .. j+1 (top wave: j+2) of column c (in range: ng >= 2), read
+    // together with the control block from the buffer the host expects to be the
+    // input (StepArgs::in_hint), so that no load waits for another: on a
+    // latency-bound small grid that is one memory round trip less. Another buffer
+    // (a graph of an odd number of steps replayed) is read again below.
+    // Every load at the head of the kernel is unconditional (the waves past a short
+    // last strip read the top row's), so that none waits in a branch.
+    double wm[4], w0[4], w1[4], w2[4] = {0.0, 0.0, 0.0, 0.0};
+    const bool top = j == j1 - 1;
+    const int jl = min(j, j1 - 1);
+    auto load_rows = [&](const double* U) {
+        const double* r = U + L.at(0, jl - 1);
 #pragma unroll
-        for (int r = 0; r < 4; r++)
+        for (int k = 0; k < 4; k++) {
+            wm[k] = ld_here(r + k * PL + cl);
+            w0[k] = ld_here(r + k * PL + L.pitch + cl);
+            w1[k] = ld_here(r + k * PL + 2 * L.pitch + cl);
+        }
+        if (top) {
 #pragma unroll
-            for (int k = 0; k < 4; k++) {
-                q0[r][k] = a.buf[0][o + r * L.pitch + k * PL];
-                q1[r][k] = a.buf[1][o + r * L.pitch + k * PL];
-            }
-    } else {
-#pragma unroll
-        for (int r = 0; r < 4; r++)
-#pragma unroll
-            for (int k = 0; k < 4; k++) q0[r][k] = q1[r][k] = 0.0;
-    }
+            for (int k = 0; k < 4; k++) w2[k] = ld_here(r + k * PL + 3 * L.pitch + cl);
+        }
+    };
+    const CtlLoads cl_now = ctl_now(ctl);
+    load_rows(a.in_hint ? a.buf[1] : a.buf[0]);
+    const uint8_t tc = __hip_atomic_load(a.type + L.at(cl, jl), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
     int cur;
     double dt;
     if (a.df) {
@@ -267,19 +268,20 @@ __device__ __forceinline__ void step_rowpar(const StepArgs& a, const int bx, con
         cur = h.cur;
         dt = h.dt;
     } else {
-        if (ctl->done) {
+        const CtlNow now = ctl_value(cl_now);
+        if (now.done) {
             if (bx == 0 && by == 0 && threadIdx.x == 0) ctl->ran = 0;
             return;
         }
-        cur = ctl->cur ^ (stage == 3 ? 1 : 0);  // the input buffer
-        dt = ctl->dt;
+        cur = now.cur ^ (stage == 3 ? 1 : 0);  // the input buffer
+        dt = now.dt;
         if (bx == 0 && by == 0 && threadIdx.x == 0) {
             ctl->ran = 1;
             ctl->out = cur ^ 1;
         }
     }
-    const double* __restrict__ Ui = a.buf[cur];
-    double* __restrict__ Uo = a.buf[cur ^ 1];
+    const double* __restrict__ Ui = cur ? a.buf[1] : a.buf[0];
+    double* __restrict__ Uo = cur ? a.buf[0] : a.buf[1];
     GasT<T> g;
     g.gam = (T)a.gam; g.gm1 = (T)a.gm1; g.gp1 = (T)a.gp1; g.c1 = (T)a.c1;
     g.r_gam = Rcp<T>{(T)a.gam, (T)a.r_gam};
@@ -290,10 +292,10 @@ __device__ __forceinline__ void step_rowpar(const StepArgs& a, const int bx, con
     const Rcp<double> r_dx{a.dx, a.r_dx}, r_dy{a.dy, a.r_dy}, r_gm1{a.gm1, a.r_gm1};
     const double dtdx = dt * a.r_dx, dtdy = dt * a.r_dy;  // mixed form only
 
-    __shared__ double rb[ROWPAR_MAX_ROWS + 1][4][64];
-    __shared__ double hb[ROWPAR_MAX_ROWS + 1][4][64];
-    __shared__ T fb[ROWPAR_MAX_ROWS + 1][4][64];
-    __shared__ T gb[ROWPAR_MAX_ROWS + 1][4][64];
+    extern __shared__ double lds[];
+    double* xb = lds + wv * 256;                                             // this wave's x exchange
+    double* hb = lds + (a.rows + 1) * 256;                                   // every wave's lower-face states
+    T* gb = (T*)(hb + (a.rows + 1) * 256);                                   // and y fluxes
     __shared__ double sp[ROWPAR_MAX_ROWS + 1][5];
 
     // reference Global_Boundary corners (Test/Sod/Global_Boudary.cpp:62-75), as in step_strip
@@ -311,58 +313,69 @@ __device__ __forceinline__ void step_rowpar(const StepArgs& a, const int bx, con
         }
     }
 
-    double wm[4], w0[4], w1[4], w2[4];
+    if (cur != a.in_hint) load_rows(Ui);
+    const bool upd = live && j >= j0 && lane >= 2 && lane < STRIP_W + 2 && c < nx + ng;
+    double uo[4] = {0.0, 0.0, 0.0, 0.0};  // RK2's U^n
+    if (stage >= 2 && upd) {
 #pragma unroll
-    for (int k = 0; k < 4; k++) {
-        wm[k] = cur ? q1[0][k] : q0[0][k];
-        w0[k] = cur ? q1[1][k] : q0[1][k];
-        w1[k] = cur ? q1[2][k] : q0[2][k];
-        w2[k] = cur ? q1[3][k] : q0[3][k];
+        for (int k = 0; k < 4; k++) uo[k] = Uo[L.at(c, j) + k * PL];
     }
-    const bool xrow = live && (j >= j0 || (a.quirks && RS != RS_SW));
+    double ylo[4], yhi[4];
+    if (live) {
+        cell_states<SCH, LIM, T, true>(wm, w0, w1, ylo, yhi, quirks);
+#pragma unroll
+        for (int k = 0; k < 4; k++) hb[(wv * 4 + k) * 64 + lane] = yhi[k];
+        if (top) {  // the state of row j + 1, which no wave of the block holds
+            double lo_unused[4];
+            cell_states<SCH, LIM, T, true>(w0, w1, w2, lo_unused, yhi, quirks);
+        }
+    }
+    const bool xrow = live && (j >= j0 || (quirks && RS != RS_SW));
     const int ln = min(lane + 1, 63), lp = max(lane - 1, 0);
     T F[4] = {0, 0, 0, 0};
-    double xp[4], xlo[4];
-#pragma unroll
-    for (int k = 0; k < 4; k++) rb[wv][k][lane] = w0[k];
-    __syncthreads();
     if (xrow) {
-        double xm[4], xhi[4];
+        double xm[4], xp[4], xlo[4], xhi[4], xr[4];
+#pragma unroll
+        for (int k = 0; k < 4; k++) xb[k * 64 + lane] = w0[k];
+        wave_lds_order();
 #pragma unroll
         for (int k = 0; k < 4; k++) {
-            xm[k] = rb[wv][k][lp];
-            xp[k] = rb[wv][k][ln];
+            xm[k] = xb[k * 64 + lp];
+            xp[k] = xb[k * 64 + ln];
         }
-        cell_states<SCH, LIM, T>(xm, w0, xp, xlo, xhi, a.quirks);
+        cell_states<SCH, LIM, T, true>(xm, w0, xp, xlo, xhi, quirks);
+        wave_lds_order();
 #pragma unroll
-        for (int k = 0; k < 4; k++) hb[wv][k][lane] = xhi[k];
+        for (int k = 0; k < 4; k++) xb[k * 64 + lane] = xhi[k];
+        wave_lds_order();
+#pragma unroll
+        for (int k = 0; k < 4; k++) xr[k] = xb[k * 64 + ln];
+        xface<SCH, RS>(g, a.gm1, dtc, quirks, [&](int k) { return w0[k]; }, [&](int k) { return xp[k]; }, xlo, xr, F);
     }
     __syncthreads();
-    if (xrow) {
-        double xr[4];
-#pragma unroll
-        for (int k = 0; k < 4; k++) xr[k] = hb[wv][k][ln];
-        xface<SCH, RS>(g, a.gm1, dtc, a.quirks, [&](int k) { return w0[k]; }, [&](int k) { return xp[k]; }, xlo, xr, F);
-    }
     T G[4] = {0, 0, 0, 0};
     if (live) {
-        double ylo[4], hi_unused[4], ynlo[4], ynhi[4];
-        cell_states<SCH, LIM, T>(wm, w0, w1, ylo, hi_unused, a.quirks);
-        cell_states<SCH, LIM, T>(w0, w1, w2, ynlo, ynhi, a.quirks);
-        yface<SCH, RS>(g, a.gm1, dtc, a.quirks, [&](int k) { return w0[k]; }, [&](int k) { return w1[k]; }, ylo, ynhi,
+        if (!top) {
+#pragma unroll
+            for (int k = 0; k < 4; k++) yhi[k] = hb[((wv + 1) * 4 + k) * 64 + lane];
+        }
+        yface<SCH, RS>(g, a.gm1, dtc, quirks, [&](int k) { return w0[k]; }, [&](int k) { return w1[k]; }, ylo, yhi,
                        [&](int k) { return F[k]; }, G);
     }
+    wave_lds_order();
+    T* fb = (T*)xb;
 #pragma unroll
     for (int k = 0; k < 4; k++) {
-        fb[wv][k][lane] = F[k];
-        gb[wv][k][lane] = G[k];
+        fb[k * 64 + lane] = F[k];
+        gb[(wv * 4 + k) * 64 + lane] = G[k];
     }
     __syncthreads();
     double amax = 0.0, umax = 0.0, vmax = 0.0, msum = 0.0;
     int bad = 0;
-    if (live && j >= j0 && lane >= 2 && lane < STRIP_W + 2 && c < nx + ng)
-        update_cell<SCH, RS, LIM, T, CUT>(a, L, c, j, w0, F, G, &fb[wv][0][lane - 1], &gb[wv - 1][0][lane], dt,
-                                          r_dx, r_dy, r_gm1, dtdx, dtdy, Uo, stage, amax, umax, vmax, msum, bad);
+    if (upd)
+        update_cell<SCH, RS, LIM, T, CUT>(a, L, c, j, tc, w0, uo, F, G, fb + lane - 1, gb + (wv - 1) * 256 + lane, dt,
+                                          quirks, r_dx, r_dy, r_gm1, dtdx, dtdy, Uo, stage, amax, umax, vmax, msum,
+                                          bad);
     // one partial record per block: each wave's, then the waves in order
     amax = wave_max(amax);
     umax = wave_max(umax);
@@ -417,12 +430,13 @@ __global__ __launch_bounds__(64 * (ROWPAR_MAX_ROWS + 1)) void k_step_rowpar(Step
 template <int SCH, int RS, int LIM>
 static hipError_t go_rowpar(int prec, const StepArgs& a, hipStream_t s) {
     const dim3 grid(a.nbx, a.nby), block(64 * (a.rows + 1));
+    const int l64 = rowpar_lds(a.rows, sizeof(double)), l32 = rowpar_lds(a.rows, sizeof(float));
     if (a.cut) {
-        if (prec == 1) hipLaunchKernelGGL((k_step_rowpar<SCH, RS, LIM, float, true>), grid, block, 0, s, a);
-        else hipLaunchKernelGGL((k_step_rowpar<SCH, RS, LIM, double, true>), grid, block, 0, s, a);
+        if (prec == 1) hipLaunchKernelGGL((k_step_rowpar<SCH, RS, LIM, float, true>), grid, block, l32, s, a);
+        else hipLaunchKernelGGL((k_step_rowpar<SCH, RS, LIM, double, true>), grid, block, l64, s, a);
     } else {
-        if (prec == 1) hipLaunchKernelGGL((k_step_rowpar<SCH, RS, LIM, float, false>), grid, block, 0, s, a);
-        else hipLaunchKernelGGL((k_step_rowpar<SCH, RS, LIM, double, false>), grid, block, 0, s, a);
+        if (prec == 1) hipLaunchKernelGGL((k_step_rowpar<SCH, RS, LIM, float, false>), grid, block, l32, s, a);
+        else hipLaunchKernelGGL((k_step_rowpar<SCH, RS, LIM, double, false>), grid, block, l64, s, a);
     }
     return hipGetLastError();
 }

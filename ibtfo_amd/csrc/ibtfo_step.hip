@@ -82,27 +82,33 @@ template <int NT> __device__ __forceinline__ void finish_body(const FinishArgs& 
     double A = 0.0, Um = 0.0, Vm = 0.0, m = 0.0;
     int bad = 0;
     // batches of FB records per thread, all loads issued before any is used, so
-    // one memory round trip covers FB records (the loop is latency bound)
-    constexpr int FB = 8;
+    // one memory round trip covers FB records (the loop is latency bound); one
+    // record per thread where that covers them (no loads of records not there)
     const int nrec = f.nblocks + (f.part2 ? f.nblocks2 : 0);
-    for (int q0 = t; q0 < nrec; q0 += FB * NT) {
-        double ra[FB], ru[FB], rv[FB], rm[FB], rb[FB];
+    auto run = [&](auto fb) {
+        constexpr int FB = decltype(fb)::value;
+        for (int q0 = t; q0 < nrec; q0 += FB * NT) {
+            double ra[FB], ru[FB], rv[FB], rm[FB], rb[FB];
 #pragma unroll
-        for (int b = 0; b < FB; b++) {
-            const int q = q0 + b * NT;
-            const double* r = part_rec(f, q < nrec ? q : q0);
-            ra[b] = r[0]; ru[b] = r[1]; rv[b] = r[2]; rm[b] = r[3]; rb[b] = r[4];
-        }
+            for (int b = 0; b < FB; b++) {
+                const int q = q0 + b * NT;
+                const double* r = part_rec(f, q < nrec ? q : q0);
+                ra[b] = ld_here(r); ru[b] = ld_here(r + 1); rv[b] = ld_here(r + 2); rm[b] = ld_here(r + 3);
+                rb[b] = ld_here(r + 4);
+            }
 #pragma unroll
-        for (int b = 0; b < FB; b++) {
-            if (q0 + b * NT >= nrec) break;
-            A = (A < ra[b]) ? ra[b] : A;
-            Um = (Um < ru[b]) ? ru[b] : Um;
-            Vm = (Vm < rv[b]) ? rv[b] : Vm;
-            m += rm[b];
-            bad |= rb[b] != 0.0;
+            for (int b = 0; b < FB; b++) {
+                if (q0 + b * NT >= nrec) break;
+                A = (A < ra[b]) ? ra[b] : A;
+                Um = (Um < ru[b]) ? ru[b] : Um;
+                Vm = (Vm < rv[b]) ? rv[b] : Vm;
+                m += rm[b];
+                bad |= rb[b] != 0.0;
+            }
         }
-    }
+    };
+    if (nrec <= NT) run(std::integral_constant<int, 1>());
+    else run(std::integral_constant<int, 8>());
     sA[t] = A; sU[t] = Um; sV[t] = Vm; sM[t] = m; sB[t] = bad;
     __syncthreads();
     for (int w = NT / 2; w > 0; w >>= 1) {
@@ -125,7 +131,6 @@ __global__ __launch_bounds__(FINISH_THREADS) void k_finish(FinishArgs f) {
 // grids, whose step is a chain of latencies): each lane reads its records in
 // one round trip, the control fields are read beside them rather than first,
 // and the lanes reduce through cross-lane shuffles instead of an LDS tree.
-constexpr int FINISH_SMALL_PER_LANE = FINISH_SMALL_MAX / 64;
 __device__ __forceinline__ void finish_small(const FinishArgs& f, const int advance) {
     Ctl* ctl = f.ctl;
     if (advance == 2) {
@@ -142,25 +147,9 @@ __device__ __forceinline__ void finish_small(const FinishArgs& f, const int adva
     const int done = ctl->done;
     const double now_t = ctl->now_t;
     const int iter = ctl->iter;
-    double ra[FINISH_SMALL_PER_LANE], ru[FINISH_SMALL_PER_LANE], rv[FINISH_SMALL_PER_LANE], rm[FINISH_SMALL_PER_LANE],
-        rb[FINISH_SMALL_PER_LANE];
-#pragma unroll
-    for (int b = 0; b < FINISH_SMALL_PER_LANE; b++) {
-        const int q = t + 64 * b;
-        const double* r = part_rec(f, q < nrec ? q : 0);
-        ra[b] = r[0]; ru[b] = r[1]; rv[b] = r[2]; rm[b] = r[3]; rb[b] = r[4];
-    }
-    double A = 0.0, Um = 0.0, Vm = 0.0, m = 0.0;
-    int bad = 0;
-#pragma unroll
-    for (int b = 0; b < FINISH_SMALL_PER_LANE; b++) {
-        if (t + 64 * b >= nrec) break;
-        A = (A < ra[b]) ? ra[b] : A;
-        Um = (Um < ru[b]) ? ru[b] : Um;
-        Vm = (Vm < rv[b]) ? rv[b] : Vm;
-        m += rm[b];
-        bad |= rb[b] != 0.0;
-    }
+    double A, Um, Vm, m;
+    int bad;
+    lane_records<FINISH_SMALL_MAX>(nrec, [&](int q) { return part_rec(f, q); }, A, Um, Vm, m, bad);
     A = wave_max(A);
     Um = wave_max(Um);
     Vm = wave_max(Vm);
@@ -244,21 +233,55 @@ __global__ __launch_bounds__(FOLD_THREADS) void k_fold(FinishArgs f) { fold_body
 // batched kernel, whose blocks each pick their solve from a block map.
 // PER: the periodic ring of the output is written beside the stores (edge_fused = 2;
 // its own kernel, so that the other kernels' register allocation is not touched).
-template <int SCH, int RS, int LIM, typename T, bool CUT, bool PER = false>
+template <int SCH, int RS, int LIM, typename T, bool CUT, bool PER = false, bool HINT = false>
 __device__ __forceinline__ void step_strip(const StepArgs& a, const int bx, const int by, const int stage) {
     constexpr bool FP64 = sizeof(T) == sizeof(double);
     Ctl* ctl = a.ctl;
     const int lane = threadIdx.x;
-    if (ctl->done) {
+    const Layout L = a.L;
+    const long long PL = L.plane;
+    const int ng = L.ng, nx = L.nx, ny = L.ny;
+    const int cb = ng + STRIP_W * bx;  // first interior column of the strip
+    const int c = cb - 2 + lane;
+    const int cl = min(max(c, 0), L.M - 1);
+    const int j0 = ng + a.rows * by;
+    const int j1 = min(j0 + a.rows, ny + ng);
+    // Rows are addressed as a wave-uniform base (scalar registers) plus the lane's
+    // 32-bit column offset: no 64-bit address arithmetic in the vector unit.
+    const unsigned int co = (unsigned int)cl * 8u, ct = (unsigned int)cl;
+    auto ld = [&](const double* base, int row, int k) {
+        return *(const double*)((const char*)(base + L.at(0, row) + k * PL) + co);
+    };
+    auto st = [&](double* base, int row, int k, double v) {
+        *(double*)((char*)(base + L.at(0, row) + k * PL) + co) = v;
+    };
+    // column window: w[0..2] = rows j, j+1, j+2 of column c at iteration j
+    double wm[4], w[3][4];
+    auto load_window = [&](const double* U) {
+        auto here = [&](int row, int k) {
+            return ld_here((const double*)((const char*)(U + L.at(0, row) + k * PL) + co));
+        };
+#pragma unroll
+        for (int k = 0; k < 4; k++) wm[k] = here(j0 - 2, k);
+#pragma unroll
+        for (int r = 0; r < 3; r++)
+#pragma unroll
+            for (int k = 0; k < 4; k++) w[r][k] = here(j0 - 1 + r, k);
+    };
+    // HINT: the first rows come from the buffer the host expects to be the input,
+    // together with the control block; another buffer is read again below
+    const CtlLoads cl_now = ctl_now(ctl);
+    if (HINT) load_window(a.in_hint ? a.buf[1] : a.buf[0]);
+    const CtlNow now = ctl_value(cl_now);
+    if (now.done) {
         if (bx == 0 && by == 0 && lane == 0) ctl->ran = 0;
         return;
     }
-    const Layout L = a.L;
-    const int cur = ctl->cur ^ (stage == 3 ? 1 : 0);  // the input buffer
-    const double dt = ctl->dt;
-    const double* __restrict__ Ui = a.buf[cur];
-    double* __restrict__ Uo = a.buf[cur ^ 1];
-    const long long PL = L.plane;
+    const int cur = now.cur ^ (stage == 3 ? 1 : 0);  // the input buffer
+    const double dt = now.dt;
+    const double* __restrict__ Ui = cur ? a.buf[1] : a.buf[0];
+    double* __restrict__ Uo = cur ? a.buf[0] : a.buf[1];
+    if (!HINT || cur != a.in_hint) load_window(Ui);
     GasT<T> g;
     g.gam = (T)a.gam; g.gm1 = (T)a.gm1; g.gp1 = (T)a.gp1; g.c1 = (T)a.c1;
     g.r_gam = Rcp<T>{(T)a.gam, (T)a.r_gam};
@@ -269,15 +292,8 @@ __device__ __forceinline__ void step_strip(const StepArgs& a, const int bx, cons
     const Rcp<double> r_dx{a.dx, a.r_dx}, r_dy{a.dy, a.r_dy}, r_gm1{a.gm1, a.r_gm1};
     const double dtdx = dt * a.r_dx, dtdy = dt * a.r_dy;  // mixed form only
     const double dx = a.dx, dy = a.dy;
-    const int ng = L.ng, nx = L.nx, ny = L.ny;
     // the cut-cell and mixed-precision forms exist in corrected mode only
     const int quirks = CUT || !FP64 ? 0 : a.quirks;
-
-    const int cb = ng + STRIP_W * bx;  // first interior column of the strip
-    const int c = cb - 2 + lane;
-    const int cl = min(max(c, 0), L.M - 1);
-    const int j0 = ng + a.rows * by;
-    const int j1 = min(j0 + a.rows, ny + ng);
 
     // 10 KB in all (FP64), so that 16 blocks, four waves per SIMD, fit a CU's 160 KB
     __shared__ double rb[4][64];     // row values of columns cb-2 .. cb+61 (read before the next barrier)
@@ -304,27 +320,8 @@ __device__ __forceinline__ void step_strip(const StepArgs& a, const int bx, cons
         }
     }
 
-    // Rows are addressed as a wave-uniform base (scalar registers) plus the lane's
-    // 32-bit column offset: no 64-bit address arithmetic in the vector unit.
-    const unsigned int co = (unsigned int)cl * 8u, ct = (unsigned int)cl;
-    auto ld = [&](const double* base, int row, int k) {
-        return *(const double*)((const char*)(base + L.at(0, row) + k * PL) + co);
-    };
-    auto st = [&](double* base, int row, int k, double v) {
-        *(double*)((char*)(base + L.at(0, row) + k * PL) + co) = v;
-    };
-
-    // column window: w[0..2] = rows j, j+1, j+2 of column c at iteration j;
     // ylb = the y state of row j on its upper face (from the previous pair)
-    double w[3][4];
     {
-        double wm[4];
-#pragma unroll
-        for (int k = 0; k < 4; k++) wm[k] = ld(Ui, j0 - 2, k);
-#pragma unroll
-        for (int r = 0; r < 3; r++)
-#pragma unroll
-            for (int k = 0; k < 4; k++) w[r][k] = ld(Ui, j0 - 1 + r, k);
         double hi_unused[4], ylo[4];
         cell_states<SCH, LIM, T>(wm, w[0], w[1], ylo, hi_unused, quirks);
 #pragma unroll
@@ -336,13 +333,17 @@ __device__ __forceinline__ void step_strip(const StepArgs& a, const int bx, cons
     const bool upd_col = lane >= 2 && lane < STRIP_W + 2 && c < nx + ng;
     const int ln = min(lane + 1, 63), lp = max(lane - 1, 0);
 
+    uint8_t tn = 0;  // type of the row after this one
     for (int j = j0 - 1; j < j1; j++) {
-        // prefetch the next window row (none after the last row: it would only be
-        // discarded; j + 3 <= ny + ng + 1 lies in the grid, ng >= 2)
+        // prefetch the next window row and cell type (none after the last row: they
+        // would only be discarded; j + 3 <= ny + ng + 1 lies in the grid, ng >= 2).
+        // Read where the update needs it, the type cost each row a memory latency.
         double nw[4];
+        const uint8_t tc = tn;
         if (j + 1 < j1) {
 #pragma unroll
             for (int k = 0; k < 4; k++) nw[k] = ld(Ui, j + 3, k);
+            tn = *(a.type + L.at(0, j + 1) + ct);
         }
         // FP64: row j's cells and x fluxes stay in LDS (rb, fb) and are read back
         // where they are used, so that no register holds them through the y face.
@@ -389,7 +390,6 @@ __device__ __forceinline__ void step_strip(const StepArgs& a, const int bx, cons
             __syncthreads();
             if (upd_col) {
                 double u0[4], un[4];
-                const uint8_t tc = *(a.type + L.at(0, j) + ct);
                 const bool fluid = CUT ? (tc & 3) == 0 : tc == 0;
                 const bool merged = CUT && (tc & MERGED_BIT);
                 // the floors; the dt / mass partials (a merge group's come from the merge)
@@ -511,11 +511,11 @@ __device__ __forceinline__ void step_strip(const StepArgs& a, const int bx, cons
 constexpr int step_waves(int rs) { return rs == RS_PVRS ? 1 : 4; }
 template <int SCH, int RS, int LIM, typename T, bool CUT>
 __global__ __launch_bounds__(64, step_waves(RS)) void k_step(StepArgs a) {
-    step_strip<SCH, RS, LIM, T, CUT>(a, blockIdx.x, blockIdx.y, a.stage);
+    step_strip<SCH, RS, LIM, T, CUT, false, true>(a, blockIdx.x, blockIdx.y, CUT ? 0 : a.stage);  // cut cells: one stage
 }
 template <int SCH, int RS, int LIM, typename T>
 __global__ __launch_bounds__(64, step_waves(RS)) void k_step_periodic(StepArgs a) {
-    step_strip<SCH, RS, LIM, T, false, true>(a, blockIdx.x, blockIdx.y, a.stage);
+    step_strip<SCH, RS, LIM, T, false, true, true>(a, blockIdx.x, blockIdx.y, a.stage);
 }
 
 // Batched step: one launch over the strips of many solves. Block b runs strip
