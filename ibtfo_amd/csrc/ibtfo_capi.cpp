@@ -81,18 +81,38 @@ static Layout make_layout(const ibtfo_config* c) {
     return L;
 }
 
-// Step-kernel grid: strips of STRIP_W columns x `rows` rows. rows_override = 0
-// picks the default shape (about 8192 blocks, 32 waves per CU to cover the
-// latency of a 3-wave occupancy, and at least 4 rows per strip);
-// ibtfo_set_rows / ibtfo_autotune choose another.
-static int step_grid(const Layout& L, int rows_override, int* nbx, int* nby, int* rows) {
+// Step-kernel grid: strips of STRIP_W columns x `rows` rows (at most the grid's).
+static int step_grid(const Layout& L, int rows, int* nbx, int* nby, int* out_rows) {
     *nbx = (L.nx + STRIP_W - 1) / STRIP_W;
-    int want_y = std::max(1, 8192 / *nbx);
-    int r = rows_override > 0 ? rows_override : std::max(4, (L.ny + want_y - 1) / want_y);
-    r = std::min(r, std::max(L.ny, 1));
-    *rows = r;
+    const int r = std::min(rows, std::max(L.ny, 1));
+    *out_rows = r;
     *nby = (L.ny + r - 1) / r;
     return 0;
+}
+
+// The default tile (rows = 0): ibtfo_set_tile / ibtfo_autotune choose another.
+// A small grid's step is one wave's chain of dependent work, 8 us for one row and
+// 2.7 us for each further row of a marching strip, however few cells there are: the
+// row-parallel form runs a strip's rows at once, and is best with the fewest rows
+// that leave at most one block per CU (256), else at most two (512), the blocks
+// that run together; with more, its 7-row strips up to two rounds of those. Measured,
+// us per step, row-parallel against the best marching strip: 64x64 8.8 / 9.7,
+// 256x128 9.9 / 13.9, 400x100 (one kernel per step) 8.8 / 13.7, 512x256 15.5 / 20.8,
+// 512x512 with two stages 42.8 / 48.1, 800x400 26.1 / 29.3 (ghost fluid: 26.8 / 25.2).
+// Larger grids march: a strip of r rows computes r + 1 y faces and r + 2 rows of y
+// states, so few rows cost work and many cost balance over the 4096 waves that run
+// together: 1024x512: 3 rows 32.3, 6 rows 35.3; 2048x1024: 3 rows 75.3, 6 rows 71.7,
+// 8 rows 77.3; 4096x2048: 6 rows 244, 8 rows 237, 18 rows 244.
+static void default_tile(const ibtfo_config& c, const Layout& L, int* rows, int* par) {
+    const long long nbx = (L.nx + STRIP_W - 1) / STRIP_W, cells = (long long)L.nx * L.ny;
+    auto blocks = [&](int r) { return nbx * ((L.ny + r - 1) / r); };
+    *par = 0;
+    *rows = cells < 900000 ? 3 : (cells < 2200000 ? 6 : 8);
+    if (c.scheme == IBTFO_LAX || blocks(ROWPAR_MAX_ROWS) > 1024) return;
+    *par = 1;
+    *rows = ROWPAR_MAX_ROWS;
+    const int cap = blocks(ROWPAR_MAX_ROWS) <= 256 ? 256 : 512;
+    while (*rows > 1 && blocks(*rows - 1) <= cap) --*rows;
 }
 
 static int validate(const ibtfo_config* c) {
@@ -164,8 +184,9 @@ int ctx_create(const ibtfo_config* cfg, Arena* arena, hipStream_t stream, int ro
     x->cfg = *cfg;
     x->L = make_layout(cfg);
     x->arena = arena;
-    x->rows_override = rows;
     const Layout& L = x->L;
+    if (rows <= 0) default_tile(*cfg, L, &rows, &x->rowpar);
+    x->rows_override = rows;
     if (hipGetDevice(&x->device) != hipSuccess) { delete x; set_error("no HIP device"); return IBTFO_E_HIP; }
     auto fail = [&](const char* what) {
         set_error("allocation of %s failed (%s)", what, arena ? "batch arena full" : hipGetErrorString(hipGetLastError()));
@@ -1167,6 +1188,7 @@ extern "C" int ibtfo_set_tile(ibtfo_ctx* x, int rows, int row_parallel) {
                   ROWPAR_MAX_ROWS, rows);
         return IBTFO_E_ARG;
     }
+    if (rows == 0) default_tile(x->cfg, x->L, &rows, &row_parallel);
     int nbx, nby, r;
     step_grid(x->L, rows, &nbx, &nby, &r);
     if (nbx * nby > x->mass_cap) {

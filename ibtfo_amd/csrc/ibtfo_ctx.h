@@ -29,7 +29,7 @@ struct ibtfo_ctx {
     double* mass_part;  // PART_STRIDE doubles per step-kernel block
     int mass_cap;       // blocks
     double* fold;       // FOLD_MAX records of the two-level finish
-    int rows_override;  // step-kernel rows per strip (0 = default shape)
+    int rows_override;  // step-kernel rows per strip
     int cur_guess;      // the current buffer after the queued steps, as far as the host knows
     int rowpar;         // 1: the row-parallel step kernel (rows + 1 waves per block)
     double* corner;

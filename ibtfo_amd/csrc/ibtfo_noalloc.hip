@@ -62,9 +62,10 @@ extern "C" int ibtfo_compute_dt_noalloc(ibtfo_ctx* x, double* out) {
         return IBTFO_E_ARG;
     }
     const ReduceArgs& base = x->ra;  // the arguments ibtfo_compute_dt launches with
-    if (base.nblocks > NOALLOC_PARTS) {
-        set_error("ibtfo_compute_dt_noalloc: %d x %d interior cells need %d partial records, more than the %d "
-                  "this entry point holds (at most %d interior cells)", x->L.nx, x->L.ny, base.nblocks,
+    const long long records = ((long long)x->L.nx * x->L.ny + 255) / 256;  // one per 256 cells
+    if (records > NOALLOC_PARTS || base.nblocks > NOALLOC_PARTS) {
+        set_error("ibtfo_compute_dt_noalloc: %d x %d interior cells need %lld partial records, more than the %d "
+                  "this entry point holds (at most %d interior cells)", x->L.nx, x->L.ny, records,
                   NOALLOC_PARTS, NOALLOC_PARTS * 256);
         return IBTFO_E_ARG;
     }

@@ -222,8 +222,8 @@ int ibtfo_boundary(ibtfo_ctx* ctx);
 int ibtfo_time_steps(ibtfo_ctx* ctx, int nsteps, double* total_ms, double* step_kernel_ms);
 
 /* Step-kernel tile shape: a block updates a strip of 60 columns x `rows` rows.
- * rows = 0 restores the default shape. May allocate (block partials). Same as
- * ibtfo_set_tile(ctx, rows, 0). */
+ * rows = 0 restores the default shape and form (row-parallel on small grids). May
+ * allocate (block partials). Same as ibtfo_set_tile(ctx, rows, 0). */
 int ibtfo_set_rows(ibtfo_ctx* ctx, int rows);
 /* Tile shape and form: row_parallel = 0 is the marching strip (one wave walks
  * the strip's rows one after the other); row_parallel = 1 gives each of the
