@@ -594,7 +594,7 @@ static int ensure_persistent(ibtfo_batch* b) {
     b->persist_grid = persist_blocks(k.scheme, k.riemann, k.limiter, k.precision);
     if (b->persist_grid <= 0) { set_error("no resident grid for the persistent step kernel"); return IBTFO_E_HIP; }
     if (dev_alloc(&b->d_counts, 3) || dev_alloc(&b->d_bar, 1) || dev_alloc(&b->d_err, 1) ||
-        host_alloc(&b->h_counts, 3) || hipMemset(b->d_err, 0, sizeof(int)) != hipSuccess) {
+        host_alloc(&b->h_counts, 3) || hipMemsetAsync(b->d_err, 0, sizeof(int), b->run) != hipSuccess) {
         set_error("allocation of the persistent kernel's state failed");
         return IBTFO_E_NOMEM;
     }
