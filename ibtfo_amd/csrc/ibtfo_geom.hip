@@ -484,10 +484,9 @@ hipError_t cut_compact(GeomArgs& g, hipStream_t s) {
 // Test/PNGGeo/Level_Set.cpp:31-149 on the device. The reference computes, for
 // every cell, the distance to every edge pixel (O(cells x edges)); here the
 // nearest edge pixel is found by a separable exact search (per pixel column the
-// nearest edge row to each cell row, then per cell row the lower envelope of the
-// parabolas (x_q - x_e)^2 + g(x_e) over pixel columns, Felzenszwalb and
-// Huttenlocher, "Distance Transforms of Sampled Functions", 2012), and the
-// distance to that pixel is evaluated with the reference's expression.
+// nearest edge row to each cell row, then per cell row the least of the parabolas
+// (x_q - x_e)^2 + g(x_e) over pixel columns), and the distance to that pixel is
+// evaluated with the reference's expression.
 
 // Level_Set.cpp:36-48: +1 where R + G + B > 0, else -1; image rows flipped so that
 // row 0 is the bottom of the domain
@@ -496,7 +495,7 @@ __global__ void k_mask_sign(MaskArgs m) {
     if (x >= m.W) return;
     const unsigned char* px = m.rgba + ((long long)y * m.W + x) * 4;
     const double s = (double)px[0] + (double)px[1] + (double)px[2];
-    m.v[(long long)(m.H - y - 1) * m.W + x] = (s > 0) * 2 - 1;
+    m.v[(long long)(m.H - y - 1) * m.W + x] = (signed char)((s > 0) * 2 - 1);
 }
 
 // Level_Set.cpp:51-76: edge pixel where max(|v - v_left|, |v - v_below|) > 0.1,
@@ -506,11 +505,8 @@ __global__ void k_mask_edge(MaskArgs m) {
     if (x >= m.W) return;
     unsigned char e = 0;
     if (x >= 1 && x < m.W - 1 && y >= 1 && y < m.H - 1) {
-        const double c = m.v[(long long)y * m.W + x];
-        const double dx = c - m.v[(long long)y * m.W + x - 1];
-        const double dy = c - m.v[(long long)(y - 1) * m.W + x];
-        const double g = (ib_fabs(dx) > ib_fabs(dy)) ? ib_fabs(dx) : ib_fabs(dy);
-        e = g > 0.1;
+        const signed char c = m.v[(long long)y * m.W + x];  // signs +-1: any difference is 2
+        e = c != m.v[(long long)y * m.W + x - 1] || c != m.v[(long long)(y - 1) * m.W + x];
     }
     m.edge[(long long)y * m.W + x] = e;
 }
@@ -554,7 +550,9 @@ __global__ void k_edt_segscan(MaskArgs m) {
 // Per (pixel column x, cell row j): the column's edge rows just below and just
 // above the cell-centre height y_j (the last with edge height <= y_j and the
 // first above it: within the 32-row segment around y_j, else from the segment
-// summaries), the nearer of them and its squared height difference.
+// summaries), and the smaller of their squared height differences (infinite
+// without an edge). In rounded arithmetic too no other edge of the column is
+// nearer: the squares grow with the distance.
 __global__ void k_edt_cols(MaskArgs m) {
     const long long t = blockIdx.x * (long long)blockDim.x + threadIdx.x;
     if (t >= (long long)m.W * m.N) return;
@@ -580,140 +578,128 @@ __global__ void k_edt_cols(MaskArgs m) {
         if (nxt < 0) nxt = m.after[(long long)s1 * m.W + x];
     }
     double best = HUGE_VAL;
-    int arg = -1;
     if (prv >= 0) {
-        double d = edge_y(m, prv) - yq;
+        const double d = edge_y(m, prv) - yq;
         best = d * d;
-        arg = prv;
     }
     if (nxt >= 0) {
-        double d = edge_y(m, nxt) - yq;
-        if (d * d < best) { best = d * d; arg = nxt; }
+        const double d = edge_y(m, nxt) - yq;
+        if (d * d < best) best = d * d;
     }
     m.g1[t] = best;
-    m.r1[t] = arg;
-    m.r2[t] = arg == prv ? nxt : prv;  // the other neighbour (near ties)
 }
 
-// phi of cell (i, j) from the lower envelope (v[0..k], boundaries z) of cell row
-// j: the envelope's parabola at the cell centre and its neighbours, each with the
-// column's two nearest edge rows; points whose distances tie with the nearest in
-// exact arithmetic but round differently are all evaluated with the reference's
-// expression, whose minimum it keeps. Then the sign sampled at pixel
-// (int((i+0.5) W / M), int((j+0.5) H / N)).
-template <typename V>
-__device__ __forceinline__ double mask_phi_cell(const MaskArgs& m, int i, int j, const V* v, const double* z,
-                                                int k) {
-    const double X = m.Li + i * m.dxc, Y = m.Hi + j * m.dxc;
-    double dmin = 100.0;  // Level_Set.cpp:131 starts every search at 100
-    if (k >= 0) {
-        // q = the last envelope piece whose left boundary lies below X
-        int lo = 0, hi = k;
-        while (lo < hi) {
-            const int mid = (lo + hi + 1) >> 1;
-            if (z[mid] < X) lo = mid;
-            else hi = mid - 1;
-        }
-        const int q = lo;
-        for (int c = (q > 0 ? q - 1 : q); c <= (q < k ? q + 1 : q); c++) {
-            const int ex = v[c];
-            const double ax = edge_x(m, ex);
-            for (int rr = 0; rr < 2; rr++) {
-                const int ey = rr == 0 ? m.r1[(long long)j * m.W + ex] : m.r2[(long long)j * m.W + ex];
-                if (ey < 0) continue;
-                const double ay = edge_y(m, ey);
-                const double d = ib_sqrt((ax - X) * (ax - X) + (ay - Y) * (ay - Y));
-                if (d < dmin) dmin = d;
-            }
-        }
-    }
-    const int xs = (int)((i + 0.5) * (m.W) / (m.M));
-    const int ys = (int)((j + 0.5) * (m.H) / (m.N));
-    const int pn = m.v[(long long)ys * m.W + xs] >= 0 ? 1 : -1;
-    return pn * dmin;
-}
-
-// Per cell row j (one 64-lane block): the lower envelope of f_x(q) = (q - x_e(x))^2
-// + g1(x, j) over the pixel columns that hold an edge (Felzenszwalb-Huttenlocher),
-// built by lane 0 with its stack in LDS, the row's g1 staged in LDS by all lanes;
-// then every lane evaluates cells i = lane, lane + 64, ...
-__global__ __launch_bounds__(64) void k_edt_rows(MaskArgs m) {
+// Per cell row j: phi of its cells, +- the distance to the nearest edge pixel, which
+// is the root of the least (x_e - X)^2 + g1 over the pixel columns that hold an edge
+// (the root is monotone, so it is taken once, of the least radicand; every radicand
+// is rounded as the reference rounds it). The columns whose parabola is least move
+// to the right with X: f_a - f_b of two columns is linear in X. So the row is cut
+// into intervals of `stride` cells; the least column is found between intervals (a
+// wave per point, its lanes over all columns), and each cell of an interval then
+// scans only the columns between its ends' (a lane per cell, all lanes the same
+// column): n + W*nq/64 steps of a wave for the row, whatever the shape. The points
+// lie half a cell from any cell, which makes the bound hold in rounded arithmetic:
+// at a cell, a column outside it is worse by at least a column spacing times a cell
+// size, the domain squared over W*M, against rounding of some 1e-16 of it.
+// A serial lower envelope (one lane per row, a division per column) took 1.49 ms for
+// a 2052x1028 mask; this takes 0.084, bound by the scans' LDS latency (0.147 with 256
+// threads a block and no unrolling: LDS holds four blocks on a CU, and 1028 of them
+// then leave a second round nearly empty; 0.088 with 1024 threads).
+constexpr int EDT_THREADS = 512;
+template <bool LDS> __global__ __launch_bounds__(EDT_THREADS) void k_edt_rows(MaskArgs m, int stride, int nq) {
     extern __shared__ double lds[];
-    const int j = blockIdx.x, lane = threadIdx.x, W = m.W;
-    double* z = lds;                                    // W + 1
-    double* gr = z + (W + 1);                           // W
-    unsigned short* v = (unsigned short*)(gr + W);      // W + 1
-    __shared__ int kk;
-    for (int x = lane; x < W; x += 64) gr[x] = m.g1[(long long)j * W + x];
-    __syncthreads();
-    if (lane == 0) {
-        int k = -1;
-        for (int x = 0; x < W; x++) {
-            const double f = gr[x];
-            if (!(f < HUGE_VAL)) continue;
-            const double p = edge_x(m, x);
-            double s = -HUGE_VAL;
-            while (k >= 0) {
-                const int u = v[k];
-                const double pu = edge_x(m, u), fu = gr[u];
-                s = ((f + p * p) - (fu + pu * pu)) / (2.0 * (p - pu));
-                if (s <= z[k]) k--;
-                else break;
+    __shared__ int wsum[EDT_THREADS / 64];
+    const int j = blockIdx.x, lane = threadIdx.x & 63, wv = threadIdx.x >> 6, W = m.W;
+    const double* grow = m.g1 + (long long)j * W;
+    double* ps = lds;                               // LDS: positions and g1 of the columns with an edge
+    double* gs = ps + W;
+    int* arg = (int*)(LDS ? (void*)(gs + W) : (void*)lds);  // nq + 1 bounds
+    int n = W;
+    if (LDS) {  // compacted in order
+        n = 0;
+        for (int x0 = 0; x0 < W; x0 += EDT_THREADS) {
+            const int x = x0 + threadIdx.x;
+            const double f = x < W ? grow[x] : HUGE_VAL;
+            const bool has = f < HUGE_VAL;
+            const unsigned long long b = __ballot(has);
+            if (lane == 0) wsum[wv] = __popcll(b);
+            __syncthreads();
+            int at = n;
+            for (int u = 0; u < EDT_THREADS / 64; u++) {
+                if (u < wv) at += wsum[u];
+                n += wsum[u];
             }
-            k++;
-            v[k] = (unsigned short)x;
-            z[k] = k == 0 ? -HUGE_VAL : s;
+            at += __popcll(b & ((1ull << lane) - 1));
+            if (has) {
+                ps[at] = edge_x(m, x);
+                gs[at] = f;
+            }
+            __syncthreads();
         }
-        kk = k;
+    }
+    auto radicand = [&](int x, double X) {
+        const double d = (LDS ? ps[x] : edge_x(m, x)) - X;
+        return d * d + (LDS ? gs[x] : grow[x]);
+    };
+    if (threadIdx.x == 0) {
+        arg[0] = 0;
+        arg[nq] = n - 1;
+    }
+    for (int q = 1 + wv; q < nq; q += EDT_THREADS / 64) {
+        const double X = m.Li + ((double)((long long)q * stride) - 0.5) * m.dxc;
+        double best = HUGE_VAL;
+        int at = 0;
+#pragma unroll 8
+        for (int x = lane; x < n; x += 64) {
+            const double v = radicand(x, X);
+            if (v < best) { best = v; at = x; }
+        }
+        for (int o = 32; o > 0; o >>= 1) {
+            const double v = __shfl_xor(best, o, 64);
+            const int a = __shfl_xor(at, o, 64);
+            if (v < best || (v == best && a < at)) { best = v; at = a; }
+        }
+        if (lane == 0) arg[q] = at;
     }
     __syncthreads();
-    const int k = kk;
-    for (int i = lane; i < m.M; i += 64) m.phi[(long long)j * m.M + i] = mask_phi_cell(m, i, j, v, z, k);
-}
-
-// The same for masks too wide for the LDS envelope: one thread per cell row,
-// its stack in global scratch.
-__global__ void k_edt_rows_global(MaskArgs m) {
-    const int j = blockIdx.x * blockDim.x + threadIdx.x;
-    if (j >= m.N) return;
-    int* v = m.vbuf + (long long)j * (m.W + 1);
-    double* z = m.zbuf + (long long)j * (m.W + 1);
-    const double* g = m.g1 + (long long)j * m.W;
-    int k = -1;
-    for (int x = 0; x < m.W; x++) {
-        const double f = g[x];
-        if (!(f < HUGE_VAL)) continue;
-        const double p = edge_x(m, x);
-        double s = -HUGE_VAL;
-        while (k >= 0) {
-            const int u = v[k];
-            const double pu = edge_x(m, u), fu = g[u];
-            s = ((f + p * p) - (fu + pu * pu)) / (2.0 * (p - pu));
-            if (s <= z[k]) k--;
-            else break;
+    const double Y0 = (j + 0.5) * (m.H) / (m.N);
+    const signed char* vrow = m.v + (long long)(int)Y0 * W;
+    for (int q = wv; q < nq; q += EDT_THREADS / 64) {
+        const int lo = arg[q], hi = min(arg[q + 1], n - 1);  // none without an edge
+        const int iend = min((q + 1) * stride, m.M);
+        for (int i = q * stride + lane; i < iend; i += 64) {
+            const double X = m.Li + i * m.dxc;
+            double best = HUGE_VAL;
+#pragma unroll 8
+            for (int x = lo; x <= hi; x++) {
+                const double v = radicand(x, X);
+                best = v < best ? v : best;
+            }
+            const double d = ib_sqrt(best);
+            const double dmin = d < 100.0 ? d : 100.0;  // Level_Set.cpp:131 starts every search at 100
+            // the sign sampled at pixel (int((i+0.5) W / M), int((j+0.5) H / N))
+            const int xs = (int)((i + 0.5) * (W) / (m.M));
+            m.phi[(long long)j * m.M + i] = (vrow[xs] >= 0 ? 1 : -1) * dmin;
         }
-        k++;
-        v[k] = x;
-        z[k] = k == 0 ? -HUGE_VAL : s;
     }
-    for (int i = 0; i < m.M; i++) m.phi[(long long)j * m.M + i] = mask_phi_cell(m, i, j, v, z, k);
 }
 
-hipError_t mask_run(MaskArgs& m, hipStream_t s) {
+hipError_t mask_run(MaskArgs& m, bool lds, hipStream_t s) {
     dim3 pg((m.W + 255) / 256, m.H);
     hipLaunchKernelGGL(k_mask_sign, pg, dim3(256), 0, s, m);
     hipLaunchKernelGGL(k_mask_edge, pg, dim3(256), 0, s, m);
     hipLaunchKernelGGL(k_edt_segs, dim3((m.W + 255) / 256, m.nseg), dim3(256), 0, s, m);
     hipLaunchKernelGGL(k_edt_segscan, dim3((m.W + 255) / 256), dim3(256), 0, s, m);
-    const long long nq = (long long)m.W * m.N;
-    hipLaunchKernelGGL(k_edt_cols, dim3((unsigned)((nq + 255) / 256)), dim3(256), 0, s, m);
-    if (!m.vbuf) {
-        hipLaunchKernelGGL(k_edt_rows, dim3(m.N), dim3(64), mask_lds_bytes(m.W), s, m);
+    const long long nc = (long long)m.W * m.N;
+    hipLaunchKernelGGL(k_edt_cols, dim3((unsigned)((nc + 255) / 256)), dim3(256), 0, s, m);
+    const int stride = edt_stride(m.M), nq = edt_intervals(m.M);
+    if (lds) {
+        hipLaunchKernelGGL(k_edt_rows<true>, dim3(m.N), dim3(EDT_THREADS), mask_lds_bytes(m.W, m.M), s, m, stride, nq);
     } else {
-        hipLaunchKernelGGL(k_edt_rows_global, dim3((m.N + 63) / 64), dim3(64), 0, s, m);
+        hipLaunchKernelGGL(k_edt_rows<false>, dim3(m.N), dim3(EDT_THREADS), (nq + 1) * sizeof(int), s, m, stride, nq);
     }
     return hipGetLastError();
 }
-const void* mask_rows_kernel() { return (const void*)k_edt_rows; }
+const void* mask_rows_kernel() { return (const void*)k_edt_rows<true>; }
 
 }  // namespace ibtfo
