@@ -292,46 +292,45 @@ extern "C" int ibtfo_cut_counts(const ibtfo_ctx* x, int* cut_cells, int* merge_g
 // --------------------------------------------------------------- geometry
 // Runs the geometry kernels for a prepared GeomArgs (hook constants and inputs
 // set) and builds the ghost list; frees `dphi` (a device input of the hook).
-// Cut-cell geometry after geom_run: dense scratch, records, types, merge
-// targets, ghosts; then the compact records, the index plane and the groups.
+// Cut-cell geometry after geom_run: types, merge targets and ghosts, then the compact
+// records, the index plane, the groups and the step kernel's type plane, in which the
+// groups' cells (targets and members) carry MERGED_BIT: the step leaves their dt /
+// mass partials to the merge kernel, which writes one record per block.
 static int cut_geometry(ibtfo_ctx* x, GeomArgs& g) {
     const Layout& L = x->L;
-    dfree(x, x->cuts); x->cuts = nullptr;
-    dfree(x, x->cut_index); x->cut_index = nullptr;
-    dfree(x, x->groups); x->groups = nullptr;
+    for (void** p : {(void**)&x->cuts, (void**)&x->cut_index, (void**)&x->groups, (void**)&x->stype,
+                     (void**)&x->merge_part}) {
+        dfree(x, *p);
+        *p = nullptr;
+    }
     x->ncut = x->ngroups = 0;
-    double* dense = nullptr;
-    if (dalloc(x, &dense, (size_t)L.M * L.N * 8 * sizeof(double)) != hipSuccess ||
-        dalloc(x, &x->cut_index, (size_t)L.plane * sizeof(int)) != hipSuccess) {
-        dfree(x, dense);
+    const size_t marks = (size_t)round_up(L.plane, 8);  // the two counters stand behind them
+    if (dalloc(x, &g.cmark, marks + 2 * sizeof(unsigned)) != hipSuccess ||
+        dalloc(x, &x->cut_index, (size_t)L.plane * sizeof(int)) != hipSuccess ||
+        dalloc(x, &x->stype, L.plane) != hipSuccess) {
+        dfree(x, g.cmark);
         set_error("cut-cell geometry: out of device memory");
         return IBTFO_E_NOMEM;
     }
-    g.dcut = dense;
+    g.ccount = (unsigned*)(g.cmark + marks);
     g.cut_index = x->cut_index;
-    g.ccount = x->dcount;
-    unsigned int zero[2] = {0, 0}, cnt[2] = {0, 0};
-    unsigned int* gcount = nullptr;
-    if (dalloc(x, &gcount, sizeof(unsigned int)) != hipSuccess) { dfree(x, dense); return IBTFO_E_NOMEM; }
-    g.gcount = gcount;
-    auto pass = [&](int fill) -> hipError_t {
-        hipError_t e = hipMemcpyAsync(x->dcount, &zero[0], sizeof(unsigned), hipMemcpyHostToDevice, x->stream);
-        if (e == hipSuccess) e = hipMemcpyAsync(gcount, &zero[1], sizeof(unsigned), hipMemcpyHostToDevice, x->stream);
-        if (e == hipSuccess && !fill) e = cut_run(g, x->stream);
-        if (e == hipSuccess) e = cut_compact(g, x->stream);
-        if (e == hipSuccess) e = hipMemcpyAsync(&cnt[0], x->dcount, sizeof(unsigned), hipMemcpyDeviceToHost, x->stream);
-        if (e == hipSuccess) e = hipMemcpyAsync(&cnt[1], gcount, sizeof(unsigned), hipMemcpyDeviceToHost, x->stream);
-        if (e == hipSuccess) e = hipStreamSynchronize(x->stream);
-        return e;
-    };
-    g.ccap = g.gcap = 0;
-    hipError_t e = pass(0);
+    g.stype = x->stype;
+    g.cuts = nullptr;
+    unsigned int cnt[2] = {0, 0};
+    hipError_t e = hipMemsetAsync(g.ccount, 0, sizeof cnt, x->stream);
+    if (e == hipSuccess) e = cut_run(g, x->stream);
+    if (e == hipSuccess) e = cut_records(g, x->stream);
+    if (e == hipSuccess) e = scopy(x, cnt, g.ccount, sizeof cnt, hipMemcpyDeviceToHost);
     int rc = IBTFO_OK;
-    if (e == hipSuccess) {
+    if (e == hipSuccess) e = hipMemcpyAsync(x->stype, x->type, L.plane, hipMemcpyDeviceToDevice, x->stream);
+    if (e == hipSuccess && cnt[0]) {  // a merge group holds cut cells
         x->ncut = (int)cnt[0];
         x->ngroups = (int)cnt[1];
-        if ((x->ncut && dalloc(x, &x->cuts, x->ncut * sizeof(CutCell)) != hipSuccess) ||
-            (x->ngroups && dalloc(x, &x->groups, x->ngroups * sizeof(MergeGroup)) != hipSuccess)) {
+        if (dalloc(x, &x->cuts, x->ncut * sizeof(CutCell)) != hipSuccess ||
+            (x->ngroups &&
+             (dalloc(x, &x->groups, x->ngroups * sizeof(MergeGroup)) != hipSuccess ||
+              dalloc(x, &x->merge_part, PART_STRIDE * (size_t)merge_blocks(x->ngroups) * sizeof(double)) !=
+                  hipSuccess))) {
             set_error("cut-cell geometry: out of device memory for %d records", x->ncut);
             rc = IBTFO_E_NOMEM;
         } else {
@@ -339,34 +338,14 @@ static int cut_geometry(ibtfo_ctx* x, GeomArgs& g) {
             g.ccap = x->ncut;
             g.groups = x->groups;
             g.gcap = x->ngroups;
-            e = pass(1);
+            e = hipMemsetAsync(g.ccount, 0, sizeof cnt, x->stream);
+            if (e == hipSuccess) e = cut_records(g, x->stream);
         }
     }
-    dfree(x, dense);
-    dfree(x, gcount);
-    g.dcut = nullptr;
+    if (e == hipSuccess) e = hipStreamSynchronize(x->stream);
+    dfree(x, g.cmark);
     if (rc) return rc;
     HIPCHK(e);
-    // the merge groups' cells (targets and members) carry MERGED_BIT in the step
-    // kernel's type plane: it leaves their dt / mass partials to the merge kernel,
-    // which writes one record per block
-    dfree(x, x->stype); x->stype = nullptr;
-    dfree(x, x->merge_part); x->merge_part = nullptr;
-    std::vector<uint8_t> mk(L.plane);
-    std::vector<MergeGroup> gr(x->ngroups);
-    HIPCHK(scopy(x, mk.data(), x->type, L.plane, hipMemcpyDeviceToHost));
-    if (x->ngroups) HIPCHK(scopy(x, gr.data(), x->groups, x->ngroups * sizeof(MergeGroup), hipMemcpyDeviceToHost));
-    for (const MergeGroup& m : gr) {
-        mk[m.target] |= MERGED_BIT;
-        for (int q = 0; q < m.n; q++) mk[m.member[q]] |= MERGED_BIT;
-    }
-    if (dalloc(x, &x->stype, L.plane) != hipSuccess ||
-        (x->ngroups && dalloc(x, &x->merge_part, PART_STRIDE * (size_t)merge_blocks(x->ngroups) * sizeof(double)) !=
-                           hipSuccess)) {
-        set_error("cut-cell geometry: out of device memory");
-        return IBTFO_E_NOMEM;
-    }
-    HIPCHK(scopy(x, x->stype, mk.data(), L.plane, hipMemcpyHostToDevice));
     return IBTFO_OK;
 }
 

@@ -22,14 +22,14 @@ struct GeomArgs {
     // cut cells (bc = IDW fill with active donors = types 0 and 3)
     int cut;
     double cdx, cdy;        // cell sizes (Psy_L / N_x, Psy_H / N_y)
-    double* dcut;           // dense scratch: M x N records of 8 doubles
-    CutCell* cuts;          // compact records of the type-3 cells
+    uint8_t* cmark;         // plane: merge direction and zero apertures (k_cut_cells, k_cut_target)
+    CutCell* cuts;          // compact records of the type-3 cells (null: counting)
     int* cut_index;         // plane: record of each type-3 cell
-    unsigned int* ccount;
+    unsigned int* ccount;   // {cut cells, merge groups}
     int ccap;
     MergeGroup* groups;
-    unsigned int* gcount;
     int gcap;
+    uint8_t* stype;         // plane: the step kernel's types, a copy of type before the filling pass
     Ghost* ghosts;
     unsigned int* count;
     int cap;
@@ -63,11 +63,10 @@ hipError_t geom_run(GeomArgs& g, hipStream_t s);
 // attribute is set by the caller), else it reads them from memory
 hipError_t mask_run(MaskArgs& m, bool lds, hipStream_t s);
 const void* mask_rows_kernel();  // the LDS form
-// cut-cell geometry on top of geom_run's phi and normals: records, types, merge
-// targets, ghosts (dense scratch g.dcut), then the compaction passes (counting
-// when ccap / gcap are 0)
+// cut-cell geometry on top of geom_run's phi and normals: types, merge targets and
+// ghosts, then the records (counting while g.cuts is null, then filling)
 hipError_t cut_run(GeomArgs& g, hipStream_t s);
-hipError_t cut_compact(GeomArgs& g, hipStream_t s);
+hipError_t cut_records(GeomArgs& g, hipStream_t s);
 hipError_t geom_ghosts(GeomArgs& g, hipStream_t s);
 
 }  // namespace ibtfo

@@ -128,16 +128,60 @@ __device__ int donor_idx(double v, double base, double h, int n) {
     return r;
 }
 
+// Lists of the interior cells that need a record (ghosts, cut cells, merge groups):
+// a block lists its tile's cells in LDS, takes their slots with one atomic and
+// shares the records among its threads. An atomic per wave on the one counter was
+// what bounded these passes: on the 2048x1024 bodies grid 51 us a pass over the
+// ghosts, 82 over the cut cells; now 8 and 29.
+constexpr int TILE_X = 64, TILE_Y = 32, TILE_THREADS = 256;
+struct TileList {
+    int n;
+    unsigned int base;
+    unsigned short cell[TILE_X * TILE_Y];
+};
+__device__ __forceinline__ void tile_cell(const Layout& L, int k, int& i, int& j) {
+    i = L.ng + blockIdx.x * TILE_X + k % TILE_X;
+    j = L.ng + blockIdx.y * TILE_Y + k / TILE_X;
+}
+template <class F> __device__ __forceinline__ void tile_each(const Layout& L, F f) {
+    for (int k = threadIdx.x; k < TILE_X * TILE_Y; k += TILE_THREADS) {
+        int i, j;
+        tile_cell(L, k, i, j);
+        if (i < L.nx + L.ng && j < L.ny + L.ng) f(k, i, j);
+    }
+}
+__device__ __forceinline__ void tile_push(TileList& l, int k) { l.cell[atomicAdd(&l.n, 1)] = (unsigned short)k; }
+__device__ __forceinline__ void tile_claim(TileList& l, unsigned int* count) {  // one thread
+    if (l.n) l.base = atomicAdd(count, (unsigned)l.n);
+}
+static dim3 tile_grid(const Layout& L) { return dim3((L.nx + TILE_X - 1) / TILE_X, (L.ny + TILE_Y - 1) / TILE_Y); }
+
+__device__ void ghost_record(const GeomArgs& g, int i, int j, unsigned int slot);
+__global__ __launch_bounds__(TILE_THREADS) void k_geom_ghosts(GeomArgs g) {
+    __shared__ TileList l;
+    if (threadIdx.x == 0) l.n = 0;
+    __syncthreads();
+    tile_each(g.L, [&](int k, int i, int j) {
+        if (g.type[g.L.at(i, j)] == 2) tile_push(l, k);
+    });
+    __syncthreads();
+    if (threadIdx.x == 0) tile_claim(l, g.count);
+    if (g.cap == 0) return;  // counting only
+    __syncthreads();
+    for (int q = threadIdx.x; q < l.n; q += TILE_THREADS) {
+        int i, j;
+        tile_cell(g.L, l.cell[q], i, j);
+        if (l.base + q < (unsigned)g.cap) ghost_record(g, i, j, l.base + q);
+    }
+}
+
 // Scheme_Index for one ghost: IDWBaseGFM/GFM_Method.cpp:20-110,
 // LinearBaseGFM/GFM_Method.cpp:19-44 + GFM_Bound.cpp:93-575 (donor choice),
 // BCGFM/BCGFM_Method.cpp:49-205, HBCGFM/HBCGFM_Method.cpp:56-91.
-__global__ void k_geom_ghosts(GeomArgs g) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x, j = blockIdx.y;
+__device__ void ghost_record(const GeomArgs& g, int i, int j, unsigned int slot) {
     const Layout L = g.L;
     const int ng = L.ng;
-    if (i < ng || i >= L.nx + ng || j < ng || j >= L.ny + ng) return;
     const long long o = L.at(i, j);
-    if (g.type[o] != 2) return;
     Ghost gh;
     gh.cell = o;
     gh.nx = g.nx[o];
@@ -172,8 +216,7 @@ __global__ void k_geom_ghosts(GeomArgs g) {
         gh.ring = (ring_cell(i + IDX, j) ? 1 : 0) | (ring_cell(i, j + IDY) ? 16 : 0);
         gh.xm = gh.ym = gh.xe = gh.ye = 0.0;
         for (int q = 0; q < 4; q++) { gh.a[q] = 0.0; gh.ae[q] = 0.0; }
-        unsigned int slot = atomicAdd(g.count, 1u);
-        if (slot < (unsigned int)g.cap) g.ghosts[slot] = gh;
+        g.ghosts[slot] = gh;
         return;
     }
     if (bc == 1 || bc == 2 || bc == 3) {
@@ -257,8 +300,7 @@ __global__ void k_geom_ghosts(GeomArgs g) {
         gh.pick = pick;
         gh.a[0] = pick;
     }
-    unsigned int slot = atomicAdd(g.count, 1u);
-    if (slot < (unsigned int)g.cap) g.ghosts[slot] = gh;
+    g.ghosts[slot] = gh;
 }
 
 hipError_t geom_run(GeomArgs& g, hipStream_t s) {
@@ -268,8 +310,7 @@ hipError_t geom_run(GeomArgs& g, hipStream_t s) {
     return hipGetLastError();
 }
 hipError_t geom_ghosts(GeomArgs& g, hipStream_t s) {
-    dim3 blk(128), grd((g.L.M + 127) / 128, g.L.N);
-    hipLaunchKernelGGL(k_geom_ghosts, grd, blk, 0, s, g);
+    hipLaunchKernelGGL(k_geom_ghosts, tile_grid(g.L), dim3(TILE_THREADS), 0, s, g);
     return hipGetLastError();
 }
 
@@ -290,23 +331,18 @@ __device__ __forceinline__ double corner_phi(const GeomArgs& g, int i, int j) { 
     const Layout& L = g.L;
     return 0.25 * (((g.phi[L.at(i, j)] + g.phi[L.at(i + 1, j)]) + g.phi[L.at(i, j + 1)]) + g.phi[L.at(i + 1, j + 1)]);
 }
-__device__ __forceinline__ long long cell_q(const Layout& L, int i, int j) { return (long long)j * L.M + i; }
-
-__global__ void k_cut_cells(GeomArgs g) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x, j = blockIdx.y;
-    const Layout L = g.L;
-    if (i >= L.M) return;
-    double* cc = g.dcut + cell_q(L, i, j) * 8;
-    for (int k = 0; k < 7; k++) cc[k] = 0.0;
-    cc[7] = -1.0;
-    const int ng = L.ng;
-    if (i < ng || i >= L.nx + ng || j < ng || j >= L.ny + ng) { g.type[L.at(i, j)] = 2; return; }
+// Volume fraction and face apertures of an interior cell: a function of phi alone,
+// so the passes below evaluate it again where they need it (cut cells are few).
+// Records of all cells kept between the passes were 135 MB on a 2048x1024 grid,
+// written once and read four times: a set-up took 1.97 ms with them, 1.30 without.
+struct CutShape { double alpha, a[4]; };  // apertures W, E, S, N
+__device__ __forceinline__ CutShape cut_shape(const GeomArgs& g, int i, int j) {
     const double sw = corner_phi(g, i - 1, j - 1), se = corner_phi(g, i, j - 1), ne = corner_phi(g, i, j),
                  nw = corner_phi(g, i - 1, j);
-    const double aw = cut_frac(sw, nw), ae = cut_frac(se, ne), as = cut_frac(sw, se), an = cut_frac(nw, ne);
-    double alpha;
-    if (sw >= 0 && se >= 0 && ne >= 0 && nw >= 0) alpha = 1.0;
-    else if (sw < 0 && se < 0 && ne < 0 && nw < 0) alpha = 0.0;
+    CutShape c;
+    c.a[0] = cut_frac(sw, nw); c.a[1] = cut_frac(se, ne); c.a[2] = cut_frac(sw, se); c.a[3] = cut_frac(nw, ne);
+    if (sw >= 0 && se >= 0 && ne >= 0 && nw >= 0) c.alpha = 1.0;
+    else if (sw < 0 && se < 0 && ne < 0 && nw < 0) c.alpha = 0.0;
     else {
         const double cx[4] = {0, 1, 1, 0}, cy[4] = {0, 0, 1, 1}, cv[4] = {sw, se, ne, nw};
         double px[8], py[8];
@@ -326,12 +362,26 @@ __global__ void k_cut_cells(GeomArgs g) {
             const int l = (k + 1) % n;
             a2 += px[k] * py[l] - px[l] * py[k];
         }
-        alpha = 0.5 * a2;
+        c.alpha = 0.5 * a2;
     }
-    cc[0] = alpha; cc[1] = aw; cc[2] = ae; cc[3] = as; cc[4] = an;
-    cc[5] = -((ae - aw) * g.cdy);
-    cc[6] = -((an - as) * g.cdx);
-    g.type[L.at(i, j)] = alpha >= 1.0 ? 0 : (alpha > 0.0 ? 3 : 1);
+    return c;
+}
+
+// A cell's mark: which neighbour it merges into (0 none, 1-4 W, E, S, N), and
+// whether one of its apertures is zero
+constexpr uint8_t CUT_INTO = 7, CUT_ZERO_FACE = 8;
+
+__global__ void k_cut_cells(GeomArgs g) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x, j = blockIdx.y;
+    const Layout L = g.L;
+    if (i >= L.M) return;
+    const long long o = L.at(i, j);
+    g.cmark[o] = 0;
+    const int ng = L.ng;
+    if (i < ng || i >= L.nx + ng || j < ng || j >= L.ny + ng) { g.type[o] = 2; return; }
+    const CutShape c = cut_shape(g, i, j);
+    if (c.a[0] == 0.0 || c.a[1] == 0.0 || c.a[2] == 0.0 || c.a[3] == 0.0) g.cmark[o] = CUT_ZERO_FACE;
+    g.type[o] = c.alpha >= 1.0 ? 0 : (c.alpha > 0.0 ? 3 : 1);
 }
 
 // A cut cell with alpha < 1/2 picks a neighbour with alpha >= 1/2: along the
@@ -343,8 +393,7 @@ __global__ void k_cut_target(GeomArgs g) {
     const int ng = L.ng;
     if (i < ng || i >= L.nx + ng || j < ng || j >= L.ny + ng) return;
     const long long o = L.at(i, j);
-    double* cc = g.dcut + cell_q(L, i, j) * 8;
-    if (g.type[o] != 3 || cc[0] >= 0.5) return;
+    if (g.type[o] != 3 || cut_shape(g, i, j).alpha >= 0.5) return;
     const double n_x = g.nx[o], n_y = g.ny[o];
     const int sx = n_x >= 0 ? 1 : -1, sy = n_y >= 0 ? 1 : -1;
     int ci[4], cj[4];
@@ -355,9 +404,10 @@ __global__ void k_cut_target(GeomArgs g) {
     }
     for (int q = 0; q < 4; q++) {
         if (ci[q] < ng || ci[q] >= L.nx + ng || cj[q] < ng || cj[q] >= L.ny + ng) continue;
+        // a neighbour that another thread makes inactive has alpha < 1/2 either way
         const uint8_t tq = g.type[L.at(ci[q], cj[q])];
-        if ((tq == 0 || tq == 3) && g.dcut[cell_q(L, ci[q], cj[q]) * 8] >= 0.5) {
-            cc[7] = (double)cell_q(L, ci[q], cj[q]);
+        if (tq == 0 || (tq == 3 && cut_shape(g, ci[q], cj[q]).alpha >= 0.5)) {
+            g.cmark[o] |= ci[q] < i ? 1 : ci[q] > i ? 2 : cj[q] < j ? 3 : 4;
             return;
         }
     }
@@ -382,86 +432,115 @@ __global__ void k_cut_ghosts(GeomArgs g) {
     }
 }
 
-// A face between an active cell and an inactive interior one (zero-area
-// polygons where corners are exactly 0, small cells without a partner) is a wall:
-// its aperture becomes 0 and the wall vector is closed again, so no flux leaves
-// the fluid through it. Each cell writes only its own record; types are read.
-__global__ void k_cut_close(GeomArgs g) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x, j = blockIdx.y;
-    const Layout L = g.L;
-    const int ng = L.ng;
-    if (i < ng || i >= L.nx + ng || j < ng || j >= L.ny + ng) return;
-    const uint8_t t = g.type[L.at(i, j)];
-    if (t != 0 && t != 3) return;
-    double* cc = g.dcut + cell_q(L, i, j) * 8;
-    const int ni[4] = {i - 1, i + 1, i, i}, nj[4] = {j, j, j - 1, j + 1};
-    bool closed = false;
-    for (int q = 0; q < 4; q++) {
-        if (ni[q] < ng || ni[q] >= L.nx + ng || nj[q] < ng || nj[q] >= L.ny + ng) continue;
-        const uint8_t tq = g.type[L.at(ni[q], nj[q])];
-        if (tq == 0 || tq == 3 || cc[1 + q] == 0.0) continue;
-        cc[1 + q] = 0.0;
-        closed = true;
-    }
-    if (!closed) return;
-    cc[5] = -((cc[2] - cc[1]) * g.cdy);
-    cc[6] = -((cc[4] - cc[3]) * g.cdx);
+// Records of the cut cells and merge groups gathered by each target from its W, E,
+// S, N neighbours; run twice, counting them first. A face between an active cell
+// and an inactive interior one (zero-area polygons where corners are exactly 0,
+// small cells without a partner) is a wall: its aperture becomes 0 and the wall
+// vector closes the faces again, so no flux leaves the fluid through it. A full
+// cell with a zero aperture takes the cut-cell update: type 3 with alpha = 1 (set by
+// the counting pass; its neighbours take types 0 and 3 alike). The filling pass also
+// marks the groups' cells in the step kernel's type plane.
+struct CutFaces {
+    bool cut;      // the cell takes the cut-cell update
+    int members;   // neighbours that merge into it: bits W, E, S, N
+    int walls;     // inactive interior neighbours: bits W, E, S, N
+};
+__device__ __forceinline__ void cut_neighbour(int q, int& i, int& j) {
+    i += q == 0 ? -1 : q == 1 ? 1 : 0;
+    j += q == 2 ? -1 : q == 3 ? 1 : 0;
 }
-
-// a full cell (type 0, all apertures 1) with a face closed above takes the
-// cut-cell update: type 3 with alpha = 1
-__global__ void k_cut_retype(GeomArgs g) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x, j = blockIdx.y;
-    const Layout L = g.L;
+__device__ __forceinline__ CutFaces cut_faces(const GeomArgs& g, int i, int j) {
+    const Layout& L = g.L;
     const int ng = L.ng;
-    if (i < ng || i >= L.nx + ng || j < ng || j >= L.ny + ng) return;
-    const long long o = L.at(i, j);
-    const double* cc = g.dcut + cell_q(L, i, j) * 8;
-    if (g.type[o] == 0 && (cc[1] == 0.0 || cc[2] == 0.0 || cc[3] == 0.0 || cc[4] == 0.0)) g.type[o] = 3;
-}
-
-// compaction: records of the type-3 cells, and merge groups gathered by each
-// target from its W, E, S, N neighbours (counting only when the capacity is 0)
-__global__ void k_cut_compact(GeomArgs g) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x, j = blockIdx.y;
-    const Layout L = g.L;
-    const int ng = L.ng;
-    if (i < ng || i >= L.nx + ng || j < ng || j >= L.ny + ng) return;
+    CutFaces c = {false, 0, 0};
     const long long o = L.at(i, j);
     const uint8_t t = g.type[o];
-    const double* cc = g.dcut + cell_q(L, i, j) * 8;
-    if (t == 3) {
-        const unsigned int slot = atomicAdd(g.ccount, 1u);
-        if (slot < (unsigned int)g.ccap) {
-            CutCell r;
-            r.alpha = cc[0]; r.aw = cc[1]; r.ae = cc[2]; r.as = cc[3]; r.an = cc[4]; r.sbx = cc[5]; r.sby = cc[6];
-            r.target = cc[7] < 0 ? -1 : L.at((int)((long long)cc[7] % L.M), (int)((long long)cc[7] / L.M));
-            g.cuts[slot] = r;
-            g.cut_index[o] = (int)slot;
-        }
+    if (t != 0 && t != 3) return c;
+    for (int q = 0; q < 4; q++) {
+        int ni = i, nj = j;
+        cut_neighbour(q, ni, nj);
+        if (ni < ng || ni >= L.nx + ng || nj < ng || nj >= L.ny + ng) continue;
+        const long long nq = L.at(ni, nj);
+        const uint8_t tq = g.type[nq];
+        const int into = g.cmark[nq] & CUT_INTO;
+        if (tq != 0 && tq != 3) c.walls |= 1 << q;
+        else if (into == (q ^ 1) + 1) c.members |= 1 << q;  // the opposite direction's mark
     }
-    if ((t == 0 || t == 3) && cc[0] >= 0.5) {
-        const int ni[4] = {i - 1, i + 1, i, i}, nj[4] = {j, j, j - 1, j + 1};
-        MergeGroup gr;
-        gr.n = 0;
+    c.cut = t == 3 || c.walls || (g.cmark[o] & CUT_ZERO_FACE);
+    return c;
+}
+
+__global__ __launch_bounds__(TILE_THREADS) void k_cut_records(GeomArgs g) {
+    __shared__ TileList cuts, groups;
+    const Layout& L = g.L;
+    const bool fill = g.cuts != nullptr;
+    if (threadIdx.x == 0) cuts.n = groups.n = 0;
+    __syncthreads();
+    tile_each(L, [&](int k, int i, int j) {
+        const CutFaces c = cut_faces(g, i, j);
+        if (c.cut) tile_push(cuts, k);
+        if (c.members) tile_push(groups, k);
+    });
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        tile_claim(cuts, &g.ccount[0]);
+        tile_claim(groups, &g.ccount[1]);
+    }
+    __syncthreads();
+    for (int q = threadIdx.x; q < cuts.n; q += TILE_THREADS) {
+        int i, j;
+        tile_cell(L, cuts.cell[q], i, j);
+        const long long o = L.at(i, j);
+        if (!fill) {
+            g.type[o] = 3;
+            continue;
+        }
+        const unsigned int slot = cuts.base + q;
+        if (slot >= (unsigned int)g.ccap) continue;
+        CutShape c = cut_shape(g, i, j);
+        const int walls = cut_faces(g, i, j).walls, into = g.cmark[o] & CUT_INTO;
+        for (int f = 0; f < 4; f++)
+            if (walls >> f & 1) c.a[f] = 0.0;
+        CutCell r;
+        r.alpha = c.alpha; r.aw = c.a[0]; r.ae = c.a[1]; r.as = c.a[2]; r.an = c.a[3];
+        r.sbx = -((r.ae - r.aw) * g.cdy);
+        r.sby = -((r.an - r.as) * g.cdx);
+        r.target = -1;
+        if (into) {
+            cut_neighbour(into - 1, i, j);
+            r.target = L.at(i, j);
+            g.stype[o] = 3 | MERGED_BIT;
+        }
+        g.cuts[slot] = r;
+        g.cut_index[o] = (int)slot;
+    }
+    if (!fill) return;
+    for (int q = threadIdx.x; q < groups.n; q += TILE_THREADS) {
+        int i, j;
+        tile_cell(L, groups.cell[q], i, j);
+        const unsigned int slot = groups.base + q;
+        if (slot >= (unsigned int)g.gcap) continue;
+        const long long o = L.at(i, j);
+        const int members = cut_faces(g, i, j).members;
+        MergeGroup& gr = g.groups[slot];
+        int n = 0;
         gr.pad = 0;
         gr.target = o;
-        gr.at = cc[0];
-        const double me = (double)cell_q(L, i, j);
-        for (int q = 0; q < 4; q++) {
-            const long long nq = L.at(ni[q], nj[q]);
-            const double* cn = g.dcut + cell_q(L, ni[q], nj[q]) * 8;
-            if (g.type[nq] == 3 && cn[7] == me) {
-                gr.member[gr.n] = nq;
-                gr.am[gr.n] = cn[0];
-                gr.n++;
-            }
+        gr.at = cut_shape(g, i, j).alpha;
+        for (int f = 0; f < 4; f++) {
+            if (!(members >> f & 1)) continue;
+            int ni = i, nj = j;
+            cut_neighbour(f, ni, nj);
+            gr.member[n] = L.at(ni, nj);
+            gr.am[n] = cut_shape(g, ni, nj).alpha;
+            n++;
         }
-        for (int q = gr.n; q < 4; q++) { gr.member[q] = o; gr.am[q] = 0.0; }
-        if (gr.n > 0) {
-            const unsigned int slot = atomicAdd(g.gcount, 1u);
-            if (slot < (unsigned int)g.gcap) g.groups[slot] = gr;
+        gr.n = n;
+        for (; n < 4; n++) {
+            gr.member[n] = o;
+            gr.am[n] = 0.0;
         }
+        g.stype[o] = g.type[o] | MERGED_BIT;
     }
 }
 
@@ -470,13 +549,10 @@ hipError_t cut_run(GeomArgs& g, hipStream_t s) {
     hipLaunchKernelGGL(k_cut_cells, grd, blk, 0, s, g);
     hipLaunchKernelGGL(k_cut_target, grd, blk, 0, s, g);
     hipLaunchKernelGGL(k_cut_ghosts, grd, blk, 0, s, g);
-    hipLaunchKernelGGL(k_cut_close, grd, blk, 0, s, g);
-    hipLaunchKernelGGL(k_cut_retype, grd, blk, 0, s, g);
     return hipGetLastError();
 }
-hipError_t cut_compact(GeomArgs& g, hipStream_t s) {
-    dim3 blk(128), grd((g.L.M + 127) / 128, g.L.N);
-    hipLaunchKernelGGL(k_cut_compact, grd, blk, 0, s, g);
+hipError_t cut_records(GeomArgs& g, hipStream_t s) {
+    hipLaunchKernelGGL(k_cut_records, tile_grid(g.L), dim3(TILE_THREADS), 0, s, g);
     return hipGetLastError();
 }
 
