@@ -534,7 +534,7 @@ extern "C" int ibtfo_geometry_mask(ibtfo_ctx* x, const unsigned char* rgba, int 
     m.eyo = -c.num_ghost_cell * (Psy_H / c.N_y);
     m.dxp = (Psy_L / c.N_x) * (c.N_x + 2 * c.num_ghost_cell) / width;
     m.dyp = (Psy_H / c.N_y) * (c.N_y + 2 * c.num_ghost_cell) / height;
-    const size_t WH = (size_t)width * height, WN = (size_t)width * L.N;
+    const size_t WH = (size_t)width * height;
     m.nseg = (height + MASK_SEG - 1) / MASK_SEG;
     const size_t SW = (size_t)m.nseg * width;
     // the row search stages its columns in LDS up to its limit
@@ -542,18 +542,13 @@ extern "C" int ibtfo_geometry_mask(ibtfo_ctx* x, const unsigned char* rgba, int 
     const bool lds_rows = lds_bytes <= MASK_LDS_MAX &&
                           hipFuncSetAttribute(mask_rows_kernel(), hipFuncAttributeMaxDynamicSharedMemorySize,
                                               (int)lds_bytes) == hipSuccess;
-    unsigned char *drgba = nullptr, *dedge = nullptr;
-    signed char* dv = nullptr;
-    double *dg1 = nullptr, *dphi = nullptr;
-    int *dsf = nullptr, *dsl = nullptr, *dbe = nullptr, *daf = nullptr;
+    unsigned *drgba = nullptr, *dbits = nullptr;
+    double* dphi = nullptr;
+    int *dbe = nullptr, *daf = nullptr;
     auto release = [&]() {
-        for (void* p : {(void*)drgba, (void*)dedge, (void*)dv, (void*)dg1, (void*)dsf, (void*)dsl, (void*)dbe,
-                        (void*)daf})
-            dfree(x, p);
+        for (void* p : {(void*)drgba, (void*)dbits, (void*)dbe, (void*)daf}) dfree(x, p);
     };
-    if (dalloc(x, &drgba, WH * 4) != hipSuccess || dalloc(x, &dedge, WH) != hipSuccess ||
-        dalloc(x, &dv, WH) != hipSuccess || dalloc(x, &dg1, WN * sizeof(double)) != hipSuccess ||
-        dalloc(x, &dsf, SW * sizeof(int)) != hipSuccess || dalloc(x, &dsl, SW * sizeof(int)) != hipSuccess ||
+    if (dalloc(x, &drgba, WH * 4) != hipSuccess || dalloc(x, &dbits, SW * sizeof(int)) != hipSuccess ||
         dalloc(x, &dbe, SW * sizeof(int)) != hipSuccess || dalloc(x, &daf, SW * sizeof(int)) != hipSuccess ||
         dalloc(x, &dphi, (size_t)L.M * L.N * sizeof(double)) != hipSuccess) {
         release();
@@ -561,8 +556,7 @@ extern "C" int ibtfo_geometry_mask(ibtfo_ctx* x, const unsigned char* rgba, int 
         set_error("ibtfo_geometry_mask: out of device memory");
         return IBTFO_E_NOMEM;
     }
-    m.rgba = drgba; m.v = dv; m.edge = dedge; m.g1 = dg1;
-    m.sfirst = dsf; m.slast = dsl; m.before = dbe; m.after = daf;
+    m.rgba = drgba; m.bits = dbits; m.before = dbe; m.after = daf;
     m.phi = dphi;
     hipError_t e = scopy(x, drgba, rgba, WH * 4, hipMemcpyHostToDevice);
     if (e == hipSuccess) e = mask_run(m, lds_rows, x->stream);

@@ -37,16 +37,13 @@ struct GeomArgs {
 
 // Mask level set (Test/PNGGeo/Level_Set.cpp:31-149): phi per cell from an RGBA image
 struct MaskArgs {
-    const unsigned char* rgba;  // W x H x 4, top row first
+    const unsigned* rgba;       // W x H pixels of four bytes, top row first
     int W, H;
-    signed char* v;             // W x H signs, bottom row first
-    unsigned char* edge;        // W x H edge flags, bottom row first
     int M, N;                   // cells with ghosts
     double Li, Hi, dxc;         // cell centres (Psy_coord)
     double exo, eyo, dxp, dyp;  // edge pixel x: exo + dxp * x, y: eyo + dyp * y
-    double* g1;                 // N x W (cell row major): squared y distance to the column's nearest edge
     int nseg;                   // 32-row segments per pixel column
-    int *sfirst, *slast;        // nseg x W: first / last edge row of each segment (-1: none)
+    unsigned* bits;             // nseg x W: edge pixels of each segment
     int *before, *after;        // nseg x W: last edge row below / first above each segment (-1: none)
     double* phi;                // M x N, reference cell order
 };

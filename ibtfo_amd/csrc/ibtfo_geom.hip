@@ -564,109 +564,86 @@ hipError_t cut_records(GeomArgs& g, hipStream_t s) {
 // (x_q - x_e)^2 + g(x_e) over pixel columns), and the distance to that pixel is
 // evaluated with the reference's expression.
 
-// Level_Set.cpp:36-48: +1 where R + G + B > 0, else -1; image rows flipped so that
-// row 0 is the bottom of the domain
-__global__ void k_mask_sign(MaskArgs m) {
-    const int x = blockIdx.x * blockDim.x + threadIdx.x, y = blockIdx.y;
-    if (x >= m.W) return;
-    const unsigned char* px = m.rgba + ((long long)y * m.W + x) * 4;
-    const double s = (double)px[0] + (double)px[1] + (double)px[2];
-    m.v[(long long)(m.H - y - 1) * m.W + x] = (signed char)((s > 0) * 2 - 1);
+// Level_Set.cpp:36-48: a pixel's sign, +1 where R + G + B > 0 (here as a bool), else
+// -1; image rows flipped so that row 0 is the bottom of the domain
+__device__ __forceinline__ bool mask_sign(const MaskArgs& m, int x, int y) {
+    return (m.rgba[(long long)(m.H - y - 1) * m.W + x] & 0xffffffu) != 0;  // the fourth byte is alpha
 }
-
-// Level_Set.cpp:51-76: edge pixel where max(|v - v_left|, |v - v_below|) > 0.1,
-// pixels 1..W-2 x 1..H-2 only
-__global__ void k_mask_edge(MaskArgs m) {
-    const int x = blockIdx.x * blockDim.x + threadIdx.x, y = blockIdx.y;
-    if (x >= m.W) return;
-    unsigned char e = 0;
-    if (x >= 1 && x < m.W - 1 && y >= 1 && y < m.H - 1) {
-        const signed char c = m.v[(long long)y * m.W + x];  // signs +-1: any difference is 2
-        e = c != m.v[(long long)y * m.W + x - 1] || c != m.v[(long long)(y - 1) * m.W + x];
-    }
-    m.edge[(long long)y * m.W + x] = e;
-}
-
 __device__ __forceinline__ double edge_x(const MaskArgs& m, int x) { return m.exo + m.dxp * x; }
 __device__ __forceinline__ double edge_y(const MaskArgs& m, int y) { return m.eyo + m.dyp * y; }
 
-// Per pixel column: the first and last edge row of each 32-row segment.
-__global__ void k_edt_segs(MaskArgs m) {
+// Level_Set.cpp:51-76: edge pixel where max(|v - v_left|, |v - v_below|) > 0.1 (signs
+// that differ), pixels 1..W-2 x 1..H-2 only: one bit each, a word per 32 rows of a
+// column. With the next pass and the row search's share 39 us for a 2052x1028 mask;
+// planes of signs, edge bytes and column distances took 95.
+__global__ void k_mask_edges(MaskArgs m) {
     const int x = blockIdx.x * blockDim.x + threadIdx.x, sg = blockIdx.y;
     if (x >= m.W) return;
-    int first = -1, last = -1;
-    const int y1 = min((sg + 1) * MASK_SEG, m.H);
-    for (int y = sg * MASK_SEG; y < y1; y++)
-        if (m.edge[(long long)y * m.W + x]) {
-            if (first < 0) first = y;
-            last = y;
+    unsigned w = 0;
+    if (x >= 1 && x < m.W - 1) {
+        const int y0 = max(sg * MASK_SEG, 1), y1 = min((sg + 1) * MASK_SEG, m.H - 1);
+        bool below = y0 < y1 && mask_sign(m, x, y0 - 1);
+#pragma unroll 8
+        for (int y = y0; y < y1; y++) {
+            const bool c = mask_sign(m, x, y);
+            if (c != below || c != mask_sign(m, x - 1, y)) w |= 1u << (y % MASK_SEG);
+            below = c;
         }
-    m.sfirst[(long long)sg * m.W + x] = first;
-    m.slast[(long long)sg * m.W + x] = last;
+    }
+    m.bits[(long long)sg * m.W + x] = w;
 }
 
-// Per pixel column: the last edge row below each segment and the first above it.
-__global__ void k_edt_segscan(MaskArgs m) {
-    const int x = blockIdx.x * blockDim.x + threadIdx.x;
+// Per word: the column's last edge row below its rows and the first above them.
+__global__ void k_mask_beyond(MaskArgs m) {
+    const int x = blockIdx.x * blockDim.x + threadIdx.x, sg = blockIdx.y;
     if (x >= m.W) return;
-    int b = -1;
-    for (int sg = 0; sg < m.nseg; sg++) {
-        const long long o = (long long)sg * m.W + x;
-        m.before[o] = b;
-        if (m.slast[o] >= 0) b = m.slast[o];
+    int b = -1, a = -1;
+    for (int s = sg - 1; s >= 0 && b < 0; s--) {
+        const unsigned w = m.bits[(long long)s * m.W + x];
+        if (w) b = s * MASK_SEG + 31 - __clz((int)w);
     }
-    int a = -1;
-    for (int sg = m.nseg - 1; sg >= 0; sg--) {
-        const long long o = (long long)sg * m.W + x;
-        m.after[o] = a;
-        if (m.sfirst[o] >= 0) a = m.sfirst[o];
+    for (int s = sg + 1; s < m.nseg && a < 0; s++) {
+        const unsigned w = m.bits[(long long)s * m.W + x];
+        if (w) a = s * MASK_SEG + __ffs((int)w) - 1;
     }
+    m.before[(long long)sg * m.W + x] = b;
+    m.after[(long long)sg * m.W + x] = a;
 }
 
-// Per (pixel column x, cell row j): the column's edge rows just below and just
-// above the cell-centre height y_j (the last with edge height <= y_j and the
-// first above it: within the 32-row segment around y_j, else from the segment
-// summaries), and the smaller of their squared height differences (infinite
-// without an edge). In rounded arithmetic too no other edge of the column is
-// nearer: the squares grow with the distance.
-__global__ void k_edt_cols(MaskArgs m) {
-    const long long t = blockIdx.x * (long long)blockDim.x + threadIdx.x;
-    if (t >= (long long)m.W * m.N) return;
-    const int x = (int)(t % m.W), j = (int)(t / m.W);
-    const double yq = m.Hi + j * m.dxc;
-    // y0: the last pixel row whose edge height is <= yq (-1: none); the heights
-    // increase with the row, so a rounded estimate is corrected by single steps
+// The last pixel row whose edge height is <= yq (-1: none); the heights increase
+// with the row, so a rounded estimate is corrected by single steps.
+__device__ __forceinline__ int row_below(const MaskArgs& m, double yq) {
     int y0 = (int)floor((yq - m.eyo) / m.dyp);
     y0 = min(max(y0, -1), m.H - 1);
     while (y0 >= 0 && edge_y(m, y0) > yq) y0--;
     while (y0 + 1 < m.H && edge_y(m, y0 + 1) <= yq) y0++;
-    int prv = -1, nxt = -1;
+    return y0;
+}
+// Column x: the squared height difference of yq and the nearer of its edge rows just
+// below and just above (infinite without an edge). In rounded arithmetic too no other
+// edge of the column is nearer: the squares grow with the distance.
+__device__ __forceinline__ double column_g(const MaskArgs& m, int x, int y0, double yq) {
+    double best = HUGE_VAL;
     if (y0 >= 0) {
-        const int s0 = y0 / MASK_SEG;
-        for (int y = y0; y >= s0 * MASK_SEG; y--)
-            if (m.edge[(long long)y * m.W + x]) { prv = y; break; }
-        if (prv < 0) prv = m.before[(long long)s0 * m.W + x];
+        const long long o = (long long)(y0 / MASK_SEG) * m.W + x;
+        const unsigned w = m.bits[o] & (~0u >> (MASK_SEG - 1 - y0 % MASK_SEG));
+        const int e = w ? y0 / MASK_SEG * MASK_SEG + 31 - __clz((int)w) : m.before[o];
+        const double d = edge_y(m, e) - yq;
+        if (e >= 0) best = d * d;
     }
     if (y0 + 1 < m.H) {
-        const int y1 = y0 + 1, s1 = y1 / MASK_SEG, ye = min((s1 + 1) * MASK_SEG, m.H);
-        for (int y = y1; y < ye; y++)
-            if (m.edge[(long long)y * m.W + x]) { nxt = y; break; }
-        if (nxt < 0) nxt = m.after[(long long)s1 * m.W + x];
+        const int y1 = y0 + 1;
+        const long long o = (long long)(y1 / MASK_SEG) * m.W + x;
+        const unsigned w = m.bits[o] & (~0u << (y1 % MASK_SEG));
+        const int e = w ? y1 / MASK_SEG * MASK_SEG + __ffs((int)w) - 1 : m.after[o];
+        const double d = edge_y(m, e) - yq;
+        if (e >= 0 && d * d < best) best = d * d;
     }
-    double best = HUGE_VAL;
-    if (prv >= 0) {
-        const double d = edge_y(m, prv) - yq;
-        best = d * d;
-    }
-    if (nxt >= 0) {
-        const double d = edge_y(m, nxt) - yq;
-        if (d * d < best) best = d * d;
-    }
-    m.g1[t] = best;
+    return best;
 }
 
 // Per cell row j: phi of its cells, +- the distance to the nearest edge pixel, which
-// is the root of the least (x_e - X)^2 + g1 over the pixel columns that hold an edge
+// is the root of the least (x_e - X)^2 + g over the pixel columns that hold an edge
 // (the root is monotone, so it is taken once, of the least radicand; every radicand
 // is rounded as the reference rounds it). The columns whose parabola is least move
 // to the right with X: f_a - f_b of two columns is linear in X. So the row is cut
@@ -686,8 +663,9 @@ template <bool LDS> __global__ __launch_bounds__(EDT_THREADS) void k_edt_rows(Ma
     extern __shared__ double lds[];
     __shared__ int wsum[EDT_THREADS / 64];
     const int j = blockIdx.x, lane = threadIdx.x & 63, wv = threadIdx.x >> 6, W = m.W;
-    const double* grow = m.g1 + (long long)j * W;
-    double* ps = lds;                               // LDS: positions and g1 of the columns with an edge
+    const double yq = m.Hi + j * m.dxc;
+    const int y0 = row_below(m, yq);
+    double* ps = lds;                               // LDS: positions and g of the columns with an edge
     double* gs = ps + W;
     int* arg = (int*)(LDS ? (void*)(gs + W) : (void*)lds);  // nq + 1 bounds
     int n = W;
@@ -695,7 +673,7 @@ template <bool LDS> __global__ __launch_bounds__(EDT_THREADS) void k_edt_rows(Ma
         n = 0;
         for (int x0 = 0; x0 < W; x0 += EDT_THREADS) {
             const int x = x0 + threadIdx.x;
-            const double f = x < W ? grow[x] : HUGE_VAL;
+            const double f = x < W ? column_g(m, x, y0, yq) : HUGE_VAL;
             const bool has = f < HUGE_VAL;
             const unsigned long long b = __ballot(has);
             if (lane == 0) wsum[wv] = __popcll(b);
@@ -715,7 +693,7 @@ template <bool LDS> __global__ __launch_bounds__(EDT_THREADS) void k_edt_rows(Ma
     }
     auto radicand = [&](int x, double X) {
         const double d = (LDS ? ps[x] : edge_x(m, x)) - X;
-        return d * d + (LDS ? gs[x] : grow[x]);
+        return d * d + (LDS ? gs[x] : column_g(m, x, y0, yq));
     };
     if (threadIdx.x == 0) {
         arg[0] = 0;
@@ -738,8 +716,7 @@ template <bool LDS> __global__ __launch_bounds__(EDT_THREADS) void k_edt_rows(Ma
         if (lane == 0) arg[q] = at;
     }
     __syncthreads();
-    const double Y0 = (j + 0.5) * (m.H) / (m.N);
-    const signed char* vrow = m.v + (long long)(int)Y0 * W;
+    const int ys = (int)((j + 0.5) * (m.H) / (m.N));
     for (int q = wv; q < nq; q += EDT_THREADS / 64) {
         const int lo = arg[q], hi = min(arg[q + 1], n - 1);  // none without an edge
         const int iend = min((q + 1) * stride, m.M);
@@ -755,19 +732,15 @@ template <bool LDS> __global__ __launch_bounds__(EDT_THREADS) void k_edt_rows(Ma
             const double dmin = d < 100.0 ? d : 100.0;  // Level_Set.cpp:131 starts every search at 100
             // the sign sampled at pixel (int((i+0.5) W / M), int((j+0.5) H / N))
             const int xs = (int)((i + 0.5) * (W) / (m.M));
-            m.phi[(long long)j * m.M + i] = (vrow[xs] >= 0 ? 1 : -1) * dmin;
+            m.phi[(long long)j * m.M + i] = (mask_sign(m, xs, ys) ? 1 : -1) * dmin;
         }
     }
 }
 
 hipError_t mask_run(MaskArgs& m, bool lds, hipStream_t s) {
-    dim3 pg((m.W + 255) / 256, m.H);
-    hipLaunchKernelGGL(k_mask_sign, pg, dim3(256), 0, s, m);
-    hipLaunchKernelGGL(k_mask_edge, pg, dim3(256), 0, s, m);
-    hipLaunchKernelGGL(k_edt_segs, dim3((m.W + 255) / 256, m.nseg), dim3(256), 0, s, m);
-    hipLaunchKernelGGL(k_edt_segscan, dim3((m.W + 255) / 256), dim3(256), 0, s, m);
-    const long long nc = (long long)m.W * m.N;
-    hipLaunchKernelGGL(k_edt_cols, dim3((unsigned)((nc + 255) / 256)), dim3(256), 0, s, m);
+    const dim3 cols((m.W + 255) / 256, m.nseg);
+    hipLaunchKernelGGL(k_mask_edges, cols, dim3(256), 0, s, m);
+    hipLaunchKernelGGL(k_mask_beyond, cols, dim3(256), 0, s, m);
     const int stride = edt_stride(m.M), nq = edt_intervals(m.M);
     if (lds) {
         hipLaunchKernelGGL(k_edt_rows<true>, dim3(m.N), dim3(EDT_THREADS), mask_lds_bytes(m.W, m.M), s, m, stride, nq);
