@@ -38,6 +38,7 @@ void set_error(const char* fmt, ...) {
     } while (0)
 
 static long long round_up(long long v, long long m) { return (v + m - 1) / m * m; }
+constexpr long long SLAB_ALIGN = 4096;
 
 // Device memory of a context: from its arena when it belongs to a batch, else hipMalloc.
 template <class P> static hipError_t dalloc(ibtfo_ctx* x, P** p, size_t bytes) {
@@ -60,9 +61,20 @@ static void drop_graph(ibtfo_ctx* x) {
 }
 
 static void dfree(ibtfo_ctx* x, void* p) {
-    if (!p) return;
+    if (!p || ((char*)p >= x->slab && (char*)p < x->slab + x->slab_bytes)) return;  // the slab's parts go with it
     if (x->arena) x->arena->free(p);
     else (void)hipFree(p);
+}
+// A buffer of at least `bytes`, kept from the last geometry where it suffices: a
+// hipMalloc and its hipFree cost 30 to 600 us with the size.
+static hipError_t dgrow(ibtfo_ctx* x, char** p, size_t* cap, size_t bytes) {
+    if (bytes <= *cap) return hipSuccess;
+    dfree(x, *p);
+    *p = nullptr;
+    *cap = 0;
+    const hipError_t e = dalloc(x, p, bytes);
+    if (e == hipSuccess) *cap = bytes;
+    return e;
 }
 // Copies ordered on the context's stream (never the null stream, which would
 // wait for every other blocking stream of the device).
@@ -162,11 +174,13 @@ extern "C" long long ibtfo_footprint(const ibtfo_config* c) {
 void ibtfo::free_ctx(ibtfo_ctx* x) {
     if (!x) return;
     if (x->graph) (void)hipGraphExecDestroy(x->graph);
-    for (void* p : {(void*)x->state[0], (void*)x->state[1], (void*)x->type, (void*)x->phi, (void*)x->gnx,
-                    (void*)x->gny, (void*)x->ghosts, (void*)x->gvals, (void*)x->dcount, (void*)x->ctl,
-                    (void*)x->mass_part, (void*)x->corner, (void*)x->cuts, (void*)x->cut_index, (void*)x->groups,
-                    (void*)x->stype, (void*)x->merge_part, (void*)x->fold, (void*)x->unew0, (void*)x->df_part})
+    if (x->arena)
+        for (void* p : {(void*)x->state[0], (void*)x->state[1], (void*)x->type, (void*)x->phi, (void*)x->gnx,
+                        (void*)x->gny, (void*)x->dcount, (void*)x->ctl, (void*)x->corner, (void*)x->fold})
+            dfree(x, p);
+    for (void* p : {(void*)x->mass_part, (void*)x->cut_mem, (void*)x->rec_mem, (void*)x->ghost_mem, (void*)x->unew0})
         dfree(x, p);
+    if (x->slab) (void)hipFree(x->slab);
     if (x->own_stream) (void)hipStreamDestroy(x->own_stream);
     delete x;
 }
@@ -193,39 +207,54 @@ int ctx_create(const ibtfo_config* cfg, Arena* arena, hipStream_t stream, int ro
         free_ctx(x);
         return IBTFO_E_NOMEM;
     };
-    if (dalloc(x, &x->state[0], 4 * L.plane * sizeof(double)) != hipSuccess) return fail("state");
-    if (dalloc(x, &x->state[1], 4 * L.plane * sizeof(double)) != hipSuccess) return fail("state");
-    if (dalloc(x, &x->type, L.plane) != hipSuccess) return fail("types");
-    if (dalloc(x, &x->phi, L.plane * sizeof(double)) != hipSuccess) return fail("phi");
-    if (dalloc(x, &x->gnx, L.plane * sizeof(double)) != hipSuccess) return fail("normals");
-    if (dalloc(x, &x->gny, L.plane * sizeof(double)) != hipSuccess) return fail("normals");
-    if (dalloc(x, &x->ctl, sizeof(Ctl)) != hipSuccess) return fail("control");
-    if (dalloc(x, &x->fold, FOLD_MAX * PART_STRIDE * sizeof(double)) != hipSuccess) return fail("partials");
-    if (dalloc(x, &x->dcount, sizeof(unsigned int)) != hipSuccess) return fail("counter");
     int nbx, nby, r;
     step_grid(L, rows, &nbx, &nby, &r);
     x->mass_cap = arena ? nbx * nby : std::max(nbx * nby, 4096);
-    if (dalloc(x, &x->mass_part, PART_STRIDE * (size_t)x->mass_cap * sizeof(double)) != hipSuccess)
-        return fail("partials");
-    if (dalloc(x, &x->corner, 2 * 2 * L.ng * 4 * sizeof(double)) != hipSuccess) return fail("corner");
-    const size_t df_bytes = 2 * (size_t)DF_MAX_REC * PART_STRIDE * sizeof(double);
-    if (!arena && dalloc(x, &x->df_part, df_bytes) != hipSuccess) return fail("partials");
+    const size_t plane8 = L.plane * sizeof(double);
+    struct Part { void** p; size_t bytes; const char* what; };
+    const Part parts[] = {
+        {(void**)&x->state[0], 4 * plane8, "state"}, {(void**)&x->state[1], 4 * plane8, "state"},
+        {(void**)&x->phi, plane8, "phi"}, {(void**)&x->gnx, plane8, "normals"}, {(void**)&x->gny, plane8, "normals"},
+        {(void**)&x->ctl, sizeof(Ctl), "control"}, {(void**)&x->corner, 2 * 2 * L.ng * 4 * sizeof(double), "corner"},
+        {(void**)&x->df_part, arena ? 0 : 2 * (size_t)DF_MAX_REC * PART_STRIDE * sizeof(double), "partials"},
+        // cleared up to here
+        {(void**)&x->type, (size_t)L.plane, "types"},
+        {(void**)&x->fold, FOLD_MAX * PART_STRIDE * sizeof(double), "partials"},
+        {(void**)&x->dcount, sizeof(unsigned int), "counter"},
+        {(void**)&x->mass_part, PART_STRIDE * (size_t)x->mass_cap * sizeof(double), "partials"}};
+    constexpr int CLEARED = 8;
+    size_t clear_bytes = 0;
+    if (!arena) {
+        for (const Part& q : parts) x->slab_bytes += (size_t)round_up((long long)q.bytes, SLAB_ALIGN);
+        if (dalloc(x, &x->slab, x->slab_bytes) != hipSuccess) {
+            x->slab_bytes = 0;
+            return fail("state");
+        }
+    }
+    size_t at = 0;
+    for (int k = 0; k < (int)(sizeof parts / sizeof *parts); k++) {
+        const Part& q = parts[k];
+        if (q.bytes == 0) continue;
+        if (arena) {
+            if (dalloc(x, (char**)q.p, q.bytes) != hipSuccess) return fail(q.what);
+        } else {
+            *q.p = x->slab + at;
+            at += (size_t)round_up((long long)q.bytes, SLAB_ALIGN);
+            if (k < CLEARED) clear_bytes = at;
+        }
+    }
     if (stream) {
         x->stream = stream;
     } else {
         if (hipStreamCreateWithFlags(&x->own_stream, hipStreamNonBlocking) != hipSuccess) return fail("stream");
         x->stream = x->own_stream;
     }
-    if (hipMemsetAsync(x->state[0], 0, 4 * L.plane * sizeof(double), x->stream) != hipSuccess ||
-        hipMemsetAsync(x->state[1], 0, 4 * L.plane * sizeof(double), x->stream) != hipSuccess ||
-        hipMemsetAsync(x->type, 2, L.plane, x->stream) != hipSuccess ||
-        hipMemsetAsync(x->ctl, 0, sizeof(Ctl), x->stream) != hipSuccess ||
-        hipMemsetAsync(x->phi, 0, L.plane * sizeof(double), x->stream) != hipSuccess ||
-        hipMemsetAsync(x->gnx, 0, L.plane * sizeof(double), x->stream) != hipSuccess ||
-        hipMemsetAsync(x->gny, 0, L.plane * sizeof(double), x->stream) != hipSuccess ||
-        hipMemsetAsync(x->corner, 0, 2 * 2 * L.ng * 4 * sizeof(double), x->stream) != hipSuccess ||
-        (x->df_part && hipMemsetAsync(x->df_part, 0, df_bytes, x->stream) != hipSuccess))
-        return fail("initial clear");  // stream-ordered before everything else on the solve's stream
+    // stream-ordered before everything else on the solve's stream
+    hipError_t e = hipMemsetAsync(x->type, 2, L.plane, x->stream);
+    if (!arena && e == hipSuccess) e = hipMemsetAsync(x->slab, 0, clear_bytes, x->stream);
+    for (int k = 0; arena && k < CLEARED && e == hipSuccess; k++)
+        if (parts[k].bytes) e = hipMemsetAsync(*parts[k].p, 0, parts[k].bytes, x->stream);
+    if (e != hipSuccess) return fail("initial clear");
     const double Psy_L = cfg->hi_x - cfg->lo_x;
     x->dxc = Psy_L / cfg->N_x;  // Psy_coord.cpp:21-22 (y spaced with dx as well)
     x->Li = -x->dxc * L.ng + cfg->lo_x + x->dxc / 2;
@@ -296,56 +325,49 @@ extern "C" int ibtfo_cut_counts(const ibtfo_ctx* x, int* cut_cells, int* merge_g
 // records, the index plane, the groups and the step kernel's type plane, in which the
 // groups' cells (targets and members) carry MERGED_BIT: the step leaves their dt /
 // mass partials to the merge kernel, which writes one record per block.
-static int cut_geometry(ibtfo_ctx* x, GeomArgs& g) {
+// Counts the ghosts of geometry_finish's list along with them.
+static int cut_geometry(ibtfo_ctx* x, GeomArgs& g, unsigned int* nghost) {
     const Layout& L = x->L;
-    for (void** p : {(void**)&x->cuts, (void**)&x->cut_index, (void**)&x->groups, (void**)&x->stype,
-                     (void**)&x->merge_part}) {
-        dfree(x, *p);
-        *p = nullptr;
-    }
-    x->ncut = x->ngroups = 0;
-    const size_t marks = (size_t)round_up(L.plane, 8);  // the two counters stand behind them
-    if (dalloc(x, &g.cmark, marks + 2 * sizeof(unsigned)) != hipSuccess ||
-        dalloc(x, &x->cut_index, (size_t)L.plane * sizeof(int)) != hipSuccess ||
-        dalloc(x, &x->stype, L.plane) != hipSuccess) {
-        dfree(x, g.cmark);
+    const size_t index = (size_t)round_up(L.plane * sizeof(int), 256), bytes = (size_t)round_up(L.plane, 256);
+    if (!x->cut_mem && dalloc(x, &x->cut_mem, index + 2 * bytes + 3 * sizeof(unsigned)) != hipSuccess) {
         set_error("cut-cell geometry: out of device memory");
         return IBTFO_E_NOMEM;
     }
-    g.ccount = (unsigned*)(g.cmark + marks);
-    g.cut_index = x->cut_index;
-    g.stype = x->stype;
+    x->cut_index = g.cut_index = (int*)x->cut_mem;
+    x->stype = g.stype = (uint8_t*)x->cut_mem + index;
+    g.cmark = g.stype + bytes;
+    g.ccount = (unsigned*)(g.cmark + bytes);
+    x->cuts = nullptr;
+    x->groups = nullptr;
+    x->merge_part = nullptr;
+    x->ncut = x->ngroups = 0;
     g.cuts = nullptr;
-    unsigned int cnt[2] = {0, 0};
-    hipError_t e = hipMemsetAsync(g.ccount, 0, sizeof cnt, x->stream);
-    if (e == hipSuccess) e = cut_run(g, x->stream);
-    if (e == hipSuccess) e = cut_records(g, x->stream);
-    if (e == hipSuccess) e = scopy(x, cnt, g.ccount, sizeof cnt, hipMemcpyDeviceToHost);
-    int rc = IBTFO_OK;
-    if (e == hipSuccess) e = hipMemcpyAsync(x->stype, x->type, L.plane, hipMemcpyDeviceToDevice, x->stream);
-    if (e == hipSuccess && cnt[0]) {  // a merge group holds cut cells
-        x->ncut = (int)cnt[0];
-        x->ngroups = (int)cnt[1];
-        if (dalloc(x, &x->cuts, x->ncut * sizeof(CutCell)) != hipSuccess ||
-            (x->ngroups &&
-             (dalloc(x, &x->groups, x->ngroups * sizeof(MergeGroup)) != hipSuccess ||
-              dalloc(x, &x->merge_part, PART_STRIDE * (size_t)merge_blocks(x->ngroups) * sizeof(double)) !=
-                  hipSuccess))) {
-            set_error("cut-cell geometry: out of device memory for %d records", x->ncut);
-            rc = IBTFO_E_NOMEM;
-        } else {
-            g.cuts = x->cuts;
-            g.ccap = x->ncut;
-            g.groups = x->groups;
-            g.gcap = x->ngroups;
-            e = hipMemsetAsync(g.ccount, 0, sizeof cnt, x->stream);
-            if (e == hipSuccess) e = cut_records(g, x->stream);
-        }
+    g.count = g.ccount + 2;
+    g.cap = 0;
+    unsigned int cnt[3] = {0, 0, 0};
+    HIPCHK(hipMemsetAsync(g.ccount, 0, sizeof cnt, x->stream));
+    HIPCHK(cut_run(g, x->stream));
+    HIPCHK(cut_records(g, x->stream));
+    HIPCHK(geom_ghosts(g, x->stream));
+    HIPCHK(hipMemcpyAsync(x->stype, x->type, L.plane, hipMemcpyDeviceToDevice, x->stream));
+    HIPCHK(scopy(x, cnt, g.ccount, sizeof cnt, hipMemcpyDeviceToHost));
+    *nghost = cnt[2];
+    if (!cnt[0]) return IBTFO_OK;  // a merge group holds cut cells
+    const size_t cb = (size_t)round_up(cnt[0] * sizeof(CutCell), 256), gb = (size_t)round_up(cnt[1] * sizeof(MergeGroup), 256);
+    if (dgrow(x, &x->rec_mem, &x->rec_cap,
+              cb + gb + PART_STRIDE * (size_t)merge_blocks((int)cnt[1]) * sizeof(double)) != hipSuccess) {
+        set_error("cut-cell geometry: out of device memory for %u records", cnt[0]);
+        return IBTFO_E_NOMEM;
     }
-    if (e == hipSuccess) e = hipStreamSynchronize(x->stream);
-    dfree(x, g.cmark);
-    if (rc) return rc;
-    HIPCHK(e);
+    x->ncut = g.ccap = (int)cnt[0];
+    x->cuts = g.cuts = (CutCell*)x->rec_mem;
+    if (cnt[1]) {
+        x->ngroups = g.gcap = (int)cnt[1];
+        x->groups = g.groups = (MergeGroup*)(x->rec_mem + cb);
+        x->merge_part = (double*)(x->rec_mem + cb + gb);
+    }
+    HIPCHK(hipMemsetAsync(g.ccount, 0, sizeof cnt, x->stream));
+    HIPCHK(cut_records(g, x->stream));
     return IBTFO_OK;
 }
 
@@ -399,45 +421,53 @@ static hipError_t launch_fill_levels(ibtfo_ctx* x, FillArgs f) {
     return hipSuccess;
 }
 
-static int geometry_finish(ibtfo_ctx* x, GeomArgs& g, double* dphi) {
-    // the ghost list, cut-cell records and merge groups are rebuilt below (new
-    // buffers and counts): a graph captured over the old ones must not replay
+// The ghost list's two passes: interior cells of type 2, counted, then their records
+static int count_ghosts(ibtfo_ctx* x, GeomArgs& g, unsigned int* cnt) {
+    HIPCHK(hipMemsetAsync(g.count, 0, sizeof *cnt, x->stream));
+    HIPCHK(geom_ghosts(g, x->stream));
+    HIPCHK(scopy(x, cnt, g.count, sizeof *cnt, hipMemcpyDeviceToHost));
+    return IBTFO_OK;
+}
+static int fill_ghosts(ibtfo_ctx* x, GeomArgs& g) {
+    HIPCHK(hipMemsetAsync(g.count, 0, sizeof(unsigned), x->stream));
+    HIPCHK(geom_ghosts(g, x->stream));
+    return IBTFO_OK;
+}
+
+static int geometry_finish(ibtfo_ctx* x, GeomArgs& g, void* dphi) {
+    // the ghost list, cut-cell records and merge groups are rebuilt below (other
+    // counts, perhaps other buffers): a graph captured over the old must not replay
     drop_graph(x);
     x->prepared = 0;
     hipError_t ge = geom_run(g, x->stream);
     if (ge != hipSuccess) { dfree(x, dphi); HIPCHK(ge); }
-    if (x->cfg.boundary == IBTFO_CUTCELL) {
-        int rc = cut_geometry(x, g);
-        if (rc) { dfree(x, dphi); return rc; }
-    }
-    // ghost list (upper bound: all interior cells of type 2; count first)
-    dfree(x, x->ghosts); x->ghosts = nullptr;
-    dfree(x, x->gvals); x->gvals = nullptr;
+    unsigned int cnt = 0;
+    x->ghosts = nullptr;
+    x->gvals = nullptr;
     x->nghost = 0;
-    if (x->cfg.boundary != IBTFO_REGULAR) {
-        unsigned int zero = 0, cnt = 0;
-        HIPCHK(hipMemcpyAsync(x->dcount, &zero, sizeof zero, hipMemcpyHostToDevice, x->stream));
-        g.count = x->dcount; g.cap = 0; g.ghosts = nullptr;
-        HIPCHK(geom_ghosts(g, x->stream));
-        HIPCHK(hipMemcpyAsync(&cnt, x->dcount, sizeof cnt, hipMemcpyDeviceToHost, x->stream));
-        HIPCHK(hipStreamSynchronize(x->stream));
-        if (cnt > 0) {
-            if (dalloc(x, &x->ghosts, cnt * sizeof(Ghost)) != hipSuccess ||
-                dalloc(x, &x->gvals, cnt * 4 * sizeof(double)) != hipSuccess) {
-                dfree(x, dphi);
-                set_error("geometry: out of device memory for %u ghost records", cnt);
-                return IBTFO_E_NOMEM;
-            }
-            HIPCHK(hipMemcpyAsync(x->dcount, &zero, sizeof zero, hipMemcpyHostToDevice, x->stream));
-            g.ghosts = x->ghosts; g.cap = (int)cnt;
-            HIPCHK(geom_ghosts(g, x->stream));
+    int rc = IBTFO_OK;
+    if (x->cfg.boundary == IBTFO_CUTCELL) {
+        rc = cut_geometry(x, g, &cnt);
+    } else if (x->cfg.boundary != IBTFO_REGULAR) {
+        g.count = x->dcount;
+        g.cap = 0;
+        rc = count_ghosts(x, g, &cnt);
+    }
+    if (!rc && cnt > 0) {
+        const size_t gb = (size_t)round_up(cnt * sizeof(Ghost), 256);
+        if (dgrow(x, &x->ghost_mem, &x->ghost_cap, gb + cnt * 4 * sizeof(double)) != hipSuccess) {
+            set_error("geometry: out of device memory for %u ghost records", cnt);
+            rc = IBTFO_E_NOMEM;
+        } else {
+            x->ghosts = g.ghosts = (Ghost*)x->ghost_mem;
+            x->gvals = (double*)(x->ghost_mem + gb);
+            x->nghost = g.cap = (int)cnt;
+            rc = fill_ghosts(x, g);
         }
-        x->nghost = (int)cnt;
     }
-    {
-        int rc = simple_bound_levels(x);
-        if (rc) { dfree(x, dphi); return rc; }
-    }
+    if (rc) { dfree(x, dphi); return rc; }
+    rc = simple_bound_levels(x);
+    if (rc) { dfree(x, dphi); return rc; }
     HIPCHK(hipStreamSynchronize(x->stream));
     dfree(x, dphi);
     x->have_geometry = 1;
@@ -542,28 +572,28 @@ extern "C" int ibtfo_geometry_mask(ibtfo_ctx* x, const unsigned char* rgba, int 
     const bool lds_rows = lds_bytes <= MASK_LDS_MAX &&
                           hipFuncSetAttribute(mask_rows_kernel(), hipFuncAttributeMaxDynamicSharedMemorySize,
                                               (int)lds_bytes) == hipSuccess;
-    unsigned *drgba = nullptr, *dbits = nullptr;
-    double* dphi = nullptr;
-    int *dbe = nullptr, *daf = nullptr;
-    auto release = [&]() {
-        for (void* p : {(void*)drgba, (void*)dbits, (void*)dbe, (void*)daf}) dfree(x, p);
-    };
-    if (dalloc(x, &drgba, WH * 4) != hipSuccess || dalloc(x, &dbits, SW * sizeof(int)) != hipSuccess ||
-        dalloc(x, &dbe, SW * sizeof(int)) != hipSuccess || dalloc(x, &daf, SW * sizeof(int)) != hipSuccess ||
-        dalloc(x, &dphi, (size_t)L.M * L.N * sizeof(double)) != hipSuccess) {
-        release();
-        dfree(x, dphi);
-        set_error("ibtfo_geometry_mask: out of device memory");
-        return IBTFO_E_NOMEM;
+    // The image and its bit words are read before geom_run writes the normals, whose
+    // planes they take where they fit (a pixel per cell and more do: two doubles)
+    const size_t rgba_bytes = (size_t)round_up(WH * 4, 256), words = (size_t)round_up(SW * 4, 256);
+    const size_t plane8 = L.plane * sizeof(double);
+    char* tmp = nullptr;
+    if (rgba_bytes > plane8 || 3 * words > plane8) {
+        if (dalloc(x, &tmp, rgba_bytes + 3 * words) != hipSuccess) {
+            set_error("ibtfo_geometry_mask: out of device memory");
+            return IBTFO_E_NOMEM;
+        }
     }
-    m.rgba = drgba; m.bits = dbits; m.before = dbe; m.after = daf;
-    m.phi = dphi;
-    hipError_t e = scopy(x, drgba, rgba, WH * 4, hipMemcpyHostToDevice);
+    m.rgba = tmp ? (unsigned*)tmp : (unsigned*)x->gnx;
+    char* w = tmp ? tmp + rgba_bytes : (char*)x->gny;
+    m.bits = (unsigned*)w;
+    m.before = (int*)(w + words);
+    m.after = (int*)(w + 2 * words);
+    m.L = L;
+    m.phi = x->phi;
+    hipError_t e = scopy(x, (void*)m.rgba, rgba, WH * 4, hipMemcpyHostToDevice);
     if (e == hipSuccess) e = mask_run(m, lds_rows, x->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(x->stream);
-    release();
     if (e != hipSuccess) {
-        dfree(x, dphi);
+        dfree(x, tmp);
         set_error("ibtfo_geometry_mask: %s", hipGetErrorString(e));
         return IBTFO_E_HIP;
     }
@@ -572,14 +602,13 @@ extern "C" int ibtfo_geometry_mask(ibtfo_ctx* x, const unsigned char* rgba, int 
     g.L = L;
     g.Li = x->Li; g.Hi = x->Hi; g.dx = x->dxc;
     g.kind = IBTFO_LS_FIELD;
-    g.phi_in = dphi;
     g.phi = x->phi; g.nx = x->gnx; g.ny = x->gny; g.type = x->type;
     g.bc = c.boundary == IBTFO_CUTCELL ? IBTFO_IDW_GFM : c.boundary;
     g.unit_normals = c.quirks == 0;
     g.cut = c.boundary == IBTFO_CUTCELL;
     g.cdx = Psy_L / c.N_x;
     g.cdy = Psy_H / c.N_y;
-    return geometry_finish(x, g, dphi);
+    return geometry_finish(x, g, tmp);
 }
 
 extern "C" int ibtfo_geometry_png(ibtfo_ctx* x, const char* path) {

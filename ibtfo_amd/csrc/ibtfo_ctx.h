@@ -52,6 +52,13 @@ struct ibtfo_ctx {
     int graph_chunk;
     std::vector<double> corner_host;
     ibtfo::Arena* arena;  // device memory from a batch engine's arena (else hipMalloc)
+    // Device memory behind the pointers above: what a context always holds (slab; one
+    // allocation, arena contexts take the parts singly), the cut-cell planes, and the
+    // cut-cell and ghost records, kept for the next geometry when they suffice
+    char* slab;
+    size_t slab_bytes;
+    char *cut_mem, *rec_mem, *ghost_mem;
+    size_t rec_cap, ghost_cap;
 };
 
 namespace ibtfo {

@@ -12,7 +12,7 @@ struct GeomArgs {
     double Li, Hi, dx;      // first cell centre (with ghosts) and spacing, Psy_coord.cpp:21-26
     int kind;               // level-set hook
     double p[8];            // hook constants (evaluated on the host)
-    const double* phi_in;   // kind 3: per-cell phi in reference cell order
+    const double* phi_in;   // kind 3: per-cell phi in reference cell order (null: phi holds it)
     const double* shapes;   // kind 5: nshapes records of SHAPE_STRIDE doubles
     int nshapes;
     double *phi, *nx, *ny;  // planes
@@ -45,7 +45,8 @@ struct MaskArgs {
     int nseg;                   // 32-row segments per pixel column
     unsigned* bits;             // nseg x W: edge pixels of each segment
     int *before, *after;        // nseg x W: last edge row below / first above each segment (-1: none)
-    double* phi;                // M x N, reference cell order
+    Layout L;
+    double* phi;                // plane
 };
 constexpr int MASK_SEG = 32;
 // The row search (k_edt_rows): cells per bounded interval, intervals, LDS bytes

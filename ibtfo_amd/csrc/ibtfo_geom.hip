@@ -305,7 +305,7 @@ __device__ void ghost_record(const GeomArgs& g, int i, int j, unsigned int slot)
 
 hipError_t geom_run(GeomArgs& g, hipStream_t s) {
     dim3 blk(128), grd((g.L.M + 127) / 128, g.L.N);
-    hipLaunchKernelGGL(k_geom_phi, grd, blk, 0, s, g);
+    if (g.kind != IBTFO_LS_FIELD || g.phi_in) hipLaunchKernelGGL(k_geom_phi, grd, blk, 0, s, g);
     hipLaunchKernelGGL(k_geom_classify, grd, blk, 0, s, g);
     return hipGetLastError();
 }
@@ -732,7 +732,7 @@ template <bool LDS> __global__ __launch_bounds__(EDT_THREADS) void k_edt_rows(Ma
             const double dmin = d < 100.0 ? d : 100.0;  // Level_Set.cpp:131 starts every search at 100
             // the sign sampled at pixel (int((i+0.5) W / M), int((j+0.5) H / N))
             const int xs = (int)((i + 0.5) * (W) / (m.M));
-            m.phi[(long long)j * m.M + i] = (mask_sign(m, xs, ys) ? 1 : -1) * dmin;
+            m.phi[m.L.at(i, j)] = (mask_sign(m, xs, ys) ? 1 : -1) * dmin;
         }
     }
 }
