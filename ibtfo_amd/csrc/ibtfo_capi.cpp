@@ -111,16 +111,22 @@ static int step_grid(const Layout& L, int rows, int* nbx, int* nby, int* out_row
 // us per step, row-parallel against the best marching strip: 64x64 8.8 / 9.7,
 // 256x128 9.9 / 13.9, 400x100 (one kernel per step) 8.8 / 13.7, 512x256 15.5 / 20.8,
 // 512x512 with two stages 42.8 / 48.1, 800x400 26.1 / 29.3 (ghost fluid: 26.8 / 25.2).
+// In FP64 with cut cells or Steger-Warming, whose marching strips hold the most work
+// beside the rows they recompute, 7-row blocks stay ahead up to 2200: 1003x517 cut HLL
+// 35.8 / 39.0, Steger-Warming 40.0 / 42.8, 1300x700 48.4 / 50.3 and 58.1 / 58.9; the
+// others are even there (1100x570 ghost fluid 38.3 / 37.2, mixed 30.7 / 28.4).
 // Larger grids march: a strip of r rows computes r + 1 y faces and r + 2 rows of y
 // states, so few rows cost work and many cost balance over the 4096 waves that run
-// together: 1024x512: 3 rows 32.3, 6 rows 35.3; 2048x1024: 3 rows 75.3, 6 rows 71.7,
-// 8 rows 77.3; 4096x2048: 6 rows 244, 8 rows 237, 18 rows 244.
+// together: 1024x512: 3 rows 32.3, 6 rows 35.3; 2048x1024 cut HLL: 3 rows 81.2, 6 rows
+// 82.7, 8 rows 84.4, mixed 57.3, 53.2, 55.6; 4096x2048 Steger-Warming: 8 rows 315.5,
+// 10 rows 309.4, 12 rows 314.0; 8192x4096 cut HLL: 8 rows 822, 10 rows 802, 12 rows 793.
 static void default_tile(const ibtfo_config& c, const Layout& L, int* rows, int* par) {
     const long long nbx = (L.nx + STRIP_W - 1) / STRIP_W, cells = (long long)L.nx * L.ny;
     auto blocks = [&](int r) { return nbx * ((L.ny + r - 1) / r); };
     *par = 0;
-    *rows = cells < 900000 ? 3 : (cells < 2200000 ? 6 : 8);
-    if (c.scheme == IBTFO_LAX || blocks(ROWPAR_MAX_ROWS) > 1024) return;
+    *rows = cells < 900000 ? 3 : cells < 2200000 ? 6 : cells < 7000000 ? 8 : cells < 12000000 ? 10 : 12;
+    const bool heavy = c.precision == IBTFO_FP64 && (c.boundary == IBTFO_CUTCELL || c.riemann == IBTFO_STEGER_WARMING);
+    if (c.scheme == IBTFO_LAX || blocks(ROWPAR_MAX_ROWS) > (heavy ? 2200 : 1024)) return;
     *par = 1;
     *rows = ROWPAR_MAX_ROWS;
     const int cap = blocks(ROWPAR_MAX_ROWS) <= 256 ? 256 : 512;
