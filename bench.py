@@ -12,8 +12,8 @@ a third leg runs the reference's IDW ghost-fluid boundary in place of the cut
 cells.
 A step = the step kernel (reconstruction, fluxes, update, per-block dt/mass
 partials), the small-cell merge kernel (with the merged cells' dt/mass
-partials), the dt/clock kernel, and the ghost-fill kernels (the first of them
-also fills the edge ring). The state is initialised on the device before the timed region and
+partials), and one kernel for the dt/clock reduction, the ghost fill and the edge
+ring. The state is initialised on the device before the timed region and
 dt never leaves the device. The step kernel's tile height is picked by the
 library's autotuner; the timed loop replays a captured HIP graph of the step
 sequence.

@@ -1,6 +1,6 @@
 // Batch engine: many independent solves served by one device-resident loop
 // (include/ibtfo.h, "Batch engine"). Solves of different sizes share batched
-// launches of the step, finish, ghost-fill and edge kernels: each launch's grid
+// launches (the step; the finish, ghost fill and edge ring): each launch's grid
 // covers the strips (ghosts, ring cells) of every resident solve through a
 // block map, and the whole chunk of steps is one captured HIP graph whose
 // arguments never change (tables and maps live at fixed device addresses and

@@ -97,8 +97,8 @@ struct StepArgs {
                             // flip: reads U1 from buf[cur ^ 1], writes over U^n in buf[cur]
     const CutCell* cut;     // cut-cell records (type-3 cells), else null
     const int* cut_index;   // plane: record of each type-3 cell
-    int in_hint;            // the buffer the host expects to be this launch's input (row-parallel
-                            // form: read before the control block says which it is)
+    int in_hint;            // the buffer the host expects to be this launch's input: its first rows
+                            // are read before the control block says which it is
     int rowpar;             // row-parallel form (k_step_rowpar: rows + 1 waves per block)
     // Deferred finish (row-parallel form, single-step, Regular boundary with a
     // ring the step kernel writes, at most DF_MAX_REC blocks): no finish kernel
