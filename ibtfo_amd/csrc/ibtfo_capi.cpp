@@ -108,18 +108,21 @@ static int step_grid(const Layout& L, int rows, int* nbx, int* nby, int* out_row
 // row-parallel form runs a strip's rows at once, and is best with the fewest rows
 // that leave at most one block per CU (256), else at most two (512), the blocks
 // that run together; with more, its 7-row strips up to two rounds of those. Measured,
-// us per step, row-parallel against the best marching strip: 64x64 8.8 / 9.7,
-// 256x128 9.9 / 13.9, 400x100 (one kernel per step) 8.8 / 13.7, 512x256 15.5 / 20.8,
-// 512x512 with two stages 42.8 / 48.1, 800x400 26.1 / 29.3 (ghost fluid: 26.8 / 25.2).
+// us per step, row-parallel against the best marching strip: 64x64 8.8 / 9.6,
+// 256x128 9.8 / 13.4, 400x100 (one kernel per step) 8.7 / 13.1, 512x256 15.4 / 20.8,
+// 512x512 with two stages 44.8 / 48.1; 800x400 is even (25.5 / 24.9, ghost fluid in
+// FP64 27.1 / 26.6), 900x460 for the row-parallel form again (990 blocks, a fuller
+// second round: 27.7 / 30.2).
 // In FP64 with cut cells or Steger-Warming, whose marching strips hold the most work
 // beside the rows they recompute, 7-row blocks stay ahead up to 2200: 1003x517 cut HLL
-// 35.8 / 39.0, Steger-Warming 40.0 / 42.8, 1300x700 48.4 / 50.3 and 58.1 / 58.9; the
-// others are even there (1100x570 ghost fluid 38.3 / 37.2, mixed 30.7 / 28.4).
+// 35.9 / 38.5, Steger-Warming 40.1 / 43.0; at the line they are even (1300x700 49.5 /
+// 48.7 and 58.9 / 58.2), as the others are before it (1100x570 ghost fluid 37.1 /
+// 36.3, mixed 30.7 / 27.9).
 // Larger grids march: a strip of r rows computes r + 1 y faces and r + 2 rows of y
 // states, so few rows cost work and many cost balance over the 4096 waves that run
-// together: 1024x512: 3 rows 32.3, 6 rows 35.3; 2048x1024 cut HLL: 3 rows 81.2, 6 rows
-// 82.7, 8 rows 84.4, mixed 57.3, 53.2, 55.6; 4096x2048 Steger-Warming: 8 rows 315.5,
-// 10 rows 309.4, 12 rows 314.0; 8192x4096 cut HLL: 8 rows 822, 10 rows 802, 12 rows 793.
+// together: 1024x512: 3 rows 32.2, 6 rows 37.4; 2048x1024 cut HLL: 3 rows 78.1, 6 rows
+// 79.2, 8 rows 80.8, mixed 54.8, 51.2, 54.0; 4096x2048 Steger-Warming: 8 rows 313.2,
+// 10 rows 305.3, 12 rows 311.5; 8192x4096 cut HLL: 8 rows 807, 10 rows 775, 12 rows 766.
 static void default_tile(const ibtfo_config& c, const Layout& L, int* rows, int* par) {
     const long long nbx = (L.nx + STRIP_W - 1) / STRIP_W, cells = (long long)L.nx * L.ny;
     auto blocks = [&](int r) { return nbx * ((L.ny + r - 1) / r); };
