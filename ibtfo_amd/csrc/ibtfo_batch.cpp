@@ -175,8 +175,8 @@ static int cfg_step_blocks(const ibtfo_config& c, int rows) {
 // or 16 where the step blocks are short: the request would not fit, or the batch
 // holds less than two rounds of the chip's 4096 waves (256 CUs, 16 waves each), so
 // that taller strips let more solves in. 24 solves of 64x64 to 1024x512 in mixed
-// precision, 3.8 M cells: 97 us per step with 16 rows (3900 waves, one round that
-// lasts as long as a strip), 86 with 8, 88 with 6, 91 with 4.
+// precision, 3.8 M cells: 93 us per step with 16 rows (3900 waves, one round that
+// lasts as long as a strip), 84 with 8, 86 with 6, 89 with 4.
 constexpr int BATCH_WAVES = 4096;
 static int batch_rows(const ibtfo_batch_config& k, const ibtfo_config& c) {
     if (k.rows > 0) return k.rows;
