@@ -447,7 +447,8 @@ static int geometry_finish(ibtfo_ctx* x, GeomArgs& g, void* dphi) {
     // the ghost list, cut-cell records and merge groups are rebuilt below (other
     // counts, perhaps other buffers): a graph captured over the old must not replay
     drop_graph(x);
-    x->prepared = 0;
+    // none until the last list is built: a failure below leaves new types beside empty lists
+    x->have_geometry = x->prepared = 0;
     hipError_t ge = geom_run(g, x->stream);
     if (ge != hipSuccess) { dfree(x, dphi); HIPCHK(ge); }
     unsigned int cnt = 0;
@@ -599,6 +600,7 @@ extern "C" int ibtfo_geometry_mask(ibtfo_ctx* x, const unsigned char* rgba, int 
     m.after = (int*)(w + 2 * words);
     m.L = L;
     m.phi = x->phi;
+    x->have_geometry = x->prepared = 0;  // its planes are written from here on
     hipError_t e = scopy(x, (void*)m.rgba, rgba, WH * 4, hipMemcpyHostToDevice);
     if (e == hipSuccess) e = mask_run(m, lds_rows, x->stream);
     if (e != hipSuccess) {

@@ -1,0 +1,265 @@
+// The library's host code (contexts, graphs, tiles, the batch engine) on the CPU:
+// linked with ibtfo_capi.cpp and ibtfo_batch.cpp, this file stands in for the HIP
+// runtime (memory is host memory, a stream runs what it is given at once or, while it
+// captures, records it) and for the kernels (their bookkeeping in the control block,
+// no flow). One check per run, named by the first argument; exit status 0 if it holds.
+#include <cstdarg>
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <functional>
+#include <map>
+#include <string>
+#include <vector>
+
+#include "../../ibtfo_amd/csrc/ibtfo_ctx.h"
+#include "../../ibtfo_amd/csrc/ibtfo_geom.h"
+
+using namespace ibtfo;
+
+// ------------------------------------------------------------------ the runtime
+struct ihipStream_t { bool capturing = false; std::vector<std::function<void()>> ops; };
+struct ihipGraph { std::vector<std::function<void()>> ops; };
+struct hipGraphExec { std::vector<std::function<void()>> ops; };
+struct ihipEvent_t { double at = 0; };
+
+namespace fake {
+long fail_alloc_over = -1;   // allocations of more bytes than this fail (-1: none)
+double clock_ms = 0;         // advanced by the step kernels
+int ghosts = 0;              // ghosts a geometry finds
+int geometries = 0;          // geometry runs
+int launches = 0, wrong_hints = 0;
+double (*step_ms)(const StepArgs&) = nullptr;
+
+void run(hipStream_t s, std::function<void()> f) {
+    if (s->capturing) s->ops.push_back(f);
+    else f();
+}
+}  // namespace fake
+
+extern "C" {
+hipError_t hipMalloc(void** p, size_t n) {
+    if (fake::fail_alloc_over >= 0 && (long)n > fake::fail_alloc_over) return hipErrorOutOfMemory;
+    *p = calloc(1, n + 1);
+    return hipSuccess;
+}
+hipError_t hipFree(void* p) { free(p); return hipSuccess; }
+hipError_t hipHostMalloc(void** p, size_t n, unsigned int) { *p = calloc(1, n + 1); return hipSuccess; }
+hipError_t hipHostFree(void* p) { free(p); return hipSuccess; }
+hipError_t hipMemcpy(void* d, const void* s, size_t n, hipMemcpyKind) { memmove(d, s, n); return hipSuccess; }
+hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind, hipStream_t st) {
+    fake::run(st, [=] { memmove(d, s, n); });
+    return hipSuccess;
+}
+hipError_t hipMemsetAsync(void* d, int v, size_t n, hipStream_t st) {
+    fake::run(st, [=] { memset(d, v, n); });
+    return hipSuccess;
+}
+hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned int) { *s = new ihipStream_t(); return hipSuccess; }
+hipError_t hipStreamDestroy(hipStream_t s) { delete s; return hipSuccess; }
+hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
+hipError_t hipStreamQuery(hipStream_t) { return hipSuccess; }
+hipError_t hipStreamBeginCapture(hipStream_t s, hipStreamCaptureMode) {
+    s->capturing = true;
+    s->ops.clear();
+    return hipSuccess;
+}
+hipError_t hipStreamEndCapture(hipStream_t s, hipGraph_t* g) {
+    s->capturing = false;
+    *g = new ihipGraph{std::move(s->ops)};
+    s->ops.clear();
+    return hipSuccess;
+}
+hipError_t hipGraphInstantiate(hipGraphExec_t* e, hipGraph_t g, hipGraphNode_t*, char*, size_t) {
+    *e = new hipGraphExec{g->ops};
+    return hipSuccess;
+}
+hipError_t hipGraphDestroy(hipGraph_t g) { delete g; return hipSuccess; }
+hipError_t hipGraphExecDestroy(hipGraphExec_t e) { delete e; return hipSuccess; }
+hipError_t hipGraphLaunch(hipGraphExec_t e, hipStream_t) {
+    for (auto& f : e->ops) f();
+    return hipSuccess;
+}
+hipError_t hipEventCreate(hipEvent_t* e) { *e = new ihipEvent_t(); return hipSuccess; }
+hipError_t hipEventDestroy(hipEvent_t e) { delete e; return hipSuccess; }
+hipError_t hipEventRecord(hipEvent_t e, hipStream_t) { e->at = fake::clock_ms; return hipSuccess; }
+hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
+hipError_t hipEventElapsedTime(float* ms, hipEvent_t a, hipEvent_t b) { *ms = (float)(b->at - a->at); return hipSuccess; }
+hipError_t hipGetDevice(int* d) { *d = 0; return hipSuccess; }
+hipError_t hipGetLastError(void) { return hipSuccess; }
+const char* hipGetErrorString(hipError_t) { return "fake"; }
+hipError_t hipFuncSetAttribute(const void*, hipFuncAttribute, int) { return hipSuccess; }
+}
+
+// ------------------------------------------------------------------ the kernels
+static void finish(const FinishArgs& f, int advance) {
+    Ctl* c = f.ctl;
+    if (!c || c->done) return;
+    if (advance == 2) { c->cur ^= 1; return; }
+    c->iter++;
+    c->now_t += c->dt;
+    c->done = !(c->now_t < f.t_end && c->iter < f.max_iter);
+    if (!f.keep_cur) c->cur ^= 1;
+}
+static void step(const StepArgs& a, int stage) {
+    Ctl* c = a.ctl;
+    c->ran = !c->done;
+    if (c->done) return;
+    c->out = c->cur ^ 1 ^ (stage == 3 ? 1 : 0);
+}
+namespace ibtfo {
+hipError_t launch_step(int, int, int, int, const StepArgs& a, hipStream_t s) {
+    fake::run(s, [a] {
+        int cur = a.ctl->cur ^ (a.stage == 3 ? 1 : 0);
+        if (a.df) {  // the head of a deferred-finish batch
+            DfHead h{};
+            if (a.df == 1) { h.iter = a.ctl->iter; h.done = a.ctl->done; h.cur = a.ctl->cur; h.now_t = a.ctl->now_t; }
+            else {
+                h = a.ctl->df[a.df_k ^ 1];
+                if (h.pending) { h.iter++; h.cur ^= 1; h.done = h.iter >= a.max_iter; }
+            }
+            h.pending = !h.done;
+            a.ctl->df[a.df_k] = h;
+            cur = h.cur;
+        } else step(a, a.stage);
+        fake::launches++;
+        fake::wrong_hints += a.in_hint != cur;
+        if (fake::step_ms) fake::clock_ms += fake::step_ms(a);
+    });
+    return hipSuccess;
+}
+hipError_t launch_df_flush(const StepArgs& a, int k, hipStream_t s) {
+    fake::run(s, [a, k] {
+        DfHead h = a.ctl->df[k];
+        a.ctl->ran = h.pending;
+        if (h.pending) { h.iter++; h.cur ^= 1; h.done = h.iter >= a.max_iter; }
+        a.ctl->iter = h.iter; a.ctl->done = h.done; a.ctl->cur = h.cur;
+    });
+    return hipSuccess;
+}
+hipError_t launch_finish(const FinishArgs& f, hipStream_t s) {
+    fake::run(s, [f] { finish(f, f.advance); });
+    return hipSuccess;
+}
+hipError_t launch_post(const FinishArgs& f, const FillArgs*, const EdgeArgs*, hipStream_t s) { return launch_finish(f, s); }
+hipError_t launch_reduce(const ReduceArgs& a, hipStream_t s) {
+    fake::run(s, [a] {
+        a.ctl->dt = 1e-6;
+        if (a.reset) { a.ctl->iter = 0; a.ctl->now_t = 0; a.ctl->done = a.max_iter <= 0; a.ctl->ran = 0; }
+    });
+    return hipSuccess;
+}
+hipError_t launch_uniform_state(double*, double*, double*, long long, const double*, Ctl* c, hipStream_t s) {
+    fake::run(s, [c] { c->cur = 0; c->ran = 0; });
+    return hipSuccess;
+}
+hipError_t launch_fill(const FillArgs&, hipStream_t) { return hipSuccess; }
+hipError_t launch_scatter(const FillArgs&, hipStream_t) { return hipSuccess; }
+hipError_t launch_edge(const EdgeArgs&, hipStream_t) { return hipSuccess; }
+hipError_t launch_edge_ref(const EdgeArgs&, const double*, int, hipStream_t) { return hipSuccess; }
+hipError_t launch_merge(const MergeArgs&, hipStream_t) { return hipSuccess; }
+// the batch's kernels over its slots (the tables are sized by the finish table's end)
+static int batch_slots = 0;
+hipError_t launch_step_batch(int, int, int, int, const StepArgs* t, const int2* map, int n, int stage, hipStream_t s) {
+    fake::run(s, [=] {
+        for (int b = 0; b < n; b++)
+            if (map[b].x >= 0 && map[b].y == 0) step(t[map[b].x], stage);
+    });
+    return hipSuccess;
+}
+hipError_t launch_post_batch(const FinishArgs* f, int ns, int advance, const FillArgs*, const int2*, int, const EdgeArgs*,
+                             const int2*, int, hipStream_t s) {
+    batch_slots = ns;
+    fake::run(s, [=] {
+        for (int q = 0; q < ns; q++)
+            if (f[q].ctl) finish(f[q], advance);
+    });
+    return hipSuccess;
+}
+hipError_t launch_gather(const FinishArgs* f, int ns, SlotStatus* out, hipStream_t s) {
+    fake::run(s, [=] {
+        for (int q = 0; q < ns; q++) {
+            SlotStatus st{};
+            if (const Ctl* c = f[q].ctl) { st.iter = c->iter; st.done = c->done; st.now_t = c->now_t; st.dt = c->dt; }
+            out[q] = st;
+        }
+    });
+    return hipSuccess;
+}
+hipError_t launch_persist(int, int, int, int, const PersistArgs&, int, hipStream_t) { return hipErrorInvalidValue; }
+int persist_blocks(int, int, int, int) { return 0; }
+hipError_t geom_run(GeomArgs& g, hipStream_t) {
+    fake::geometries++;
+    memset(g.type, 0, g.L.plane);
+    return hipSuccess;
+}
+hipError_t geom_ghosts(GeomArgs& g, hipStream_t) { *g.count = (unsigned)fake::ghosts; return hipSuccess; }
+hipError_t cut_run(GeomArgs&, hipStream_t) { return hipSuccess; }
+hipError_t cut_records(GeomArgs&, hipStream_t) { return hipSuccess; }
+hipError_t mask_run(MaskArgs&, bool, hipStream_t) { return hipSuccess; }
+const void* mask_rows_kernel() { return nullptr; }
+int png_read_file(const char*, std::vector<unsigned char>&, int*, int*) { return IBTFO_E_IO; }
+int write_vtk(const ::ibtfo_config*, int, double, const double*, const double*, const char*) { return IBTFO_E_IO; }
+int host_initialize(int, const double*, int, int, int, int, double, const double*, const double*, const unsigned char*,
+                    double*) { return IBTFO_E_ARG; }
+}  // namespace ibtfo
+
+// ------------------------------------------------------------------ the checks
+static int failures = 0;
+#define CHECK(c) do { if (!(c)) { failures++; printf("%s:%d: %s\n", __FILE__, __LINE__, #c); } } while (0)
+
+static ibtfo_config config(int nx, int ny, int boundary, int edge) {
+    ibtfo_config c;
+    memset(&c, 0, sizeof c);
+    c.N_x = nx; c.N_y = ny; c.num_ghost_cell = 2;
+    c.hi_x = 1.0; c.hi_y = (double)ny / nx;
+    c.Psy_time = 1e30; c.max_iter = 1 << 30;
+    c.CFL_number = 0.5; c.gamma = 1.4;
+    c.scheme = IBTFO_MUSCL; c.riemann = IBTFO_HLL; c.limiter = IBTFO_MINMOD;
+    c.boundary = boundary; c.time = IBTFO_SINGLESTEP; c.edge = edge; c.precision = IBTFO_FP64;
+    const double flow[4] = {1.4, 3.0, 0.0, 1.0};
+    memcpy(c.edge_state, flow, sizeof flow);
+    return c;
+}
+static const double UNIFORM[4] = {1.4, 3.0, 0.0, 1.0};
+static ibtfo_ctx* solve(const ibtfo_config& c) {
+    ibtfo_ctx* x = nullptr;
+    CHECK(ibtfo_create(&c, &x) == IBTFO_OK);
+    CHECK(ibtfo_geometry(x, IBTFO_LS_NONE, nullptr, 0, nullptr) == IBTFO_OK);
+    CHECK(ibtfo_initialize(x, IBTFO_INIT_UNIFORM, UNIFORM, 4) == IBTFO_OK);
+    CHECK(ibtfo_prepare(x, 1) == IBTFO_OK);
+    return x;
+}
+
+// A geometry that fails after its types were written leaves a solve without one:
+// nothing runs on the new types with an empty ghost list.
+static void geometry_failure() {
+    fake::ghosts = 0;
+    ibtfo_ctx* x = solve(config(96, 64, IBTFO_IDW_GFM, IBTFO_EDGE_INFLOW));
+    fake::ghosts = 5000;
+    fake::fail_alloc_over = 1000;
+    CHECK(ibtfo_geometry(x, IBTFO_LS_NONE, nullptr, 0, nullptr) == IBTFO_E_NOMEM);
+    fake::fail_alloc_over = -1;
+    double v;
+    CHECK(ibtfo_prepare(x, 1) == IBTFO_E_STATE);
+    CHECK(ibtfo_boundary(x) == IBTFO_E_STATE);
+    CHECK(ibtfo_compute_dt(x, &v) == IBTFO_E_STATE);
+    CHECK(ibtfo_step(x, 1) == IBTFO_E_STATE);
+    CHECK(ibtfo_geometry(x, IBTFO_LS_NONE, nullptr, 0, nullptr) == IBTFO_OK);
+    CHECK(ibtfo_num_ghosts(x) == 5000);
+    CHECK(ibtfo_prepare(x, 1) == IBTFO_OK);
+    CHECK(ibtfo_step(x, 1) == IBTFO_OK);
+    ibtfo_destroy(x);
+}
+
+int main(int argc, char** argv) {
+    const std::map<std::string, void (*)()> checks = {{"geometry_failure", geometry_failure}};
+    const auto it = argc > 1 ? checks.find(argv[1]) : checks.end();
+    if (it == checks.end()) {
+        for (auto& c : checks) printf("%s\n", c.first.c_str());
+        return 2;
+    }
+    it->second();
+    printf("%s: %s\n", argv[1], failures ? "FAILED" : "ok");
+    return failures ? 1 : 0;
+}
