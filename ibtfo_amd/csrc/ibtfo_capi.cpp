@@ -577,11 +577,12 @@ extern "C" int ibtfo_geometry_mask(ibtfo_ctx* x, const unsigned char* rgba, int 
     const size_t WH = (size_t)width * height;
     m.nseg = (height + MASK_SEG - 1) / MASK_SEG;
     const size_t SW = (size_t)m.nseg * width;
-    // the row search stages its columns in LDS up to its limit
-    const size_t lds_bytes = mask_lds_bytes(width, L.M);
-    const bool lds_rows = lds_bytes <= MASK_LDS_MAX &&
+    // The row search stages its columns in LDS up to its limit. The kernel's attribute
+    // belongs to the process: one value for every mask, so that a thread with a narrow
+    // one does not lower it between another's call and its launch.
+    const bool lds_rows = mask_lds_bytes(width, L.M) <= MASK_LDS_MAX &&
                           hipFuncSetAttribute(mask_rows_kernel(), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                              (int)lds_bytes) == hipSuccess;
+                                              (int)MASK_LDS_MAX) == hipSuccess;
     // The image and its bit words are read before geom_run writes the normals, whose
     // planes they take where they fit (a pixel per cell and more do: two doubles)
     const size_t rgba_bytes = (size_t)round_up(WH * 4, 256), words = (size_t)round_up(SW * 4, 256);

@@ -29,6 +29,8 @@ double clock_ms = 0;         // advanced by the step kernels
 int ghosts = 0;              // ghosts a geometry finds
 int geometries = 0;          // geometry runs
 int launches = 0, wrong_hints = 0;
+int lds_limit = 0, lds_refused = 0;  // the mask kernel's LDS attribute; launches above it
+std::function<void()> after_attribute;
 double (*step_ms)(const StepArgs&) = nullptr;
 
 void run(hipStream_t s, std::function<void()> f) {
@@ -88,7 +90,13 @@ hipError_t hipEventElapsedTime(float* ms, hipEvent_t a, hipEvent_t b) { *ms = (f
 hipError_t hipGetDevice(int* d) { *d = 0; return hipSuccess; }
 hipError_t hipGetLastError(void) { return hipSuccess; }
 const char* hipGetErrorString(hipError_t) { return "fake"; }
-hipError_t hipFuncSetAttribute(const void*, hipFuncAttribute, int) { return hipSuccess; }
+hipError_t hipFuncSetAttribute(const void*, hipFuncAttribute, int v) {
+    fake::lds_limit = v;
+    auto f = std::move(fake::after_attribute);
+    fake::after_attribute = nullptr;
+    if (f) f();
+    return hipSuccess;
+}
 }
 
 // ------------------------------------------------------------------ the kernels
@@ -196,7 +204,10 @@ hipError_t geom_run(GeomArgs& g, hipStream_t) {
 hipError_t geom_ghosts(GeomArgs& g, hipStream_t) { *g.count = (unsigned)fake::ghosts; return hipSuccess; }
 hipError_t cut_run(GeomArgs&, hipStream_t) { return hipSuccess; }
 hipError_t cut_records(GeomArgs&, hipStream_t) { return hipSuccess; }
-hipError_t mask_run(MaskArgs&, bool, hipStream_t) { return hipSuccess; }
+hipError_t mask_run(MaskArgs& m, bool lds, hipStream_t) {
+    if (lds && (int)mask_lds_bytes(m.W, m.M) > fake::lds_limit) fake::lds_refused++;
+    return hipSuccess;
+}
 const void* mask_rows_kernel() { return nullptr; }
 int png_read_file(const char*, std::vector<unsigned char>&, int*, int*) { return IBTFO_E_IO; }
 int write_vtk(const ::ibtfo_config*, int, double, const double*, const double*, const char*) { return IBTFO_E_IO; }
@@ -252,8 +263,22 @@ static void geometry_failure() {
     ibtfo_destroy(x);
 }
 
+// Two threads with masks of different widths: the narrow one's call falls between the
+// wide one's attribute and its launch.
+static void mask_attribute() {
+    ibtfo_ctx* a = solve(config(64, 32, IBTFO_IDW_GFM, IBTFO_EDGE_INFLOW));
+    ibtfo_ctx* b = solve(config(64, 32, IBTFO_IDW_GFM, IBTFO_EDGE_INFLOW));
+    const std::vector<unsigned char> wide(4 * 6000 * 8, 255), narrow(4 * 8 * 8, 255);
+    fake::after_attribute = [&] { CHECK(ibtfo_geometry_mask(b, narrow.data(), 8, 8) == IBTFO_OK); };
+    CHECK(ibtfo_geometry_mask(a, wide.data(), 6000, 8) == IBTFO_OK);
+    CHECK(fake::lds_limit > 0 && fake::lds_refused == 0);
+    ibtfo_destroy(a);
+    ibtfo_destroy(b);
+}
+
 int main(int argc, char** argv) {
-    const std::map<std::string, void (*)()> checks = {{"geometry_failure", geometry_failure}};
+    const std::map<std::string, void (*)()> checks = {{"geometry_failure", geometry_failure},
+                                                         {"mask_attribute", mask_attribute}};
     const auto it = argc > 1 ? checks.find(argv[1]) : checks.end();
     if (it == checks.end()) {
         for (auto& c : checks) printf("%s\n", c.first.c_str());
