@@ -48,8 +48,8 @@ struct ibtfo_ctx {
     uint8_t* stype;       // the cut-cell step kernel's type plane: type | MERGED_BIT for group cells
     double* merge_part;   // PART_STRIDE doubles per merge block
     double* df_part;      // deferred finish: 2 x DF_MAX_REC partial records (single solves only)
-    hipGraphExec_t graph;
-    int graph_chunk;
+    hipGraphExec_t graph[2];  // graph_chunk steps that start from state[0] / state[1]
+    int graph_chunk;          // 0: none captured
     std::vector<double> corner_host;
     ibtfo::Arena* arena;  // device memory from a batch engine's arena (else hipMalloc)
     // Device memory behind the pointers above: what a context always holds (slab; one

@@ -238,7 +238,7 @@ __device__ __forceinline__ void step_rowpar(const StepArgs& a, const int bx, con
     // together with the control block from the buffer the host expects to be the
     // input (StepArgs::in_hint), so that no load waits for another: on a
     // latency-bound small grid that is one memory round trip less. Another buffer
-    // (a graph of an odd number of steps replayed) is read again below.
+    // (steps that the host does not see: a caller's own graph replayed) is read again below.
     // Every load at the head of the kernel is unconditional (the waves past a short
     // last strip read the top row's), so that none waits in a branch.
     double wm[4], w0[4], w1[4], w2[4] = {0.0, 0.0, 0.0, 0.0};

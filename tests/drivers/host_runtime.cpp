@@ -276,9 +276,36 @@ static void mask_attribute() {
     ibtfo_destroy(b);
 }
 
+// Replays after an odd number of single steps, and replays of an odd number of steps:
+// every step kernel is told the buffer that it then finds current.
+static void graph_start() {
+    for (int nx : {96, 1200})  // one kernel per step; a finish kernel between
+        for (int time : {IBTFO_SINGLESTEP, IBTFO_RK2}) {
+            ibtfo_config c = config(nx, nx / 2, IBTFO_REGULAR, IBTFO_EDGE_REFERENCE);
+            c.time = time;
+            ibtfo_ctx* x = solve(c);
+            fake::launches = fake::wrong_hints = 0;
+            CHECK(ibtfo_step_graph(x, 0, 50) == IBTFO_OK && fake::launches == 0);
+            int steps = 0;
+            for (int n : {75, 75, 50, 1, 100, 125}) {
+                CHECK(ibtfo_step_graph(x, n, 50) == IBTFO_OK);
+                steps += n;
+            }
+            for (int n : {28, 7, 1, 70}) {
+                CHECK(ibtfo_step_graph(x, n, 7) == IBTFO_OK);
+                steps += n;
+            }
+            int it = 0;
+            CHECK(ibtfo_status(x, &it, nullptr, nullptr) == IBTFO_OK && it == steps);
+            CHECK(fake::launches == steps * (time == IBTFO_RK2 ? 2 : 1) && fake::wrong_hints == 0);
+            ibtfo_destroy(x);
+        }
+}
+
 int main(int argc, char** argv) {
     const std::map<std::string, void (*)()> checks = {{"geometry_failure", geometry_failure},
-                                                         {"mask_attribute", mask_attribute}};
+                                                         {"mask_attribute", mask_attribute},
+                                                         {"graph_start", graph_start}};
     const auto it = argc > 1 ? checks.find(argv[1]) : checks.end();
     if (it == checks.end()) {
         for (auto& c : checks) printf("%s\n", c.first.c_str());
