@@ -1289,6 +1289,7 @@ extern "C" int ibtfo_autotune(ibtfo_ctx* x, int probe_steps, int* best_rows, dou
         HIPCHK(hipMemcpyAsync(save ? ct : (char*)x->ctl, save ? (char*)x->ctl : ct, sizeof(Ctl),
                               hipMemcpyDeviceToDevice, x->stream));
         HIPCHK(hipStreamSynchronize(x->stream));
+        x->cur_guess = head.cur;
         return IBTFO_OK;
     };
     const int keep = x->rows_override, keep_par = x->rowpar;

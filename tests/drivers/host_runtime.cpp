@@ -302,10 +302,29 @@ static void graph_start() {
         }
 }
 
+// The autotuner's probes and the steps after it, for an even and an odd probe: the state
+// put back is the one that the next probe is told.
+static double every_step_alike(const StepArgs&) { return 1.0; }
+static void autotune_start() {
+    fake::step_ms = every_step_alike;
+    for (int probe : {3, 4}) {
+        ibtfo_ctx* x = solve(config(1200, 600, IBTFO_IDW_GFM, IBTFO_EDGE_INFLOW));
+        CHECK(ibtfo_step(x, 5) == IBTFO_OK);
+        fake::launches = fake::wrong_hints = 0;
+        CHECK(ibtfo_autotune(x, probe, nullptr, nullptr) == IBTFO_OK);
+        CHECK(ibtfo_step(x, 4) == IBTFO_OK);
+        CHECK(fake::launches > 20 * probe && fake::wrong_hints == 0);
+        int it = 0;
+        CHECK(ibtfo_status(x, &it, nullptr, nullptr) == IBTFO_OK && it == 9);
+        ibtfo_destroy(x);
+    }
+}
+
 int main(int argc, char** argv) {
     const std::map<std::string, void (*)()> checks = {{"geometry_failure", geometry_failure},
                                                          {"mask_attribute", mask_attribute},
-                                                         {"graph_start", graph_start}};
+                                                         {"graph_start", graph_start},
+                                                         {"autotune_start", autotune_start}};
     const auto it = argc > 1 ? checks.find(argv[1]) : checks.end();
     if (it == checks.end()) {
         for (auto& c : checks) printf("%s\n", c.first.c_str());
