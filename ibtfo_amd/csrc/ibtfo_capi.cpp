@@ -1301,6 +1301,15 @@ extern "C" int ibtfo_autotune(ibtfo_ctx* x, int probe_steps, int* best_rows, dou
     for (int r : {1, 2, 3, 4, 6, 8, 12, 16, 24, 32, 48, 64, 96, 128, 192, 256}) cand.push_back({r, 0});
     if (x->cfg.scheme != IBTFO_LAX)
         for (int r = 1; r <= ROWPAR_MAX_ROWS; r++) cand.push_back({r, 1});
+    // and the default tile and the one in force (10 rows at 4096x2048 is not in the
+    // list), so that tuning never leaves a slower one
+    Cand own[2] = {{0, 0}, {keep, keep_par}};
+    default_tile(x->cfg, L, &own[0].rows, &own[0].par);
+    for (Cand& o : own) {
+        o.rows = std::min(o.rows, L.ny);
+        if (std::none_of(cand.begin(), cand.end(), [&](const Cand& c) { return c.rows == o.rows && c.par == o.par; }))
+            cand.push_back(o);
+    }
     int best = 0, best_par = 0;
     double bms = 1e300;
     hipEvent_t e0 = nullptr, e1 = nullptr;

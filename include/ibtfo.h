@@ -244,8 +244,8 @@ int ibtfo_tile_ex(const ibtfo_ctx* ctx, int* rows, int* nbx, int* nby, int* row_
 int ibtfo_one_kernel_steps(const ibtfo_ctx* ctx);
 /* Tile-shape autotuner: times `probe_steps` steps of the current solve for each
  * candidate shape (marching strips of 1 .. 256 rows, row-parallel strips of 1 ..
- * 7 rows), restoring the state and clock after each probe, and keeps the
- * fastest (ibtfo_tile_ex reports its form). Allocates a temporary snapshot of
+ * 7 rows, the default tile and the current one), restoring the state and clock
+ * after each probe, and keeps the fastest (ibtfo_tile_ex reports its form). Allocates a temporary snapshot of
  * both state buffers. Fails with IBTFO_E_STATE when the run would end within a
  * probe. */
 int ibtfo_autotune(ibtfo_ctx* ctx, int probe_steps, int* best_rows, double* best_ms_per_step);

@@ -320,11 +320,32 @@ static void autotune_start() {
     }
 }
 
+// The autotuner keeps a tile that is faster than every shape of its list, where that is
+// the default tile (10 rows) or the one in force.
+static int best_rows = 0;
+static double one_tile_best(const StepArgs& a) { return a.rows == best_rows && !a.rowpar ? 1.0 : 2.0; }
+static void autotune_own_tile() {
+    fake::step_ms = one_tile_best;
+    for (int in_force : {0, 11}) {
+        ibtfo_ctx* x = solve(config(4096, 2048, IBTFO_REGULAR, IBTFO_EDGE_REFERENCE));
+        int rows = 0, par = 1;
+        CHECK(ibtfo_set_rows(x, in_force) == IBTFO_OK && ibtfo_tile(x, &best_rows, nullptr, nullptr) == IBTFO_OK);
+        CHECK(best_rows == (in_force ? in_force : 10));
+        for (int again = 0; again < 2; again++) {
+            CHECK(ibtfo_autotune(x, 2, &rows, nullptr) == IBTFO_OK && rows == best_rows);
+            CHECK(ibtfo_tile_ex(x, &rows, nullptr, nullptr, &par) == IBTFO_OK && rows == best_rows && !par);
+            if (!in_force) CHECK(ibtfo_set_rows(x, 48) == IBTFO_OK);  // the default, found from another tile
+        }
+        ibtfo_destroy(x);
+    }
+}
+
 int main(int argc, char** argv) {
     const std::map<std::string, void (*)()> checks = {{"geometry_failure", geometry_failure},
                                                          {"mask_attribute", mask_attribute},
                                                          {"graph_start", graph_start},
-                                                         {"autotune_start", autotune_start}};
+                                                         {"autotune_start", autotune_start},
+                                                         {"autotune_own_tile", autotune_own_tile}};
     const auto it = argc > 1 ? checks.find(argv[1]) : checks.end();
     if (it == checks.end()) {
         for (auto& c : checks) printf("%s\n", c.first.c_str());
