@@ -171,16 +171,19 @@ static int cfg_step_blocks(const ibtfo_config& c, int rows) {
     const int r = std::max(1, std::min(rows, c.N_y));
     return nbx * ((c.N_y + r - 1) / r);
 }
-// Strip height of a request in a batch whose configuration leaves it open: 8 rows,
-// or 16 where the step blocks are short: the request would not fit, or the batch
-// holds less than two rounds of the chip's 4096 waves (256 CUs, 16 waves each), so
+// Strip height of a request in a batch whose configuration leaves it open (rows = 0):
+// 8 rows, or 16 where the step blocks are short: the request would not fit, or the batch
+// holds less than three rounds of the chip's 4096 waves (256 CUs, 16 waves each), so
 // that taller strips let more solves in. 24 solves of 64x64 to 1024x512 in mixed
 // precision, 3.8 M cells: 93 us per step with 16 rows (3900 waves, one round that
-// lasts as long as a strip), 84 with 8, 86 with 6, 89 with 4.
+// lasts as long as a strip), 84 with 8, 86 with 6, 89 with 4. A stream that keeps the
+// blocks taken, 256 solves x 100 steps, ms with 16 rows / 8: 8192 blocks mixed 78.4 /
+// 83.3, FP64 100.1 / 105.2; 12288 blocks 78.4 / 77.3 and 98.6 / 95.7; 16384 blocks 78.8 /
+// 79.0 and 99.1 / 95.7.
 constexpr int BATCH_WAVES = 4096;
 static int batch_rows(const ibtfo_batch_config& k, const ibtfo_config& c) {
     if (k.rows > 0) return k.rows;
-    return k.max_step_blocks >= 2 * BATCH_WAVES && cfg_step_blocks(c, 8) <= k.max_step_blocks ? 8 : 16;
+    return k.max_step_blocks >= 3 * BATCH_WAVES && cfg_step_blocks(c, 8) <= k.max_step_blocks ? 8 : 16;
 }
 static int cfg_ring_blocks(const ibtfo_config& c) {
     if (c.edge == IBTFO_EDGE_REFERENCE) return 0;

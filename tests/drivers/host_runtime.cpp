@@ -29,6 +29,7 @@ double clock_ms = 0;         // advanced by the step kernels
 int ghosts = 0;              // ghosts a geometry finds
 int geometries = 0;          // geometry runs
 int launches = 0, wrong_hints = 0;
+int batch_rows = 0;          // strip height of the batch's last solve stepped
 int lds_limit = 0, lds_refused = 0;  // the mask kernel's LDS attribute; launches above it
 std::function<void()> after_attribute;
 double (*step_ms)(const StepArgs&) = nullptr;
@@ -167,18 +168,19 @@ hipError_t launch_scatter(const FillArgs&, hipStream_t) { return hipSuccess; }
 hipError_t launch_edge(const EdgeArgs&, hipStream_t) { return hipSuccess; }
 hipError_t launch_edge_ref(const EdgeArgs&, const double*, int, hipStream_t) { return hipSuccess; }
 hipError_t launch_merge(const MergeArgs&, hipStream_t) { return hipSuccess; }
-// the batch's kernels over its slots (the tables are sized by the finish table's end)
-static int batch_slots = 0;
+// the batch's kernels over its slots
 hipError_t launch_step_batch(int, int, int, int, const StepArgs* t, const int2* map, int n, int stage, hipStream_t s) {
     fake::run(s, [=] {
         for (int b = 0; b < n; b++)
-            if (map[b].x >= 0 && map[b].y == 0) step(t[map[b].x], stage);
+            if (map[b].x >= 0 && map[b].y == 0) {
+                step(t[map[b].x], stage);
+                fake::batch_rows = t[map[b].x].rows;
+            }
     });
     return hipSuccess;
 }
 hipError_t launch_post_batch(const FinishArgs* f, int ns, int advance, const FillArgs*, const int2*, int, const EdgeArgs*,
                              const int2*, int, hipStream_t s) {
-    batch_slots = ns;
     fake::run(s, [=] {
         for (int q = 0; q < ns; q++)
             if (f[q].ctl) finish(f[q], advance);
@@ -341,12 +343,58 @@ static void autotune_own_tile() {
     }
 }
 
+static ibtfo_batch_config batch_config(int rows, int blocks, int slots) {
+    ibtfo_batch_config k;
+    ibtfo_batch_config_default(&k);
+    k.boundary = IBTFO_IDW_GFM;
+    k.quirks = 0;
+    k.hbm_budget = 1ll << 30;
+    k.max_slots = slots;
+    k.max_step_blocks = blocks;
+    k.max_ghost_blocks = k.max_ring_blocks = 4096;
+    k.rows = rows;
+    k.chunk = 4;
+    return k;
+}
+static int submit(ibtfo_batch* b, int nx, int ny, int steps) {
+    ibtfo_request r;
+    memset(&r, 0, sizeof r);
+    r.cfg = config(nx, ny, IBTFO_IDW_GFM, IBTFO_EDGE_INFLOW);
+    r.cfg.max_iter = steps;
+    r.ls_kind = IBTFO_LS_NONE;
+    r.init_kind = IBTFO_INIT_UNIFORM;
+    r.init_nprm = 4;
+    r.init_prm = UNIFORM;
+    r.arrival = -1;
+    return ibtfo_batch_submit(b, &r, nullptr);
+}
+static int drain(ibtfo_batch* b) {
+    int active = 1, queued = 1, finished = 0;
+    for (int k = 0; k < 1000 && (active || queued); k++) CHECK(ibtfo_batch_progress(b, &active, &queued, &finished) == IBTFO_OK);
+    return finished;
+}
+
+// rows = 0: 8-row strips from three rounds of the chip's waves on, where the solve fits.
+static void batch_open_rows() {
+    struct { int rows, blocks, want; } cases[] = {{0, 8192, 16}, {0, 12287, 16}, {0, 12288, 8}, {0, 65536, 8}, {4, 8192, 4},
+                                                  {16, 65536, 16}};
+    for (auto& c : cases) {
+        ibtfo_batch_config k = batch_config(c.rows, c.blocks, 4);
+        ibtfo_batch* b = nullptr;
+        CHECK(ibtfo_batch_create(&k, &b) == IBTFO_OK);
+        CHECK(submit(b, 128, 64, 6) == IBTFO_OK);
+        CHECK(drain(b) == 1 && fake::batch_rows == c.want);
+        ibtfo_batch_destroy(b);
+    }
+}
+
 int main(int argc, char** argv) {
     const std::map<std::string, void (*)()> checks = {{"geometry_failure", geometry_failure},
                                                          {"mask_attribute", mask_attribute},
                                                          {"graph_start", graph_start},
                                                          {"autotune_start", autotune_start},
-                                                         {"autotune_own_tile", autotune_own_tile}};
+                                                         {"autotune_own_tile", autotune_own_tile},
+                                                         {"batch_open_rows", batch_open_rows}};
     const auto it = argc > 1 ? checks.find(argv[1]) : checks.end();
     if (it == checks.end()) {
         for (auto& c : checks) printf("%s\n", c.first.c_str());
