@@ -352,8 +352,15 @@ static void retire_head(ibtfo_batch* b, int rc) {
 // request error (the request is then retired with that status).
 static int admit_one(ibtfo_batch* b, int reserved_step, int reserved_ghost, int reserved_ring) {
     Req& q = b->queue.front();
+    const int rows = batch_rows(b->bc, q.cfg);
+    // strips and ring cells are known from the grid: a request that waits for them costs
+    // nothing per call (its context and geometry used to be built and freed each time)
+    if (q.cfg.N_x > 0 && q.cfg.N_y > 0 &&
+        (b->used_step + reserved_step + cfg_step_blocks(q.cfg, rows) > b->bc.max_step_blocks ||
+         b->used_ring + reserved_ring + cfg_ring_blocks(q.cfg) > b->bc.max_ring_blocks))
+        return 0;
     ibtfo_ctx* x = nullptr;
-    int rc = ctx_create(&q.cfg, &b->arena, b->adm, batch_rows(b->bc, q.cfg), &x);
+    int rc = ctx_create(&q.cfg, &b->arena, b->adm, rows, &x);
     if (rc == IBTFO_E_NOMEM) return 0;
     if (rc == IBTFO_OK)
         rc = ibtfo_geometry(x, q.ls_kind, q.ls_prm.empty() ? nullptr : q.ls_prm.data(), (int)q.ls_prm.size(),

@@ -388,13 +388,44 @@ static void batch_open_rows() {
     }
 }
 
+// Requests that wait for step blocks (96x64: 2 strips x 4) or ring blocks (1312 cells: 3)
+// are built once each, in the order of their arrival.
+static void batch_waiting() {
+    for (int ring : {0, 1}) {
+        ibtfo_batch_config k = batch_config(16, ring ? 4096 : 20, 8);
+        if (ring) k.max_ring_blocks = 7;
+        ibtfo_batch* b = nullptr;
+        CHECK(ibtfo_batch_create(&k, &b) == IBTFO_OK);
+        fake::geometries = 0;
+        for (int q = 0; q < 5; q++) CHECK(submit(b, 96, 64, 40 + q) == IBTFO_OK);
+        int active = 0, queued = 0;
+        CHECK(ibtfo_batch_progress(b, &active, &queued, nullptr) == IBTFO_OK && active == 2 && queued == 3);
+        CHECK(ibtfo_batch_progress(b, &active, &queued, nullptr) == IBTFO_OK && active == 2 && queued == 3);
+        CHECK(fake::geometries == 2);
+        CHECK(drain(b) == 5 && fake::geometries == 5);
+        long long t = 0, last = 0;
+        while (ibtfo_batch_poll(b, &t) == 1) {
+            ibtfo_result r;
+            CHECK(ibtfo_batch_result(b, t, &r, nullptr) == IBTFO_OK && r.status == IBTFO_OK && r.iter == 39 + t && t > last);
+            last = t;
+        }
+        CHECK(last == 5);
+        // a grid that no context takes is still retired with its error
+        CHECK(submit(b, 3, 64, 4) == IBTFO_OK && drain(b) == 6);
+        ibtfo_result r;
+        CHECK(ibtfo_batch_poll(b, &t) == 1 && ibtfo_batch_result(b, t, &r, nullptr) == IBTFO_OK && r.status == IBTFO_E_ARG);
+        ibtfo_batch_destroy(b);
+    }
+}
+
 int main(int argc, char** argv) {
     const std::map<std::string, void (*)()> checks = {{"geometry_failure", geometry_failure},
                                                          {"mask_attribute", mask_attribute},
                                                          {"graph_start", graph_start},
                                                          {"autotune_start", autotune_start},
                                                          {"autotune_own_tile", autotune_own_tile},
-                                                         {"batch_open_rows", batch_open_rows}};
+                                                         {"batch_open_rows", batch_open_rows},
+                                                         {"batch_waiting", batch_waiting}};
     const auto it = argc > 1 ? checks.find(argv[1]) : checks.end();
     if (it == checks.end()) {
         for (auto& c : checks) printf("%s\n", c.first.c_str());
