@@ -256,6 +256,16 @@ struct PersistArgs {
     long long spin_limit;
 };
 
+// Blocks (one wave each) per CU of the persistent launch, of the `fit` that its kernel's
+// registers allow: one per SIMD. Every block has to be resident, or the barrier times
+// out. A wave's registers are contiguous, and an admission kernel's waves that lie
+// between the launch's own while it is dispatched can leave gaps none of which takes one
+// more wave, even after they end: of 512 registers, three waves of 168, two of 176 or
+// three of 128 may find no room, one always does. More blocks also cost time, the
+// barriers': two waves per SIMD in place of one, MUSCL HLL mixed, 6 solves x 200 steps
+// 165 ms / 92, 24 x 100 176 / 102, 256 x 50 428 / 245.
+inline int persist_per_cu(int fit) { return fit > 4 ? 4 : fit; }
+
 // per-slot status record of the batch engine (k_gather)
 struct SlotStatus {
     int iter, done, status, pad;

@@ -1162,13 +1162,7 @@ int persist_blocks(int scheme, int rs, int lim, int prec) {
         hipGetDevice(&dev) != hipSuccess ||
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
         return 0;
-    // One wave per SIMD fewer than fits: a wave's registers are contiguous, and with
-    // three waves of 168 in 512 an admission kernel's wave that lies between two of
-    // them while the launch is being dispatched leaves no room for the third even
-    // after it ends, so that block would never start and the barrier would time out.
-    // With two, the larger gap beside the first always holds the second. (Fewer
-    // blocks are no loss here: the barriers, whose cost grows with them, set the time.)
-    return (per_cu > 4 ? per_cu - 4 : 1) * cus;
+    return persist_per_cu(per_cu) * cus;
 }
 hipError_t launch_persist(int scheme, int rs, int lim, int prec, const PersistArgs& p, int blocks, hipStream_t s) {
     if (scheme == SCH_LAX || blocks <= 0) return hipErrorInvalidValue;

@@ -418,6 +418,18 @@ static void batch_waiting() {
     }
 }
 
+// The persistent kernel's waves on a SIMD, for every register count (of 512, by eights):
+// however the first of them lie, among other waves that end later, the next has room.
+static bool stuck(int free, int gaps, int size) { return free <= gaps * (size - 1); }
+static void persistent_grid() {
+    for (int size = 1; size <= 64; size++) {
+        const int fit = std::min(64 / size, 8), waves = persist_per_cu(4 * fit) / 4;
+        CHECK(waves >= 1 && waves <= fit);
+        for (int placed = 0; placed < waves; placed++) CHECK(!stuck(64 - placed * size, placed + 1, size));
+    }
+    CHECK(persist_per_cu(3) == 3 && persist_per_cu(1) == 1);  // kernels that other limits hold below one per SIMD
+}
+
 int main(int argc, char** argv) {
     const std::map<std::string, void (*)()> checks = {{"geometry_failure", geometry_failure},
                                                          {"mask_attribute", mask_attribute},
@@ -425,7 +437,8 @@ int main(int argc, char** argv) {
                                                          {"autotune_start", autotune_start},
                                                          {"autotune_own_tile", autotune_own_tile},
                                                          {"batch_open_rows", batch_open_rows},
-                                                         {"batch_waiting", batch_waiting}};
+                                                         {"batch_waiting", batch_waiting},
+                                                         {"persistent_grid", persistent_grid}};
     const auto it = argc > 1 ? checks.find(argv[1]) : checks.end();
     if (it == checks.end()) {
         for (auto& c : checks) printf("%s\n", c.first.c_str());

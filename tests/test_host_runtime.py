@@ -11,7 +11,7 @@ ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 HIP = os.environ.get("ROCM_PATH", "/opt/rocm")
 
 CHECKS = ["geometry_failure", "mask_attribute", "graph_start", "autotune_start", "autotune_own_tile",
-          "batch_open_rows", "batch_waiting"]
+          "batch_open_rows", "batch_waiting", "persistent_grid"]
 
 
 @pytest.fixture(scope="module")
