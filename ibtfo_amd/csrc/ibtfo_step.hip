@@ -356,13 +356,14 @@ __device__ __forceinline__ void step_strip(const StepArgs& a, const int bx, cons
             for (int k = 0; k < 4; k++) nw[k] = ld(Ui, j + 3, k);
             tn = *(a.type + L.at(0, j + 1) + ct);
         }
-        // FP64: row j's cells and x fluxes stay in LDS (rb, fb) and are read back
-        // where they are used, so that no register holds them through the y face.
+        // Row j's cells (and in FP64 its x fluxes) stay in LDS (rb, fb) and are read back
+        // where they are used, so that no register holds them through the y face. In mixed
+        // precision the cells in registers cost the MUSCL forms 8 to 32 bytes of scratch.
 #pragma unroll
         for (int k = 0; k < 4; k++) rb[k][lane] = w[0][k];
         __syncthreads();
         T F[4] = {0, 0, 0, 0};
-        auto cell = [&](int k) { return FP64 ? rb[k][lane] : w[0][k]; };
+        auto cell = [&](int k) { return rb[k][lane]; };
         auto flux = [&](int k) { return FP64 ? fb[k][lane] : F[k]; };
         // x faces of row j; the first iteration (j = j0-1) only needs the y face
         // below row j0, unless that face may take the aliased x flux
@@ -526,13 +527,20 @@ __device__ __forceinline__ void step_strip(const StepArgs& a, const int bx, cons
 // LDS exchanges need them (4096x2048 cut cells, HLL: 245 us at three waves, 226 at
 // four; Steger-Warming, 132 VGPRs unbounded: 325 us, 302 us with 12 bytes spilled).
 // PVRS, whose pow() calls need far more registers, is left to the compiler.
-constexpr int step_waves(int rs) { return rs == RS_PVRS ? 1 : 4; }
+// MUSCL-Hancock with HLL in mixed precision takes 138 to 142 registers: held to four
+// waves, 36 to 56 bytes of scratch in the row loop cost more than the fourth wave gives
+// (ghost fluid 2048x1024 76.9 us per step, 71.2 with three; 4096x2048 234 / 201, cut
+// cells 236 / 213; 24 batched solves x 200 steps 29.4 ms / 26.8). The other mixed forms
+// keep to four without scratch (MUSCL cut cells 4096x2048 185; at three 189).
+template <typename T> constexpr int step_waves(int sch, int rs) {
+    return rs == RS_PVRS ? 1 : sch == SCH_MHM && rs == RS_HLL && sizeof(T) == sizeof(float) ? 3 : 4;
+}
 template <int SCH, int RS, int LIM, typename T, bool CUT>
-__global__ __launch_bounds__(64, step_waves(RS)) void k_step(StepArgs a) {
+__global__ __launch_bounds__(64, step_waves<T>(SCH, RS)) void k_step(StepArgs a) {
     step_strip<SCH, RS, LIM, T, CUT, false, true>(a, blockIdx.x, blockIdx.y, CUT ? 0 : a.stage);  // cut cells: one stage
 }
 template <int SCH, int RS, int LIM, typename T>
-__global__ __launch_bounds__(64, step_waves(RS)) void k_step_periodic(StepArgs a) {
+__global__ __launch_bounds__(64, step_waves<T>(SCH, RS)) void k_step_periodic(StepArgs a) {
     step_strip<SCH, RS, LIM, T, false, true, true>(a, blockIdx.x, blockIdx.y, a.stage);
 }
 
@@ -541,7 +549,7 @@ __global__ __launch_bounds__(64, step_waves(RS)) void k_step_periodic(StepArgs a
 // map[b].x < 0 marks an idle block (the grid is sized for the batch capacity so
 // that a captured graph stays valid while solves come and go).
 template <int SCH, int RS, int LIM, typename T>
-__global__ __launch_bounds__(64, step_waves(RS)) void k_step_batch(const StepArgs* __restrict__ slots, const int2* __restrict__ map,
+__global__ __launch_bounds__(64, step_waves<T>(SCH, RS)) void k_step_batch(const StepArgs* __restrict__ slots, const int2* __restrict__ map,
                                                    int stage) {
     const int2 m = map[blockIdx.x];
     if (m.x < 0) return;
