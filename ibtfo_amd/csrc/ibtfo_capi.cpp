@@ -1043,10 +1043,20 @@ extern "C" int ibtfo_boundary(ibtfo_ctx* x) {
     return IBTFO_OK;
 }
 
+// The step kernels' code object (load_step), where this context has not asked yet
+static hipError_t load_kernels(ibtfo_ctx* x) {
+    const ibtfo_config& c = x->cfg;
+    if (x->loaded[x->rowpar]) return hipSuccess;
+    const hipError_t e = load_step(c.scheme, c.riemann, c.limiter, c.precision, x->rowpar);
+    x->loaded[x->rowpar] = e == hipSuccess;
+    return e;
+}
+
 extern "C" int ibtfo_prepare(ibtfo_ctx* x, int apply_boundary) {
     if (!x) return IBTFO_E_ARG;
     if (!x->have_geometry || !x->have_state) { set_error("prepare needs geometry and state"); return IBTFO_E_STATE; }
     build_args(x);
+    HIPCHK(load_kernels(x));
     int rc;
     if (apply_boundary && (rc = ibtfo_boundary(x))) return rc;
     if ((rc = run_reduce(x, 1))) return rc;
@@ -1236,6 +1246,7 @@ extern "C" int ibtfo_set_tile(ibtfo_ctx* x, int rows, int row_parallel) {
     x->rowpar = row_parallel;
     drop_graph(x);
     build_args(x);
+    if (x->prepared) HIPCHK(load_kernels(x));
     return IBTFO_OK;
 }
 

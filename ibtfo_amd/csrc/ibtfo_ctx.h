@@ -32,6 +32,7 @@ struct ibtfo_ctx {
     int rows_override;  // step-kernel rows per strip
     int cur_guess;      // the current buffer after the queued steps, as far as the host knows
     int rowpar;         // 1: the row-parallel step kernel (rows + 1 waves per block)
+    int loaded[2];      // the code objects of the marching / row-parallel kernels
     double* corner;
     double Li, Hi, dxc;  // cell-centre origin and spacing (Psy_coord)
     int have_geometry, have_state, prepared;

@@ -274,6 +274,7 @@ struct SlotStatus {
 
 // kernel launchers (ibtfo_step.hip)
 hipError_t launch_step(int scheme, int rs, int lim, int prec, const StepArgs& a, hipStream_t s);
+hipError_t load_step(int scheme, int rs, int lim, int prec, int rowpar);
 hipError_t launch_fill(const FillArgs& a, hipStream_t s);
 hipError_t launch_scatter(const FillArgs& a, hipStream_t s);
 hipError_t launch_edge(const EdgeArgs& a, hipStream_t s);
@@ -300,6 +301,7 @@ hipError_t launch_persist(int scheme, int rs, int lim, int prec, const PersistAr
 int persist_blocks(int scheme, int rs, int lim, int prec);
 hipError_t launch_step_lax(const StepArgs& a, hipStream_t s);
 // the row-parallel step kernel (StepArgs::rowpar; 1 <= rows <= ROWPAR_MAX_ROWS), ibtfo_rowpar.hip
+const void* rowpar_kernel(int scheme, int rs);  // one of a scheme's and solver's row-parallel kernels
 hipError_t launch_step_rowpar(int scheme, int rs, int lim, int prec, const StepArgs& a, hipStream_t s);
 // the closing kernel of a deferred-finish batch whose last kernel had parity k
 hipError_t launch_df_flush(const StepArgs& a, int k, hipStream_t s);

@@ -402,6 +402,45 @@ __device__ __forceinline__ void step_rowpar(const StepArgs& a, const int bx, con
     }
 }
 
+template <int SCH, int RS, int LIM, typename T, bool CUT>
+__global__ __launch_bounds__(64 * (ROWPAR_MAX_ROWS + 1)) void k_step_rowpar(StepArgs a) {
+    step_rowpar<SCH, RS, LIM, T, CUT>(a, blockIdx.x, blockIdx.y, a.stage);
+}
+
+// Compiled in nine objects, one per scheme and Riemann solver (STEP_SCHEME,
+// STEP_RIEMANN), so that a solve loads its own kernels only (a process's first steps on
+// a small grid: 4.5 ms with all of them in one object).
+template <int SCH, int RS> hipError_t go_rowpar_l(int lim, int prec, const StepArgs& a, hipStream_t s);
+template <int SCH, int RS> const void* rowpar_kernel_l();
+
+#ifdef STEP_SCHEME
+template <int SCH, int RS, int LIM>
+static hipError_t go_rowpar(int prec, const StepArgs& a, hipStream_t s) {
+    const dim3 grid(a.nbx, a.nby), block(64 * (a.rows + 1));
+    const int l64 = rowpar_lds(a.rows, sizeof(double)), l32 = rowpar_lds(a.rows, sizeof(float));
+    if (a.cut) {
+        if (prec == 1) hipLaunchKernelGGL((k_step_rowpar<SCH, RS, LIM, float, true>), grid, block, l32, s, a);
+        else hipLaunchKernelGGL((k_step_rowpar<SCH, RS, LIM, double, true>), grid, block, l64, s, a);
+    } else {
+        if (prec == 1) hipLaunchKernelGGL((k_step_rowpar<SCH, RS, LIM, float, false>), grid, block, l32, s, a);
+        else hipLaunchKernelGGL((k_step_rowpar<SCH, RS, LIM, double, false>), grid, block, l64, s, a);
+    }
+    return hipGetLastError();
+}
+template <int SCH, int RS>
+hipError_t go_rowpar_l(int lim, int prec, const StepArgs& a, hipStream_t s) {
+    if (lim == LIM_MINMOD) return go_rowpar<SCH, RS, LIM_MINMOD>(prec, a, s);
+    if (lim == LIM_VANLEER) return go_rowpar<SCH, RS, LIM_VANLEER>(prec, a, s);
+    return go_rowpar<SCH, RS, LIM_VANALBADA>(prec, a, s);
+}
+template <int SCH, int RS> const void* rowpar_kernel_l() {
+    return (const void*)k_step_rowpar<SCH, RS, LIM_MINMOD, double, false>;
+}
+template hipError_t go_rowpar_l<STEP_SCHEME, STEP_RIEMANN>(int, int, const StepArgs&, hipStream_t);
+template const void* rowpar_kernel_l<STEP_SCHEME, STEP_RIEMANN>();
+
+#else  // ------------------------------------------- the flush and the dispatch
+
 // The end of a deferred-finish batch: the finish of its last kernel (parity
 // k), if that kernel ran its step, published to the control block as the
 // finish kernel leaves it (ran = whether that step ran).
@@ -422,30 +461,6 @@ __global__ __launch_bounds__(64) void k_df_flush(StepArgs a, int k) {
     ctl->ran = h.pending;
 }
 
-template <int SCH, int RS, int LIM, typename T, bool CUT>
-__global__ __launch_bounds__(64 * (ROWPAR_MAX_ROWS + 1)) void k_step_rowpar(StepArgs a) {
-    step_rowpar<SCH, RS, LIM, T, CUT>(a, blockIdx.x, blockIdx.y, a.stage);
-}
-
-template <int SCH, int RS, int LIM>
-static hipError_t go_rowpar(int prec, const StepArgs& a, hipStream_t s) {
-    const dim3 grid(a.nbx, a.nby), block(64 * (a.rows + 1));
-    const int l64 = rowpar_lds(a.rows, sizeof(double)), l32 = rowpar_lds(a.rows, sizeof(float));
-    if (a.cut) {
-        if (prec == 1) hipLaunchKernelGGL((k_step_rowpar<SCH, RS, LIM, float, true>), grid, block, l32, s, a);
-        else hipLaunchKernelGGL((k_step_rowpar<SCH, RS, LIM, double, true>), grid, block, l64, s, a);
-    } else {
-        if (prec == 1) hipLaunchKernelGGL((k_step_rowpar<SCH, RS, LIM, float, false>), grid, block, l32, s, a);
-        else hipLaunchKernelGGL((k_step_rowpar<SCH, RS, LIM, double, false>), grid, block, l64, s, a);
-    }
-    return hipGetLastError();
-}
-template <int SCH, int RS>
-static hipError_t go_rowpar_l(int lim, int prec, const StepArgs& a, hipStream_t s) {
-    if (lim == LIM_MINMOD) return go_rowpar<SCH, RS, LIM_MINMOD>(prec, a, s);
-    if (lim == LIM_VANLEER) return go_rowpar<SCH, RS, LIM_VANLEER>(prec, a, s);
-    return go_rowpar<SCH, RS, LIM_VANALBADA>(prec, a, s);
-}
 template <int SCH>
 static hipError_t go_rowpar_r(int rs, int lim, int prec, const StepArgs& a, hipStream_t s) {
     if (rs == RS_SW) return go_rowpar_l<SCH, RS_SW>(lim, prec, a, s);
@@ -466,5 +481,18 @@ hipError_t launch_step_rowpar(int scheme, int rs, int lim, int prec, const StepA
     if (scheme == SCH_GODUNOV) return go_rowpar_r<SCH_GODUNOV>(rs, lim, prec, a, s);
     return go_rowpar_r<SCH_MUSCL>(rs, lim, prec, a, s);
 }
+
+template <int SCH> static const void* rowpar_kernel_r(int rs) {
+    if (rs == RS_SW) return rowpar_kernel_l<SCH, RS_SW>();
+    if (rs == RS_PVRS) return rowpar_kernel_l<SCH, RS_PVRS>();
+    return rowpar_kernel_l<SCH, RS_HLL>();
+}
+const void* rowpar_kernel(int scheme, int rs) {
+    if (scheme == SCH_MHM) return rowpar_kernel_r<SCH_MHM>(rs);
+    if (scheme == SCH_GODUNOV) return rowpar_kernel_r<SCH_GODUNOV>(rs);
+    return rowpar_kernel_r<SCH_MUSCL>(rs);
+}
+
+#endif  // STEP_SCHEME
 
 }  // namespace ibtfo

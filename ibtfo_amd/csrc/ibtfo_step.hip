@@ -127,10 +127,6 @@ __device__ __forceinline__ void finish_body(const FinishArgs& f, const int advan
     }
     if (t == 0) finish_clock(f, ctl, sA[0], sU[0], sV[0], sM[0], sB[0], advance, ctl->now_t, ctl->iter);
 }
-__global__ __launch_bounds__(FINISH_THREADS) void k_finish(FinishArgs f) {
-    finish_body<FINISH_THREADS>(f, f.advance);
-}
-
 // The same finish in one wave, for at most FINISH_SMALL_MAX records (small
 // grids, whose step is a chain of latencies): each lane reads its records in
 // one round trip, the control fields are read beside them rather than first,
@@ -162,8 +158,6 @@ __device__ __forceinline__ void finish_small(const FinishArgs& f, const int adva
     if (advance && done) return;  // the step kernel did not run
     if (t == 0) finish_clock(f, ctl, A, Um, Vm, m, bad, advance, now_t, iter);
 }
-__global__ __launch_bounds__(64) void k_finish_small(FinishArgs f) { finish_small(f, f.advance); }
-
 // Partial record of a 256-thread block (valid in thread 0): wave reductions, then
 // the four waves in order.
 __device__ __forceinline__ void block4_reduce(double& amax, double& umax, double& vmax, double& msum, int& bad) {
@@ -232,8 +226,6 @@ __device__ __forceinline__ void fold_body(const FinishArgs& f, const int block) 
     g.nblocks2 = 0;
     finish_body<FOLD_THREADS, true>(g, 1);
 }
-__global__ __launch_bounds__(FOLD_THREADS) void k_fold(FinishArgs f) { fold_body(f, blockIdx.x); }
-
 // The step body for one 64-lane block: strip (bx, by) of the solve described
 // by `a`; `stage` as StepArgs::stage. Used by the single-solve kernel and by the
 // batched kernel, whose blocks each pick their solve from a block map.
@@ -557,6 +549,371 @@ __global__ __launch_bounds__(64, step_waves<T>(SCH, RS)) void k_step_batch(const
     step_strip<SCH, RS, LIM, T, false>(a, m.y % a.nbx, m.y / a.nbx, stage);
 }
 
+// A ghost's new value v (Boundary): IDWBaseGFM/GFM_Bound.cpp:65-106,
+// LinearBaseGFM/GFM_Bound.cpp:58-575, BCGFM/BCGFM_Bound.cpp:81-175,
+// HBCGFM/HBCGFM_Bound.cpp:163-178, SimpleBound/LS_SimpleBound.cpp:38-105. U: the
+// state right after the update, before any ghost is rewritten; Uring: where the
+// donors marked in Ghost::ring are read.
+__device__ __forceinline__ void ghost_value(const FillArgs& a, const Ghost& gh, const double* U, const double* Uring,
+                                            double (&v4)[4]) {
+    const long long PL = a.L.plane, P = a.L.pitch;
+    const double gm1 = a.gm1;
+    auto prim = [&](long long d, bool ring, double& r, double& u, double& v, double& p) {
+        const double* S = ring ? Uring : U;
+        double q[4] = {S[d], S[d + PL], S[d + 2 * PL], S[d + 3 * PL]};
+        primitives(gm1, q, r, u, v, p);
+    };
+    auto idw = [&](long long d1, int rbits, const double* w, double& R, double& Uu, double& V, double& Pp) {
+        double r[4], u[4], v[4], p[4];
+        const long long dd[4] = {d1, d1 + P, d1 + P + 1, d1 + 1};
+        for (int q = 0; q < 4; q++) prim(dd[q], (rbits >> q) & 1, r[q], u[q], v[q], p[q]);
+        if (!a.quirks)  // corrected mode: a donor at the point itself (1/0 weight) is the value
+            for (int q = 0; q < 4; q++)
+                if (__builtin_isinf(w[q])) { R = r[q]; Uu = u[q]; V = v[q]; Pp = p[q]; return; }
+        double s = w[0] + w[1] + w[2] + w[3];
+        R = (w[0] * r[0] + w[1] * r[1] + w[2] * r[2] + w[3] * r[3]) / s;
+        Uu = (w[0] * u[0] + w[1] * u[1] + w[2] * u[2] + w[3] * u[3]) / s;
+        V = (w[0] * v[0] + w[1] * v[1] + w[2] * v[2] + w[3] * v[3]) / s;
+        Pp = (w[0] * p[0] + w[1] * p[1] + w[2] * p[2] + w[3] * p[3]) / s;
+    };
+    const double n_x = gh.nx, n_y = gh.ny;
+    double rw, uw, vw, pw;
+    if (a.bc == 1) {  // IDWBaseGFM
+        if (!a.quirks && gh.a[0] + gh.a[1] + gh.a[2] + gh.a[3] == 0.0) {
+            // corrected mode: no fluid donor, the ghost keeps its value
+            for (int k = 0; k < 4; k++) v4[k] = U[gh.cell + k * PL];
+            return;
+        }
+        idw(gh.d1, gh.ring & 15, gh.a, rw, uw, vw, pw);
+        double u_n = uw * n_x + vw * n_y;
+        double u_t = uw * n_y - vw * n_x;
+        u_n = -u_n;
+        uw = u_n * n_x + u_t * n_y;
+        vw = u_n * n_y - u_t * n_x;
+    } else if (a.bc == IBTFO_SIMPLE_BOUND) {
+        // SimpleBound/LS_SimpleBound.cpp:38-105: reflect the x donor's u and/or the y
+        // donor's v (the mean of both reflections when both exist). A donor that is
+        // a ghost filled earlier in the reference's order is read from its new
+        // value (an earlier dependency level), any other from the state.
+        const int IDX = gh.idx, IDY = gh.idy;
+        if (IDX == 0 && IDY == 0) {  // no fluid within reach: the ghost keeps its value
+            for (int k = 0; k < 4; k++) v4[k] = U[gh.cell + k * PL];
+            return;
+        }
+        auto donor = [&](long long d, int earlier, bool ring, double& r, double& u, double& v, double& p) {
+            if (earlier >= 0) {
+                const double* q = a.out + 4 * (long long)earlier;
+                double qq[4] = {q[0], q[1], q[2], q[3]};
+                primitives(gm1, qq, r, u, v, p);
+            } else {
+                prim(d, ring, r, u, v, p);
+            }
+        };
+        double rx = 0, ux = 0, vx = 0, px = 0, ry = 0, uy = 0, vy = 0, py = 0;
+        if (IDX != 0) donor(gh.d1, gh.idxe, gh.ring & 1, rx, ux, vx, px);
+        if (IDY != 0) donor(gh.d1e, gh.idye, (gh.ring >> 4) & 1, ry, uy, vy, py);
+        if (IDX != 0 && IDY != 0) {
+            rw = 0.5 * (rx + ry); uw = 0.5 * (-ux + uy); vw = 0.5 * (vx - vy); pw = 0.5 * (px + py);
+        } else if (IDX != 0) {
+            rw = rx; uw = -ux; vw = vx; pw = px;
+        } else {
+            rw = ry; uw = uy; vw = -vy; pw = py;
+        }
+    } else if (a.bc == 2 || a.bc == 3) {  // Linear/RiemannBaseGFM: one donor
+        int pick = (int)gh.a[0];
+        if (pick >= 0) {
+            const long long dd[4] = {gh.d1, gh.d1 + P, gh.d1 + P + 1, gh.d1 + 1};
+            prim(dd[pick], (gh.ring >> pick) & 1, rw, uw, vw, pw);
+        } else {
+            rw = 0; uw = 0; vw = 0; pw = 0;
+        }
+        double u_n = uw * n_x + vw * n_y;
+        double u_t = uw * n_y - vw * n_x;
+        u_n = -u_n;
+        uw = u_n * n_x + u_t * n_y;
+        vw = u_n * n_y - u_t * n_x;
+    } else {  // BCGFM / HBCGFM
+        double delta = ib_sqrt(a.dxg * a.dxg + a.dyg * a.dyg) / 2;
+        double R_E = delta, R_G = gh.phi;
+        double ri, ui, vi, pi_, re, ue, ve, pe;
+        idw(gh.d1, gh.ring & 15, gh.a, ri, ui, vi, pi_);
+        double uni = ui * n_x + vi * n_y, uti = ui * n_y - vi * n_x;
+        idw(gh.d1e, (gh.ring >> 4) & 15, gh.ae, re, ue, ve, pe);
+        double une = ue * n_x + ve * n_y, ute = ue * n_y - ve * n_x;
+        double un, ut;
+        if (a.bc == 5 && R_G > delta) {
+            rw = ri; pw = pi_; ut = uti; un = -uni;
+        } else {
+            double A = ((delta + R_E) * (delta + R_E) - R_G * R_G), B = (delta * delta - R_G * R_G);
+            double D = (R_E * R_E + 2 * delta * R_E);
+            rw = (ri * A - re * B) / D;
+            pw = (pi_ * A - pe * B) / D;
+            ut = (uti * A - ute * B) / D;
+            un = -(uni * A - une * B) / D;
+        }
+        uw = un * n_x + ut * n_y;
+        vw = un * n_y - ut * n_x;
+    }
+    v4[0] = rw;
+    v4[1] = rw * uw;
+    v4[2] = rw * vw;
+    v4[3] = pw / gm1 + 0.5 * rw * (uw * uw + vw * vw);
+}
+
+// Ghost-cell fill, phase 1: the values into a compact buffer (stand-alone
+// Boundary, SimpleBound's dependency levels, the persistent batch kernel).
+__device__ __forceinline__ void fill_one(const FillArgs& a, const int gi) {
+    if (a.require_ran && !a.ctl->ran) return;
+    if (gi >= a.nghost) return;
+    const Ghost gh = a.ghosts[gi];
+    if (a.bc == IBTFO_SIMPLE_BOUND && gh.pick != a.level) return;
+    const int cur = a.use_cur ? a.ctl->cur : a.fixed;
+    const double* U = a.buf[cur];
+    // Boundary runs before Global_Boundary in the reference, so a donor in the
+    // domain ring still holds the ring of the previous state
+    double v[4];
+    ghost_value(a, gh, U, a.ring_prev ? a.buf[cur ^ 1] : U, v);
+    double* o = a.out + 4 * (long long)gi;
+    for (int k = 0; k < 4; k++) o[k] = v[k];
+}
+// The fill after a step in one phase, in place. The reference's Boundary reads
+// every donor before any ghost is rewritten; a step leaves non-active cells as
+// they were (U_NEW = U_OLD there), so a donor that is a ghost, or lies in the
+// ring, still holds its value in the state before the step, which nothing in
+// this launch writes. The active donors are written by no one here either.
+__device__ __forceinline__ void fill_in_place(const FillArgs& a, const int gi) {
+    if (gi >= a.nghost) return;
+    // the record and the flags in one round trip
+    const Ghost gh = a.ghosts[gi];
+    const int ran = a.ctl->ran, out = a.ctl->out;
+    if (!ran) return;
+    double* U = a.buf[out];
+    double v[4];
+    ghost_value(a, gh, U, a.buf[out ^ 1], v);
+    for (int k = 0; k < 4; k++) U[gh.cell + k * a.L.plane] = v[k];
+}
+
+// Ghost-cell fill, phase 2: write the values into the current state.
+__device__ __forceinline__ void scatter_one(const FillArgs& a, const int gi) {
+    if (a.require_ran && !a.ctl->ran) return;
+    if (gi >= a.nghost) return;
+    double* U = a.buf[a.use_cur ? a.ctl->cur : a.fixed];
+    const long long c = a.ghosts[gi].cell, PL = a.L.plane;
+    const double* v = a.out + 4 * (long long)gi;
+    U[c] = v[0];
+    U[c + PL] = v[1];
+    U[c + 2 * PL] = v[2];
+    U[c + 3 * PL] = v[3];
+}
+// Ring of the current state for the edge policies that are not fused into the
+// step (the reference policy for Lax; periodic; inflow). Reads the interior of
+// the current state, writes its ring; one thread per ring cell.
+// PREV: beside the in-place fill: the state is the buffer the step wrote, and a
+// non-active source cell is read from the state before the step, where it has
+// the value it had before the fill.
+template <bool PREV> __device__ __forceinline__ void edge_one(const EdgeArgs& a, const int q) {
+    if (PREV ? !a.ctl->ran : a.require_ran && !a.ctl->ran) return;
+    const Layout L = a.L;
+    const int ng = L.ng, nx = L.nx, ny = L.ny;
+    const int nring = L.M * L.N - nx * ny;
+    if (q >= nring) return;
+    // enumerate ring cells: bottom rows, top rows, then left/right columns of interior rows
+    int i, j;
+    int nb = L.M * ng;
+    if (q < nb) { j = q / L.M; i = q % L.M; }
+    else if (q < 2 * nb) { int r = q - nb; j = ny + ng + r / L.M; i = r % L.M; }
+    else { int r = q - 2 * nb; j = ng + r / (2 * ng); int s = r % (2 * ng); i = s < ng ? s : nx + s; }
+    const int b = PREV ? a.ctl->out : a.ctl->cur;
+    double* U = a.buf[b];
+    auto source = [&](long long s) -> const double* {
+        if (PREV) {
+            const uint8_t t = a.type[s];
+            return t == 0 || t == 3 ? U : a.buf[b ^ 1];
+        }
+        return (a.unew_nf && a.type[s] != 0) ? a.unew_nf : U;
+    };
+    const long long PL = L.plane;
+    double v[4];
+    if (a.kind == 1) {  // periodic
+        int si = i < ng ? i + nx : (i >= nx + ng ? i - nx : i);
+        int sj = j < ng ? j + ny : (j >= ny + ng ? j - ny : j);
+        long long s = L.at(si, sj);
+        const double* S = source(s);
+        for (int k = 0; k < 4; k++) v[k] = S[s + k * PL];
+    } else if (a.kind == 3) {
+        // Test/PNGGeo/Global_Boudary.cpp:14-79 (U_NEW = the state before the ghost
+        // fill's phase 2): rows as the Sod hook over the interior columns, the
+        // right columns zero-gradient, the left columns held at the inflow state;
+        // the ring corners are not written
+        const bool row = j < ng || j >= ny + ng;
+        if (row && (i < ng || i >= nx + ng)) return;
+        auto src = [&](long long s, int k) { return source(s)[s + k * PL]; };
+        if (row) {
+            const int sr = j < ng ? 2 * ng - 1 : ny + ng - 1;
+            const int rr = j < ng ? 2 * ng - j - 1 : 2 * (ny + ng) - 1 - j;
+            for (int k = 0; k < 4; k++) v[k] = src(L.at(i, sr), k);
+            v[2] = -src(L.at(i, rr), 2);
+        } else if (i < ng) {
+            for (int k = 0; k < 4; k++) v[k] = a.inflow[k];
+        } else {
+            for (int k = 0; k < 4; k++) v[k] = src(L.at(nx + ng - 1, j), k);
+        }
+    } else if (a.kind == 2) {  // inflow left, zero gradient elsewhere
+        if (i < ng) {
+            for (int k = 0; k < 4; k++) v[k] = a.inflow[k];
+        } else {
+            int si = i >= nx + ng ? nx + ng - 1 : i;
+            int sj = j < ng ? ng : (j >= ny + ng ? ny + ng - 1 : j);
+            long long s = L.at(si, sj);
+            const double* S = source(s);
+            for (int k = 0; k < 4; k++) v[k] = S[s + k * PL];
+        }
+    } else {
+        return;  // the reference policy is written by the step kernel
+    }
+    long long o = L.at(i, j);
+    for (int k = 0; k < 4; k++) U[o + k * PL] = v[k];
+}
+// ------------------------------------------------------ persistent batched step
+// Grid barrier among all blocks of a launch (every block resident): arrivals
+// counted in bar[0], which only grows during a launch, so barrier k completes
+// when it reaches (k + 1) x blocks. Device-scope fences before the arrival
+// (release: this block's stores reach the coherence point past its XCD's L2)
+// and after the wait (acquire: no stale lines of other XCDs' stores). A wait
+// longer than spin_limit polls sets *err and every block leaves the launch.
+__device__ __forceinline__ bool grid_sync(const PersistArgs& p, unsigned int& target) {
+    target += gridDim.x;
+    int ok = 1;
+    if (threadIdx.x == 0) {
+        __threadfence();
+        atomicAdd(p.bar, 1u);
+        long long spins = 0;
+        while (__hip_atomic_load(p.bar, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < target) {
+            __builtin_amdgcn_s_sleep(2);
+            if (++spins > p.spin_limit || __hip_atomic_load(p.err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
+                atomicExch(p.err, 1);
+                ok = 0;
+                break;
+            }
+        }
+        __threadfence();
+    }
+    return __shfl(ok, 0, 64) != 0;
+}
+
+template <int SCH, int RS, int LIM, typename T>
+__global__ __launch_bounds__(64) void k_persist(PersistArgs p) {
+    const int G = gridDim.x;
+    unsigned int target = 0;
+    const int nstrip = p.counts[0], nghost = p.counts[1], nring = p.counts[2];
+    for (int s = 0; s < p.nsteps; s++) {
+        for (int stage = p.rk2 ? 1 : 0;;) {
+            // strips of every resident solve (TimeAdvance; reference ring fused)
+            for (int w = blockIdx.x; w < nstrip; w += G) {
+                const int2 m = p.smap[w];
+                const StepArgs& a = p.step[m.x];
+                step_strip<SCH, RS, LIM, T, false>(a, m.y % a.nbx, m.y / a.nbx, stage);
+            }
+            if (!grid_sync(p, target)) return;
+            // ComputeDt / mass / clock per solve (RK2 stage 1: make the stage buffer current)
+            for (int q = blockIdx.x; q < p.nslots; q += G)
+                if (p.fin[q].ctl) finish_body<64>(p.fin[q], stage == 1 ? 2 : 1);
+            if (!grid_sync(p, target)) return;
+            // Boundary phase 1 and Global_Boundary
+            if (p.has_fill)
+                for (int w = blockIdx.x; w < nghost; w += G) {
+                    const int2 m = p.gmap[w];
+                    for (int k = threadIdx.x; k < FILL_THREADS; k += 64) fill_one(p.fill[m.x], m.y + k);
+                }
+            for (int w = blockIdx.x; w < nring; w += G) {
+                const int2 m = p.rmap[w];
+                for (int k = threadIdx.x; k < EDGE_THREADS; k += 64) edge_one<false>(p.edge[m.x], m.y + k);
+            }
+            if (!grid_sync(p, target)) return;
+            // Boundary phase 2
+            if (p.has_fill) {
+                for (int w = blockIdx.x; w < nghost; w += G) {
+                    const int2 m = p.gmap[w];
+                    for (int k = threadIdx.x; k < FILL_THREADS; k += 64) scatter_one(p.fill[m.x], m.y + k);
+                }
+                if (!grid_sync(p, target)) return;
+            }
+            if (stage == 1) { stage = 2; continue; }
+            break;
+        }
+    }
+}
+
+// The strip kernels are compiled in nine objects, one per scheme and Riemann solver
+// (STEP_SCHEME, STEP_RIEMANN) of 0.4 to 1.2 MB, each a code object that a process loads
+// when it first needs one of its kernels; the rest are 0.1 MB. In one object of 6.6 MB
+// they loaded for any solve. An 800x400 channel, the first solve of a process, from its
+// creation to two steps: 42 ms with one object each for the strips and the row-parallel
+// kernels, 26 with these.
+// A batched launch (k_step_batch) instead of a single-solve one when non-null.
+struct BatchLaunch {
+    const StepArgs* slots;
+    const int2* map;
+    int nblocks;
+    int stage;
+};
+// launches of one scheme and solver, and its persistent kernel
+template <int SCH, int RS>
+hipError_t go_l(int lim, int prec, const StepArgs* a, const BatchLaunch* b, hipStream_t s);
+template <int SCH, int RS> const void* persist_l(int lim, int prec);
+
+#ifdef STEP_SCHEME
+template <int SCH, int RS, int LIM>
+static hipError_t go(int prec, const StepArgs* a, const BatchLaunch* b, hipStream_t s) {
+    if (b) {
+        if (prec == 1)
+            hipLaunchKernelGGL((k_step_batch<SCH, RS, LIM, float>), dim3(b->nblocks), dim3(64), 0, s, b->slots, b->map,
+                               b->stage);
+        else
+            hipLaunchKernelGGL((k_step_batch<SCH, RS, LIM, double>), dim3(b->nblocks), dim3(64), 0, s, b->slots,
+                               b->map, b->stage);
+    } else if (a->cut) {  // cut-cell variant (its extra registers stay out of the plain kernel)
+        if (prec == 1) hipLaunchKernelGGL((k_step<SCH, RS, LIM, float, true>), dim3(a->nbx, a->nby), dim3(64), 0, s, *a);
+        else hipLaunchKernelGGL((k_step<SCH, RS, LIM, double, true>), dim3(a->nbx, a->nby), dim3(64), 0, s, *a);
+    } else if (a->edge_fused == 2) {  // periodic ring written by the step kernel
+        if (prec == 1) hipLaunchKernelGGL((k_step_periodic<SCH, RS, LIM, float>), dim3(a->nbx, a->nby), dim3(64), 0, s, *a);
+        else hipLaunchKernelGGL((k_step_periodic<SCH, RS, LIM, double>), dim3(a->nbx, a->nby), dim3(64), 0, s, *a);
+    } else {
+        if (prec == 1) hipLaunchKernelGGL((k_step<SCH, RS, LIM, float, false>), dim3(a->nbx, a->nby), dim3(64), 0, s, *a);
+        else hipLaunchKernelGGL((k_step<SCH, RS, LIM, double, false>), dim3(a->nbx, a->nby), dim3(64), 0, s, *a);
+    }
+    return hipGetLastError();
+}
+template <int SCH, int RS>
+hipError_t go_l(int lim, int prec, const StepArgs* a, const BatchLaunch* b, hipStream_t s) {
+    if (lim == LIM_MINMOD) return go<SCH, RS, LIM_MINMOD>(prec, a, b, s);
+    if (lim == LIM_VANLEER) return go<SCH, RS, LIM_VANLEER>(prec, a, b, s);
+    return go<SCH, RS, LIM_VANALBADA>(prec, a, b, s);
+}
+template <int SCH, int RS, int LIM>
+static const void* persist_fn(int prec) {
+    if (prec == IBTFO_MIXED) return (const void*)k_persist<SCH, RS, LIM, float>;
+    return (const void*)k_persist<SCH, RS, LIM, double>;
+}
+template <int SCH, int RS> const void* persist_l(int lim, int prec) {
+    if (lim == LIM_MINMOD) return persist_fn<SCH, RS, LIM_MINMOD>(prec);
+    if (lim == LIM_VANLEER) return persist_fn<SCH, RS, LIM_VANLEER>(prec);
+    return persist_fn<SCH, RS, LIM_VANALBADA>(prec);
+}
+template hipError_t go_l<STEP_SCHEME, STEP_RIEMANN>(int, int, const StepArgs*, const BatchLaunch*, hipStream_t);
+template const void* persist_l<STEP_SCHEME, STEP_RIEMANN>(int, int);
+
+#else  // ------------------------------------------- the other kernels and the dispatch
+
+__global__ __launch_bounds__(FINISH_THREADS) void k_finish(FinishArgs f) {
+    finish_body<FINISH_THREADS>(f, f.advance);
+}
+
+__global__ __launch_bounds__(64) void k_finish_small(FinishArgs f) { finish_small(f, f.advance); }
+
+__global__ __launch_bounds__(FOLD_THREADS) void k_fold(FinishArgs f) { fold_body(f, blockIdx.x); }
+
+
 // Lax-Friedrichs, Lax_Scheme.cpp:27-62: U_new = average of the 4 neighbours minus
 // central flux differences. Same strip decomposition; lane t owns column cb-1+t.
 __global__ __launch_bounds__(64) void k_step_lax(StepArgs a) {
@@ -688,236 +1045,12 @@ __global__ __launch_bounds__(MERGE_THREADS) void k_merge(MergeArgs a) {
     block_partials(a.part, blockIdx.x, amax, umax, vmax, msum, bad);
 }
 
-// A ghost's new value v (Boundary): IDWBaseGFM/GFM_Bound.cpp:65-106,
-// LinearBaseGFM/GFM_Bound.cpp:58-575, BCGFM/BCGFM_Bound.cpp:81-175,
-// HBCGFM/HBCGFM_Bound.cpp:163-178, SimpleBound/LS_SimpleBound.cpp:38-105. U: the
-// state right after the update, before any ghost is rewritten; Uring: where the
-// donors marked in Ghost::ring are read.
-__device__ __forceinline__ void ghost_value(const FillArgs& a, const Ghost& gh, const double* U, const double* Uring,
-                                            double (&v4)[4]) {
-    const long long PL = a.L.plane, P = a.L.pitch;
-    const double gm1 = a.gm1;
-    auto prim = [&](long long d, bool ring, double& r, double& u, double& v, double& p) {
-        const double* S = ring ? Uring : U;
-        double q[4] = {S[d], S[d + PL], S[d + 2 * PL], S[d + 3 * PL]};
-        primitives(gm1, q, r, u, v, p);
-    };
-    auto idw = [&](long long d1, int rbits, const double* w, double& R, double& Uu, double& V, double& Pp) {
-        double r[4], u[4], v[4], p[4];
-        const long long dd[4] = {d1, d1 + P, d1 + P + 1, d1 + 1};
-        for (int q = 0; q < 4; q++) prim(dd[q], (rbits >> q) & 1, r[q], u[q], v[q], p[q]);
-        if (!a.quirks)  // corrected mode: a donor at the point itself (1/0 weight) is the value
-            for (int q = 0; q < 4; q++)
-                if (__builtin_isinf(w[q])) { R = r[q]; Uu = u[q]; V = v[q]; Pp = p[q]; return; }
-        double s = w[0] + w[1] + w[2] + w[3];
-        R = (w[0] * r[0] + w[1] * r[1] + w[2] * r[2] + w[3] * r[3]) / s;
-        Uu = (w[0] * u[0] + w[1] * u[1] + w[2] * u[2] + w[3] * u[3]) / s;
-        V = (w[0] * v[0] + w[1] * v[1] + w[2] * v[2] + w[3] * v[3]) / s;
-        Pp = (w[0] * p[0] + w[1] * p[1] + w[2] * p[2] + w[3] * p[3]) / s;
-    };
-    const double n_x = gh.nx, n_y = gh.ny;
-    double rw, uw, vw, pw;
-    if (a.bc == 1) {  // IDWBaseGFM
-        if (!a.quirks && gh.a[0] + gh.a[1] + gh.a[2] + gh.a[3] == 0.0) {
-            // corrected mode: no fluid donor, the ghost keeps its value
-            for (int k = 0; k < 4; k++) v4[k] = U[gh.cell + k * PL];
-            return;
-        }
-        idw(gh.d1, gh.ring & 15, gh.a, rw, uw, vw, pw);
-        double u_n = uw * n_x + vw * n_y;
-        double u_t = uw * n_y - vw * n_x;
-        u_n = -u_n;
-        uw = u_n * n_x + u_t * n_y;
-        vw = u_n * n_y - u_t * n_x;
-    } else if (a.bc == IBTFO_SIMPLE_BOUND) {
-        // SimpleBound/LS_SimpleBound.cpp:38-105: reflect the x donor's u and/or the y
-        // donor's v (the mean of both reflections when both exist). A donor that is
-        // a ghost filled earlier in the reference's order is read from its new
-        // value (an earlier dependency level), any other from the state.
-        const int IDX = gh.idx, IDY = gh.idy;
-        if (IDX == 0 && IDY == 0) {  // no fluid within reach: the ghost keeps its value
-            for (int k = 0; k < 4; k++) v4[k] = U[gh.cell + k * PL];
-            return;
-        }
-        auto donor = [&](long long d, int earlier, bool ring, double& r, double& u, double& v, double& p) {
-            if (earlier >= 0) {
-                const double* q = a.out + 4 * (long long)earlier;
-                double qq[4] = {q[0], q[1], q[2], q[3]};
-                primitives(gm1, qq, r, u, v, p);
-            } else {
-                prim(d, ring, r, u, v, p);
-            }
-        };
-        double rx = 0, ux = 0, vx = 0, px = 0, ry = 0, uy = 0, vy = 0, py = 0;
-        if (IDX != 0) donor(gh.d1, gh.idxe, gh.ring & 1, rx, ux, vx, px);
-        if (IDY != 0) donor(gh.d1e, gh.idye, (gh.ring >> 4) & 1, ry, uy, vy, py);
-        if (IDX != 0 && IDY != 0) {
-            rw = 0.5 * (rx + ry); uw = 0.5 * (-ux + uy); vw = 0.5 * (vx - vy); pw = 0.5 * (px + py);
-        } else if (IDX != 0) {
-            rw = rx; uw = -ux; vw = vx; pw = px;
-        } else {
-            rw = ry; uw = uy; vw = -vy; pw = py;
-        }
-    } else if (a.bc == 2 || a.bc == 3) {  // Linear/RiemannBaseGFM: one donor
-        int pick = (int)gh.a[0];
-        if (pick >= 0) {
-            const long long dd[4] = {gh.d1, gh.d1 + P, gh.d1 + P + 1, gh.d1 + 1};
-            prim(dd[pick], (gh.ring >> pick) & 1, rw, uw, vw, pw);
-        } else {
-            rw = 0; uw = 0; vw = 0; pw = 0;
-        }
-        double u_n = uw * n_x + vw * n_y;
-        double u_t = uw * n_y - vw * n_x;
-        u_n = -u_n;
-        uw = u_n * n_x + u_t * n_y;
-        vw = u_n * n_y - u_t * n_x;
-    } else {  // BCGFM / HBCGFM
-        double delta = ib_sqrt(a.dxg * a.dxg + a.dyg * a.dyg) / 2;
-        double R_E = delta, R_G = gh.phi;
-        double ri, ui, vi, pi_, re, ue, ve, pe;
-        idw(gh.d1, gh.ring & 15, gh.a, ri, ui, vi, pi_);
-        double uni = ui * n_x + vi * n_y, uti = ui * n_y - vi * n_x;
-        idw(gh.d1e, (gh.ring >> 4) & 15, gh.ae, re, ue, ve, pe);
-        double une = ue * n_x + ve * n_y, ute = ue * n_y - ve * n_x;
-        double un, ut;
-        if (a.bc == 5 && R_G > delta) {
-            rw = ri; pw = pi_; ut = uti; un = -uni;
-        } else {
-            double A = ((delta + R_E) * (delta + R_E) - R_G * R_G), B = (delta * delta - R_G * R_G);
-            double D = (R_E * R_E + 2 * delta * R_E);
-            rw = (ri * A - re * B) / D;
-            pw = (pi_ * A - pe * B) / D;
-            ut = (uti * A - ute * B) / D;
-            un = -(uni * A - une * B) / D;
-        }
-        uw = un * n_x + ut * n_y;
-        vw = un * n_y - ut * n_x;
-    }
-    v4[0] = rw;
-    v4[1] = rw * uw;
-    v4[2] = rw * vw;
-    v4[3] = pw / gm1 + 0.5 * rw * (uw * uw + vw * vw);
-}
-
-// Ghost-cell fill, phase 1: the values into a compact buffer (stand-alone
-// Boundary, SimpleBound's dependency levels, the persistent batch kernel).
-__device__ __forceinline__ void fill_one(const FillArgs& a, const int gi) {
-    if (a.require_ran && !a.ctl->ran) return;
-    if (gi >= a.nghost) return;
-    const Ghost gh = a.ghosts[gi];
-    if (a.bc == IBTFO_SIMPLE_BOUND && gh.pick != a.level) return;
-    const int cur = a.use_cur ? a.ctl->cur : a.fixed;
-    const double* U = a.buf[cur];
-    // Boundary runs before Global_Boundary in the reference, so a donor in the
-    // domain ring still holds the ring of the previous state
-    double v[4];
-    ghost_value(a, gh, U, a.ring_prev ? a.buf[cur ^ 1] : U, v);
-    double* o = a.out + 4 * (long long)gi;
-    for (int k = 0; k < 4; k++) o[k] = v[k];
-}
 __global__ void k_fill(FillArgs a) { fill_one(a, blockIdx.x * blockDim.x + threadIdx.x); }
 
-// The fill after a step in one phase, in place. The reference's Boundary reads
-// every donor before any ghost is rewritten; a step leaves non-active cells as
-// they were (U_NEW = U_OLD there), so a donor that is a ghost, or lies in the
-// ring, still holds its value in the state before the step, which nothing in
-// this launch writes. The active donors are written by no one here either.
-__device__ __forceinline__ void fill_in_place(const FillArgs& a, const int gi) {
-    if (gi >= a.nghost) return;
-    // the record and the flags in one round trip
-    const Ghost gh = a.ghosts[gi];
-    const int ran = a.ctl->ran, out = a.ctl->out;
-    if (!ran) return;
-    double* U = a.buf[out];
-    double v[4];
-    ghost_value(a, gh, U, a.buf[out ^ 1], v);
-    for (int k = 0; k < 4; k++) U[gh.cell + k * a.L.plane] = v[k];
-}
-
-// Ghost-cell fill, phase 2: write the values into the current state.
-__device__ __forceinline__ void scatter_one(const FillArgs& a, const int gi) {
-    if (a.require_ran && !a.ctl->ran) return;
-    if (gi >= a.nghost) return;
-    double* U = a.buf[a.use_cur ? a.ctl->cur : a.fixed];
-    const long long c = a.ghosts[gi].cell, PL = a.L.plane;
-    const double* v = a.out + 4 * (long long)gi;
-    U[c] = v[0];
-    U[c + PL] = v[1];
-    U[c + 2 * PL] = v[2];
-    U[c + 3 * PL] = v[3];
-}
 __global__ void k_scatter(FillArgs a) { scatter_one(a, blockIdx.x * blockDim.x + threadIdx.x); }
 
-// Ring of the current state for the edge policies that are not fused into the
-// step (the reference policy for Lax; periodic; inflow). Reads the interior of
-// the current state, writes its ring; one thread per ring cell.
-// PREV: beside the in-place fill: the state is the buffer the step wrote, and a
-// non-active source cell is read from the state before the step, where it has
-// the value it had before the fill.
-template <bool PREV> __device__ __forceinline__ void edge_one(const EdgeArgs& a, const int q) {
-    if (PREV ? !a.ctl->ran : a.require_ran && !a.ctl->ran) return;
-    const Layout L = a.L;
-    const int ng = L.ng, nx = L.nx, ny = L.ny;
-    const int nring = L.M * L.N - nx * ny;
-    if (q >= nring) return;
-    // enumerate ring cells: bottom rows, top rows, then left/right columns of interior rows
-    int i, j;
-    int nb = L.M * ng;
-    if (q < nb) { j = q / L.M; i = q % L.M; }
-    else if (q < 2 * nb) { int r = q - nb; j = ny + ng + r / L.M; i = r % L.M; }
-    else { int r = q - 2 * nb; j = ng + r / (2 * ng); int s = r % (2 * ng); i = s < ng ? s : nx + s; }
-    const int b = PREV ? a.ctl->out : a.ctl->cur;
-    double* U = a.buf[b];
-    auto source = [&](long long s) -> const double* {
-        if (PREV) {
-            const uint8_t t = a.type[s];
-            return t == 0 || t == 3 ? U : a.buf[b ^ 1];
-        }
-        return (a.unew_nf && a.type[s] != 0) ? a.unew_nf : U;
-    };
-    const long long PL = L.plane;
-    double v[4];
-    if (a.kind == 1) {  // periodic
-        int si = i < ng ? i + nx : (i >= nx + ng ? i - nx : i);
-        int sj = j < ng ? j + ny : (j >= ny + ng ? j - ny : j);
-        long long s = L.at(si, sj);
-        const double* S = source(s);
-        for (int k = 0; k < 4; k++) v[k] = S[s + k * PL];
-    } else if (a.kind == 3) {
-        // Test/PNGGeo/Global_Boudary.cpp:14-79 (U_NEW = the state before the ghost
-        // fill's phase 2): rows as the Sod hook over the interior columns, the
-        // right columns zero-gradient, the left columns held at the inflow state;
-        // the ring corners are not written
-        const bool row = j < ng || j >= ny + ng;
-        if (row && (i < ng || i >= nx + ng)) return;
-        auto src = [&](long long s, int k) { return source(s)[s + k * PL]; };
-        if (row) {
-            const int sr = j < ng ? 2 * ng - 1 : ny + ng - 1;
-            const int rr = j < ng ? 2 * ng - j - 1 : 2 * (ny + ng) - 1 - j;
-            for (int k = 0; k < 4; k++) v[k] = src(L.at(i, sr), k);
-            v[2] = -src(L.at(i, rr), 2);
-        } else if (i < ng) {
-            for (int k = 0; k < 4; k++) v[k] = a.inflow[k];
-        } else {
-            for (int k = 0; k < 4; k++) v[k] = src(L.at(nx + ng - 1, j), k);
-        }
-    } else if (a.kind == 2) {  // inflow left, zero gradient elsewhere
-        if (i < ng) {
-            for (int k = 0; k < 4; k++) v[k] = a.inflow[k];
-        } else {
-            int si = i >= nx + ng ? nx + ng - 1 : i;
-            int sj = j < ng ? ng : (j >= ny + ng ? ny + ng - 1 : j);
-            long long s = L.at(si, sj);
-            const double* S = source(s);
-            for (int k = 0; k < 4; k++) v[k] = S[s + k * PL];
-        }
-    } else {
-        return;  // the reference policy is written by the step kernel
-    }
-    long long o = L.at(i, j);
-    for (int k = 0; k < 4; k++) U[o + k * PL] = v[k];
-}
 __global__ void k_edge(EdgeArgs a) { edge_one<false>(a, blockIdx.x * blockDim.x + threadIdx.x); }
+
 
 // What follows a step's update in one launch: the dt / mass reduction and clock
 // (blocks below nfin), the ghost fill in place (the next nfb) and the edge ring.
@@ -968,76 +1101,6 @@ __global__ __launch_bounds__(POST_BATCH_THREADS) void k_post_batch(
     for (int k = threadIdx.x; k < EDGE_THREADS; k += POST_BATCH_THREADS) edge_one<true>(edge[m.x], m.y + k);
 }
 
-// ------------------------------------------------------ persistent batched step
-// Grid barrier among all blocks of a launch (every block resident): arrivals
-// counted in bar[0], which only grows during a launch, so barrier k completes
-// when it reaches (k + 1) x blocks. Device-scope fences before the arrival
-// (release: this block's stores reach the coherence point past its XCD's L2)
-// and after the wait (acquire: no stale lines of other XCDs' stores). A wait
-// longer than spin_limit polls sets *err and every block leaves the launch.
-__device__ __forceinline__ bool grid_sync(const PersistArgs& p, unsigned int& target) {
-    target += gridDim.x;
-    int ok = 1;
-    if (threadIdx.x == 0) {
-        __threadfence();
-        atomicAdd(p.bar, 1u);
-        long long spins = 0;
-        while (__hip_atomic_load(p.bar, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < target) {
-            __builtin_amdgcn_s_sleep(2);
-            if (++spins > p.spin_limit || __hip_atomic_load(p.err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
-                atomicExch(p.err, 1);
-                ok = 0;
-                break;
-            }
-        }
-        __threadfence();
-    }
-    return __shfl(ok, 0, 64) != 0;
-}
-
-template <int SCH, int RS, int LIM, typename T>
-__global__ __launch_bounds__(64) void k_persist(PersistArgs p) {
-    const int G = gridDim.x;
-    unsigned int target = 0;
-    const int nstrip = p.counts[0], nghost = p.counts[1], nring = p.counts[2];
-    for (int s = 0; s < p.nsteps; s++) {
-        for (int stage = p.rk2 ? 1 : 0;;) {
-            // strips of every resident solve (TimeAdvance; reference ring fused)
-            for (int w = blockIdx.x; w < nstrip; w += G) {
-                const int2 m = p.smap[w];
-                const StepArgs& a = p.step[m.x];
-                step_strip<SCH, RS, LIM, T, false>(a, m.y % a.nbx, m.y / a.nbx, stage);
-            }
-            if (!grid_sync(p, target)) return;
-            // ComputeDt / mass / clock per solve (RK2 stage 1: make the stage buffer current)
-            for (int q = blockIdx.x; q < p.nslots; q += G)
-                if (p.fin[q].ctl) finish_body<64>(p.fin[q], stage == 1 ? 2 : 1);
-            if (!grid_sync(p, target)) return;
-            // Boundary phase 1 and Global_Boundary
-            if (p.has_fill)
-                for (int w = blockIdx.x; w < nghost; w += G) {
-                    const int2 m = p.gmap[w];
-                    for (int k = threadIdx.x; k < FILL_THREADS; k += 64) fill_one(p.fill[m.x], m.y + k);
-                }
-            for (int w = blockIdx.x; w < nring; w += G) {
-                const int2 m = p.rmap[w];
-                for (int k = threadIdx.x; k < EDGE_THREADS; k += 64) edge_one<false>(p.edge[m.x], m.y + k);
-            }
-            if (!grid_sync(p, target)) return;
-            // Boundary phase 2
-            if (p.has_fill) {
-                for (int w = blockIdx.x; w < nghost; w += G) {
-                    const int2 m = p.gmap[w];
-                    for (int k = threadIdx.x; k < FILL_THREADS; k += 64) scatter_one(p.fill[m.x], m.y + k);
-                }
-                if (!grid_sync(p, target)) return;
-            }
-            if (stage == 1) { stage = 2; continue; }
-            break;
-        }
-    }
-}
-
 __global__ void k_zero_u32(unsigned int* p, int n) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) p[i] = 0;
@@ -1083,40 +1146,6 @@ __global__ void k_edge_ref(EdgeArgs a, const double* corner, int corner_from_inp
 }
 
 // ------------------------------------------------------------------ launchers
-// A batched launch (k_step_batch) instead of a single-solve one when non-null.
-struct BatchLaunch {
-    const StepArgs* slots;
-    const int2* map;
-    int nblocks;
-    int stage;
-};
-template <int SCH, int RS, int LIM>
-static hipError_t go(int prec, const StepArgs* a, const BatchLaunch* b, hipStream_t s) {
-    if (b) {
-        if (prec == 1)
-            hipLaunchKernelGGL((k_step_batch<SCH, RS, LIM, float>), dim3(b->nblocks), dim3(64), 0, s, b->slots, b->map,
-                               b->stage);
-        else
-            hipLaunchKernelGGL((k_step_batch<SCH, RS, LIM, double>), dim3(b->nblocks), dim3(64), 0, s, b->slots,
-                               b->map, b->stage);
-    } else if (a->cut) {  // cut-cell variant (its extra registers stay out of the plain kernel)
-        if (prec == 1) hipLaunchKernelGGL((k_step<SCH, RS, LIM, float, true>), dim3(a->nbx, a->nby), dim3(64), 0, s, *a);
-        else hipLaunchKernelGGL((k_step<SCH, RS, LIM, double, true>), dim3(a->nbx, a->nby), dim3(64), 0, s, *a);
-    } else if (a->edge_fused == 2) {  // periodic ring written by the step kernel
-        if (prec == 1) hipLaunchKernelGGL((k_step_periodic<SCH, RS, LIM, float>), dim3(a->nbx, a->nby), dim3(64), 0, s, *a);
-        else hipLaunchKernelGGL((k_step_periodic<SCH, RS, LIM, double>), dim3(a->nbx, a->nby), dim3(64), 0, s, *a);
-    } else {
-        if (prec == 1) hipLaunchKernelGGL((k_step<SCH, RS, LIM, float, false>), dim3(a->nbx, a->nby), dim3(64), 0, s, *a);
-        else hipLaunchKernelGGL((k_step<SCH, RS, LIM, double, false>), dim3(a->nbx, a->nby), dim3(64), 0, s, *a);
-    }
-    return hipGetLastError();
-}
-template <int SCH, int RS>
-static hipError_t go_l(int lim, int prec, const StepArgs* a, const BatchLaunch* b, hipStream_t s) {
-    if (lim == LIM_MINMOD) return go<SCH, RS, LIM_MINMOD>(prec, a, b, s);
-    if (lim == LIM_VANLEER) return go<SCH, RS, LIM_VANLEER>(prec, a, b, s);
-    return go<SCH, RS, LIM_VANALBADA>(prec, a, b, s);
-}
 template <int SCH>
 static hipError_t go_r(int rs, int lim, int prec, const StepArgs* a, const BatchLaunch* b, hipStream_t s) {
     if (rs == RS_SW) return go_l<SCH, RS_SW>(lim, prec, a, b, s);
@@ -1140,28 +1169,25 @@ hipError_t launch_step_batch(int scheme, int rs, int lim, int prec, const StepAr
     BatchLaunch b{slots, map, nblocks, stage};
     return go_s(scheme, rs, lim, prec, nullptr, &b, s);
 }
-// persistent batched step: the kernel for a slot selection, and its resident grid
-template <int SCH, int RS, int LIM>
-static const void* persist_fn(int prec) {
-    if (prec == IBTFO_MIXED) return (const void*)k_persist<SCH, RS, LIM, float>;
-    return (const void*)k_persist<SCH, RS, LIM, double>;
-}
 static const void* persist_kernel(int scheme, int rs, int lim, int prec) {
-    auto by_lim = [&](auto sch, auto r) -> const void* {
-        constexpr int S = decltype(sch)::value, R = decltype(r)::value;
-        if (lim == LIM_MINMOD) return persist_fn<S, R, LIM_MINMOD>(prec);
-        if (lim == LIM_VANLEER) return persist_fn<S, R, LIM_VANLEER>(prec);
-        return persist_fn<S, R, LIM_VANALBADA>(prec);
-    };
     auto by_rs = [&](auto sch) -> const void* {
-        if (rs == RS_SW) return by_lim(sch, std::integral_constant<int, RS_SW>());
-        if (rs == RS_PVRS) return by_lim(sch, std::integral_constant<int, RS_PVRS>());
-        return by_lim(sch, std::integral_constant<int, RS_HLL>());
+        constexpr int S = decltype(sch)::value;
+        if (rs == RS_SW) return persist_l<S, RS_SW>(lim, prec);
+        if (rs == RS_PVRS) return persist_l<S, RS_PVRS>(lim, prec);
+        return persist_l<S, RS_HLL>(lim, prec);
     };
     if (scheme == SCH_MHM) return by_rs(std::integral_constant<int, SCH_MHM>());
     if (scheme == SCH_GODUNOV) return by_rs(std::integral_constant<int, SCH_GODUNOV>());
     return by_rs(std::integral_constant<int, SCH_MUSCL>());
 }
+// Loads the code object that a solve's launches come from (the first launch in a process
+// would), so that neither a step nor a stream capture pays for it.
+hipError_t load_step(int scheme, int rs, int lim, int prec, int rowpar) {
+    hipFuncAttributes at;
+    if (scheme == SCH_LAX) return hipSuccess;  // beside the reductions
+    return hipFuncGetAttributes(&at, rowpar ? rowpar_kernel(scheme, rs) : persist_kernel(scheme, rs, lim, prec));
+}
+// the persistent kernel's resident grid
 int persist_blocks(int scheme, int rs, int lim, int prec) {
     int per_cu = 0, dev = 0, cus = 0;
     if (scheme == SCH_LAX) return 0;
@@ -1296,5 +1322,7 @@ hipError_t launch_post(const FinishArgs& f, const FillArgs* fill, const EdgeArgs
                        edge ? *edge : EdgeArgs(), nfin, nfb);
     return hipGetLastError();
 }
+
+#endif  // STEP_SCHEME
 
 }  // namespace ibtfo

@@ -138,6 +138,7 @@ hipError_t launch_step(int, int, int, int, const StepArgs& a, hipStream_t s) {
     });
     return hipSuccess;
 }
+hipError_t load_step(int, int, int, int, int) { return hipSuccess; }
 hipError_t launch_df_flush(const StepArgs& a, int k, hipStream_t s) {
     fake::run(s, [a, k] {
         DfHead h = a.ctl->df[k];

@@ -12,7 +12,7 @@ READELF = os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "lib", "llvm", 
 
 
 def kernels(tmp_path):
-    """{mangled name: (registers, scratch bytes)} of the gfx950 code objects."""
+    """{mangled name: (registers, scratch bytes, code object)} of the gfx950 code objects."""
     lib = os.path.join(ROOT, "ibtfo_amd", "libibtfo_amd.so")
     tool = READELF if os.path.isfile(READELF) else shutil.which("llvm-readelf")
     if not os.path.isfile(lib) or tool is None:
@@ -35,7 +35,7 @@ def kernels(tmp_path):
             for block in re.split(r"\n\s+- \.agpr_count", notes)[1:]:
                 field = {k: re.search(r"\.%s:\s+(\S+)" % k, block).group(1)
                          for k in ("name", "vgpr_count", "private_segment_fixed_size")}
-                out[field["name"]] = (int(field["vgpr_count"]), int(field["private_segment_fixed_size"]))
+                out[field["name"]] = (int(field["vgpr_count"]), int(field["private_segment_fixed_size"]), at)
         at = data.find(magic, at + 1)
     return out
 
@@ -48,3 +48,19 @@ def test_mixed_precision_strips_hold_no_scratch(tmp_path):
     # 3 schemes x 3 solvers x 3 limiters, each plain, with cut cells, periodic and batched
     assert len(strips) == 108
     assert {n: r for n, r in strips.items() if r[1]} == {}
+
+
+def test_step_kernels_load_with_their_scheme_and_solver(tmp_path):
+    """A solve loads one scheme's and solver's step kernels and none of the others': a
+    code object of step kernels holds one pair, and the other kernels lie elsewhere (all
+    pairs in one object cost a process's first solve 14 ms)."""
+    pairs = {}
+    other = set()
+    for name, (_, _, obj) in kernels(tmp_path).items():
+        m = re.search(r"k_(step|step_batch|step_periodic|step_rowpar|persist)ILi(\d+)ELi(\d+)E", name)
+        if m:
+            pairs.setdefault(obj, set()).add(m.groups()[1:])
+        else:
+            other.add(obj)
+    assert len(pairs) == 18 and all(len(p) == 1 for p in pairs.values())
+    assert not other & set(pairs)
