@@ -224,8 +224,8 @@ struct FinishArgs {
 };
 constexpr int FOLD_THREADS = 256;
 constexpr int FOLD_MAX = 128;      // fold records
-// Fewer partials: one block reads them all (a finish of 1258 records alone, 10 us; folded
-// 3; of 812 records 2.4, folded 3).
+// Fewer partials: one block reads them all, one per thread (816 records 4.7 us, 12.1 for
+// 1258; folded, 5.7 for 1037 and 5.9 for 3077).
 constexpr int FOLD_MIN_PARTS = 1025;
 
 constexpr int FILL_THREADS = 128;  // ghost-fill and scatter blocks
@@ -296,7 +296,7 @@ hipError_t launch_step_batch(int scheme, int rs, int lim, int prec, const StepAr
                              int nblocks, int stage, hipStream_t s);
 hipError_t launch_gather(const FinishArgs* f, int nslots, SlotStatus* out, hipStream_t s);
 // the persistent batched step: a zeroing of the barrier counter, then one launch of
-// `blocks` blocks (persist_blocks: the grid the kernel can hold resident at once)
+// `blocks` blocks (persist_blocks: a grid that is always resident at once)
 hipError_t launch_persist(int scheme, int rs, int lim, int prec, const PersistArgs& p, int blocks, hipStream_t s);
 int persist_blocks(int scheme, int rs, int lim, int prec);
 hipError_t launch_step_lax(const StepArgs& a, hipStream_t s);

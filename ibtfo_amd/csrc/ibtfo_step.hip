@@ -190,8 +190,8 @@ __device__ __forceinline__ void block4_reduce(double& amax, double& umax, double
 // blocks. They are written, counted and read by device-scope atomics, which act
 // where every XCD sees them, and a block's count follows the completion of its
 // stores (the wait). A device-scope fence instead writes back and invalidates the
-// XCD's whole L2, in every fold block (4096x2048, 17664 records: 236.7 -> 233.4 us per
-// step at 12-row strips, 1003x517: 41.1 -> 40.4).
+// XCD's whole L2, in every fold block (4096x2048 cut cells 236.7 -> 233.4 us per
+// step, 1003x517 41.1 -> 40.4).
 __device__ __forceinline__ void fold_body(const FinishArgs& f, const int block) {
     if (f.ctl->done) return;  // the step kernel did not run (every block sees the same flag)
     const int nrec = f.nblocks + (f.part2 ? f.nblocks2 : 0);
@@ -517,7 +517,9 @@ __device__ __forceinline__ void step_strip(const StepArgs& a, const int bx, cons
 
 // Four waves per SIMD (128 VGPRs): the strip's chains of dependent FP64 work and
 // LDS exchanges need them (4096x2048 cut cells, HLL: 245 us at three waves, 226 at
-// four; Steger-Warming, 132 VGPRs unbounded: 325 us, 302 us with 12 bytes spilled).
+// four). Steger-Warming in FP64 takes 128 to 135 registers unbounded and 12 to 28 bytes
+// of scratch at four waves, which are ahead with a ghost fluid (4096x2048 310.6 us per
+// step, 314.1 at three) and even with cut cells (319.5 / 319.2).
 // PVRS, whose pow() calls need far more registers, is left to the compiler.
 // MUSCL-Hancock with HLL in mixed precision takes 138 to 142 registers: held to four
 // waves, 36 to 56 bytes of scratch in the row loop cost more than the fourth wave gives

@@ -311,11 +311,12 @@ typedef struct ibtfo_batch_config {
     int max_step_blocks;   /* step-kernel grid capacity (strips of 60 columns x rows) */
     int max_ghost_blocks;  /* ghost-fill grid capacity (128 ghosts per block) */
     int max_ring_blocks;   /* edge-ring grid capacity (256 ring cells per block) */
-    int rows;              /* strip height of every solve (0: 8, or 16 where step blocks are short) */
+    int rows;              /* strip height of every solve (0: 8, or 16 where max_step_blocks is below
+                              12288 or the solve fits only so) */
     int chunk;             /* steps per graph replay */
     int persistent;        /* 1: each replay is one persistent kernel that runs the chunk's steps of
                               every resident solve, its phases separated by grid barriers (the grid
-                              sized to what the device holds resident); 0: one launch per phase */
+                              one wave per SIMD, which is always resident); 0: one launch per phase */
 } ibtfo_batch_config;
 
 typedef struct ibtfo_request {
