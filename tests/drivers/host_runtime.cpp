@@ -29,6 +29,7 @@ double clock_ms = 0;         // advanced by the step kernels
 int ghosts = 0;              // ghosts a geometry finds
 int geometries = 0;          // geometry runs
 int launches = 0, wrong_hints = 0;
+int captures = 0, first_record = -1, last_record = -1;  // captures so far; at the first and last event
 int batch_rows = 0;          // strip height of the batch's last solve stepped
 int lds_limit = 0, lds_refused = 0;  // the mask kernel's LDS attribute; launches above it
 std::function<void()> after_attribute;
@@ -65,6 +66,7 @@ hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
 hipError_t hipStreamQuery(hipStream_t) { return hipSuccess; }
 hipError_t hipStreamBeginCapture(hipStream_t s, hipStreamCaptureMode) {
     s->capturing = true;
+    fake::captures++;
     s->ops.clear();
     return hipSuccess;
 }
@@ -86,7 +88,12 @@ hipError_t hipGraphLaunch(hipGraphExec_t e, hipStream_t) {
 }
 hipError_t hipEventCreate(hipEvent_t* e) { *e = new ihipEvent_t(); return hipSuccess; }
 hipError_t hipEventDestroy(hipEvent_t e) { delete e; return hipSuccess; }
-hipError_t hipEventRecord(hipEvent_t e, hipStream_t) { e->at = fake::clock_ms; return hipSuccess; }
+hipError_t hipEventRecord(hipEvent_t e, hipStream_t) {
+    e->at = fake::clock_ms;
+    if (fake::first_record < 0) fake::first_record = fake::captures;
+    fake::last_record = fake::captures;
+    return hipSuccess;
+}
 hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
 hipError_t hipEventElapsedTime(float* ms, hipEvent_t a, hipEvent_t b) { *ms = (float)(b->at - a->at); return hipSuccess; }
 hipError_t hipGetDevice(int* d) { *d = 0; return hipSuccess; }
@@ -302,6 +309,14 @@ static void graph_start() {
             int it = 0;
             CHECK(ibtfo_status(x, &it, nullptr, nullptr) == IBTFO_OK && it == steps);
             CHECK(fake::launches == steps * (time == IBTFO_RK2 ? 2 : 1) && fake::wrong_hints == 0);
+            // a timed run from either buffer: nothing is captured between its events
+            for (int odd : {0, 1}) {
+                CHECK(ibtfo_step_graph(x, 0, 20 + odd * 2) == IBTFO_OK && ibtfo_step(x, odd) == IBTFO_OK);
+                fake::first_record = -1;
+                double ms = 0;
+                CHECK(ibtfo_time_steps(x, 100, &ms, nullptr) == IBTFO_OK);
+                CHECK(fake::first_record >= 0 && fake::first_record == fake::last_record);
+            }
             ibtfo_destroy(x);
         }
 }
